@@ -40,6 +40,12 @@ constexpr int kFftChunk = 64;
 int fft_exec(int inverse, const void* in, void* out, int rows, int N, void* stream);
 int fft_rows(int inverse, const void* in, void* out, int n, int N, void* stream);
 
+// The library's own forward transforms (fft_kernels.hip): log2 N when they take
+// these n rows, else 0; and the launch.  They take N = 2^10 .. 2^21 with
+// 16-byte aligned rows and an output that does not overlap the input.
+int rfft_own_log2(const void* in, const void* out, int n, int N);
+int rfft_own(const double* in, double* out, int n, int log2N, hipStream_t st);
+
 }  // namespace eobhip_detail
 
 #define EOBHIP_REQUIRE(cond, ...)                        \

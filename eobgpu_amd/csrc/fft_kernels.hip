@@ -1,0 +1,246 @@
+// Batched real-to-complex FFTs (see fft.hpp) and the weighted norm of the
+// transforms that the support-length likelihood needs, computed in the last
+// pass so that those transforms are never written.
+#include <hip/hip_runtime.h>
+
+#include "eobhip_common.hpp"
+#include "fft.hpp"
+
+using namespace eobhip_detail;
+
+namespace {
+
+// Where a pass of a batch of rows finds its input and leaves its output.
+// in: rows of N doubles (stride in_stride doubles); out: rows of complex bins
+// (stride out_stride).  nvalid (optional): samples of the row that are not
+// zero by definition, count[map[first + row]]; the rest are not read.
+struct Rows {
+    const double* in;
+    double2* out;
+    long long in_stride, out_stride;
+    const int* count;
+    const long long* map;
+    int rows;
+};
+
+// Sum of |X_k|^2 w_k instead of the bins: w (stride 1) and one partial per
+// (row, block of the row), partial[map[row] * pstride + block].
+struct Norm {
+    const double* w;
+    double* partial;
+    int pstride;
+};
+
+__device__ __forceinline__ long long valid_samples(const Rows& a, int row, long long N) {
+    if (!a.count) return N;
+    const long long c = a.count[a.map[row]];
+    return c < 0 ? 0 : (c > N ? N : c);
+}
+
+// the two real samples of point j, zero past the row's samples (the caller
+// keeps samples up to the next even count defined)
+__device__ __forceinline__ double2 load_point(const double2* __restrict__ z, long long j, long long nv) {
+    return 2 * j < nv ? z[j] : make_double2(0.0, 0.0);
+}
+
+// Sum of a value over the block's threads with the same (threadIdx.x / G); G a
+// power of two.  The result is valid on the first thread of each G.
+template <int G>
+__device__ __forceinline__ double group_sum(double v, double* red) {
+    constexpr int W = G < 64 ? G : 64;
+#pragma unroll
+    for (int off = W / 2; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
+    if constexpr (G > 64) {
+        __syncthreads();
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+        __syncthreads();
+        if (threadIdx.x % G == 0) {
+            v = 0.0;
+            for (int k = 0; k < G / 64; ++k) v += red[(threadIdx.x >> 6) + k];
+        }
+    }
+    return v;
+}
+
+// ------------------------------------------------------------ whole rows
+// H = 2^LH points per row, kFftPoints / H rows per block.  Twiddles of up to
+// 8192 points are products of two small tables.
+template <int LH, bool kNorm>
+__global__ __launch_bounds__(kFftThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_rfft_one(Rows a, Norm nm) {
+    constexpr int H = 1 << LH, per = H / 16;   // threads per row
+    __shared__ double buf[kFftPoints + kFftPoints / 16];
+    __shared__ double2 hi[H / 64], lo[64];
+    const int t = threadIdx.x, rr = t / per, p = t % per;
+    const long long row = (long long)blockIdx.x * (kFftPoints / H) + rr;
+    const bool on = row < a.rows;
+    for (int i = t; i < H / 64; i += kFftThreads) hi[i] = fft_unit((double)i * (64.0 / H));
+    if (t < 64) lo[t] = fft_unit((double)t * (1.0 / H));
+    const double2* z = reinterpret_cast<const double2*>(a.in + (on ? row : 0) * a.in_stride);
+    const long long nv = on ? valid_samples(a, (int)row, 2LL * H) : 0;
+    double2 v[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) v[u] = load_point(z, p + per * u, nv);
+    const auto addr = [&](int pos) { return rr * (H + H / 16) + pos + (pos >> 4); };
+    const SplitTable tw{hi, lo};
+    fft_stages<LH>(v, p, p, buf, tw, addr, addr, addr);
+    double acc = 0.0;
+    real_bins(v, buf, rr * per + ((per - p) & (per - 1)), p == 0, fft_unit((double)p * (0.5 / H)), [&](int u, double2 x) {
+        const int k = p + per * u;
+        if constexpr (kNorm) acc += (x.x * x.x + x.y * x.y) * nm.w[k];
+        else if (on) a.out[row * a.out_stride + k] = x;
+    });
+    if (p == 0) {
+        const double nyq = v[0].x - v[0].y;   // X_H
+        if constexpr (kNorm) acc += nyq * nyq * nm.w[H];
+        else if (on) a.out[row * a.out_stride + H] = make_double2(nyq, 0.0);
+    }
+    if constexpr (kNorm) {
+        const double s = group_sum<per>(acc, buf);   // the first barrier inside is after every thread's reads of buf
+        if (p == 0 && on) nm.partial[a.map[row] * nm.pstride] = s;
+    }
+}
+
+// --------------------------------------------------- columns of an A x B row
+template <int LA>
+__global__ __launch_bounds__(kFftThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_rfft_cols(Rows a, int LB) {
+    constexpr int A = 1 << LA, C = kFftPoints / A, per = A / 16;
+    constexpr int pad = C >= 32 ? 1 : 32 / C;
+    constexpr int skew = kFftPoints / 16;
+    constexpr int kWords = kFftPoints + (skew > C * pad ? skew : C * pad);
+    __shared__ double buf[kWords];
+    __shared__ double2 tab[A / 2], step[C][16];
+    const int B = 1 << LB, t = threadIdx.x;
+    const unsigned id = xcd_run(blockIdx.x, gridDim.x);
+    const int groups = B / C;
+    const int row = (int)(id / groups), b0 = (int)(id % groups) * C;
+    const long long N = 2LL * A * B;
+    const double invH = 2.0 / (double)N;
+    if (t < A / 2) tab[t] = fft_unit((double)t * (1.0 / A));
+    // W_H^(b (A/16) u): the between-pass twiddle's step along a thread's outputs
+    for (int e = t; e < C * 16; e += kFftThreads) {
+        const int u = e & 15, i = e >> 4;
+        step[i][u] = fft_unit((double)((long long)(b0 + i) * u) * ((double)per * invH));
+    }
+    const int i = t % C, p = t / C;
+    const double2* z = reinterpret_cast<const double2*>(a.in + row * a.in_stride);
+    const long long nv = valid_samples(a, row, N);
+    double2 v[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) v[u] = load_point(z, ((long long)(p + per * u) << LB) + b0 + i, nv);
+    // column fastest until the last exchange, which turns to position fastest
+    // (a column's outputs are stored contiguously)
+    const int i2 = t / per, p2 = t % per;
+    const HalfTable tw{tab, A};
+    fft_stages<LA>(v, p, p2, buf, tw, [&](int pos) { return (pos + (pos >> 4)) * C + i; }, [&](int pos) { return i * (A + pad) + pos; },
+                   [&](int pos) { return i2 * (A + pad) + pos; });
+    const long long b = b0 + i2;
+    const double2 w0 = fft_unit((double)(b * p2) * invH);
+    double2* o = a.out + row * a.out_stride + (b << LA);
+#pragma unroll
+    for (int u = 0; u < 16; ++u) o[p2 + per * u] = cmul2(v[u], cmul2(w0, step[i2][u]));
+}
+
+// ------------------------------------------------------ rows of an A x B row
+template <int LB, bool kNorm>
+__global__ __launch_bounds__(kFftThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_rfft_rows(Rows a, Norm nm, int LA) {
+    constexpr int B = 1 << LB, C2 = kFftPoints / B, C = C2 / 2, per = B / 16;
+    __shared__ double buf[kFftPoints + kFftPoints / 16];
+    __shared__ double2 tab[B / 2];
+    const int A = 1 << LA, t = threadIdx.x;
+    const unsigned id = xcd_run(blockIdx.x, gridDim.x);
+    const int groups = A / C2;
+    const int row = (int)(id / groups), g = (int)(id % groups);
+    const long long H = (long long)A * B;
+    if (t < B / 2) tab[t] = fft_unit((double)t * (1.0 / B));
+    const int i = t % C2, p = t / C2;
+    // slots i < C: ka = g C + i; the others their partners A - ka (ka = A/2 in the place of 0's)
+    const int kl = g * C + (i & (C - 1));
+    const int ka = i < C ? kl : (kl == 0 ? A / 2 : A - kl);
+    // a row is at most 16 MiB + 16 bytes: 32-bit byte offsets from its (uniform) start
+    char* o = reinterpret_cast<char*>(a.out + row * a.out_stride);
+    const unsigned at = ((unsigned)ka + ((unsigned)p << LA)) * 16u, up = (unsigned)(per << LA) * 16u;
+    double2 v[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) v[u] = *reinterpret_cast<const double2*>(o + (at + up * u));
+    const HalfTable tw{tab, B};
+    const auto addr = [&](int pos) { return (pos + (pos >> 4)) * C2 + i; };
+    fft_stages<LB>(v, p, p, buf, tw, addr, addr, addr);
+    // the partner H - k of k = ka + A kb: row A - ka, kb' = B - 1 - kb; rows 0
+    // (kb' = B - kb) and A/2 are their own
+    const int mate = (kl == 0 ? i : (i ^ C)) + C2 * (((ka == 0 ? per : per - 1) - p) & (per - 1));
+    const char* wt = reinterpret_cast<const char*>(nm.w);
+    double acc = 0.0;
+    real_bins(v, buf, mate, ka == 0 && p == 0, fft_unit((double)(ka + (long long)p * A) * (0.5 / (double)H)), [&](int u, double2 x) {
+        if constexpr (kNorm) acc += (x.x * x.x + x.y * x.y) * *reinterpret_cast<const double*>(wt + ((at + up * u) >> 1));
+        else *reinterpret_cast<double2*>(o + (at + up * u)) = x;
+    });
+    if (ka == 0 && p == 0) {
+        const double nyq = v[0].x - v[0].y;   // X_H
+        if constexpr (kNorm) acc += nyq * nyq * nm.w[H];
+        else *reinterpret_cast<double2*>(o + 16 * H) = make_double2(nyq, 0.0);
+    }
+    if constexpr (kNorm) {
+        const double s = group_sum<kFftThreads>(acc, buf);
+        if (t == 0) nm.partial[a.map[row] * nm.pstride + g] = s;
+    }
+}
+
+// A of H = A B for H > kFftPoints: the larger half
+int log2_cols(int lh) { return (lh + 1) / 2; }
+
+template <bool kNorm>
+int launch_rows(const Rows& a, const Norm& nm, int LN, hipStream_t st) {
+    const int lh = LN - 1;
+    if (LN <= kFftOneMaxLog2) {
+        const unsigned nb = blocks_for(a.rows, kFftPoints >> lh);
+        switch (lh) {
+#define EOBHIP_ONE(L) \
+    case L: hipLaunchKernelGGL((k_rfft_one<L, kNorm>), dim3(nb), dim3(kFftThreads), 0, st, a, nm); break;
+            EOBHIP_ONE(9) EOBHIP_ONE(10) EOBHIP_ONE(11) EOBHIP_ONE(12) EOBHIP_ONE(13)
+#undef EOBHIP_ONE
+            default: set_error("rfft: unsupported length 2^%d", LN); return EOBHIP_EINVAL;
+        }
+        return check_launch("rfft");
+    }
+    const int la = log2_cols(lh), lb = lh - la;
+    const long long nc = (long long)a.rows << (lb - (13 - la)), nr = (long long)a.rows << (la - (13 - lb));
+    EOBHIP_REQUIRE(nc < (1LL << 31) && nr < (1LL << 31), "rfft: too many rows");
+    switch (la) {
+#define EOBHIP_COLS(L) \
+    case L: hipLaunchKernelGGL(k_rfft_cols<L>, dim3((unsigned)nc), dim3(kFftThreads), 0, st, a, lb); break;
+        EOBHIP_COLS(7) EOBHIP_COLS(8) EOBHIP_COLS(9) EOBHIP_COLS(10)
+#undef EOBHIP_COLS
+        default: set_error("rfft: unsupported length 2^%d", LN); return EOBHIP_EINVAL;
+    }
+    int rc = check_launch("rfft columns");
+    if (rc) return rc;
+    switch (lb) {
+#define EOBHIP_ROWS(L) \
+    case L: hipLaunchKernelGGL((k_rfft_rows<L, kNorm>), dim3((unsigned)nr), dim3(kFftThreads), 0, st, a, nm, la); break;
+        EOBHIP_ROWS(7) EOBHIP_ROWS(8) EOBHIP_ROWS(9) EOBHIP_ROWS(10)
+#undef EOBHIP_ROWS
+        default: set_error("rfft: unsupported length 2^%d", LN); return EOBHIP_EINVAL;
+    }
+    return check_launch("rfft rows");
+}
+
+}  // namespace
+
+namespace eobhip_detail {
+
+int rfft_own_log2(const void* in, const void* out, int n, int N) {
+    if (n < 1 || N < (1 << kFftMinLog2) || N > (1 << kFftMaxLog2) || (N & (N - 1))) return 0;
+    const uintptr_t a = reinterpret_cast<uintptr_t>(in), b = reinterpret_cast<uintptr_t>(out);
+    if ((a | b) & 15) return 0;
+    const uintptr_t na = (uintptr_t)n * N * 8, nb = (uintptr_t)n * (N / 2 + 1) * 16;
+    if (a < b + nb && b < a + na) return 0;
+    return __builtin_ctz((unsigned)N);
+}
+
+int rfft_own(const double* in, double* out, int n, int log2N, hipStream_t st) {
+    const long long N = 1LL << log2N;
+    return launch_rows<false>(Rows{in, reinterpret_cast<double2*>(out), N, N / 2 + 1, nullptr, nullptr, n}, Norm{nullptr, nullptr, 0}, log2N,
+                              st);
+}
+
+}  // namespace eobhip_detail
