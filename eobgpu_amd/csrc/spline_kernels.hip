@@ -14,6 +14,7 @@
 #include <tuple>
 #include <utility>
 
+#include "eob_fastmath.hpp"
 #include "eobhip_common.hpp"
 #include "knot_window.hpp"
 #include "spline_nak.hpp"
@@ -179,6 +180,226 @@ __global__ __launch_bounds__(kBlock) void k_interpolate_TD(const double* __restr
 // nser interpolants per binary over its trajectory knots t_k (units of M):
 // knots [n][max_step][nser] (for the (2,2) pipeline nser = 3: phi, Re and Im of
 // h22 e^{2 i phi}), coef [n][max_step][4 nser] = (y, c1, c2, c3) per interpolant.
+//
+// ------------------------------------------------ (2,2) pipeline: tiles
+// The three interpolants of the likelihood pipeline's (2,2) mode (and any three
+// series on long knots).  The work is split by tiles of kTile rows of one
+// binary.  The block forms the tile's spacings and slopes from rows loaded in
+// order, once, in LDS; lane c of wavefront q then solves rows 16 c .. 16 c + 15
+// of series q: it eliminates the kHalo rows below its own upwards and the kHalo
+// rows above downwards, side by side (two independent chains) and both from a
+// cut system, closes its own 16 rows between the two and puts their knot slopes
+// in LDS, from which the block writes the coefficients in memory order.
+//
+// The effect of a cut is damped as the sweep kernel's comment below says; the
+// lane multiplies the damping factors of its own halo rows, and where their
+// product is not below 2^-54 (spacings that shrink over tens of rows) it starts
+// again kHaloMax = 64 rows away, where the dominance alone gives 2^-64.  The
+// not-a-knot end rows are never cut.
+//
+// Bound by memory: per knot t (its trajectory row's 40 bytes), the series (8
+// bytes each) and the coefficients (32 bytes per series) once each; the halos
+// cost five eliminated rows per row but read LDS.  512 chirps of 5k-60k knots
+// (16.6 M knots, 160 bytes each): 2.23 ms for the sweep kernel (one wavefront
+// per binary, each lane a 21st of the rows, read from memory as it goes),
+// 0.60 now; 256 trajectories of 600 knots: 176 and 39 us.
+constexpr int kTile = 1024;              // rows per block
+constexpr int kOwn = 16;                 // rows per lane
+constexpr int kTileSeries = 3;           // one wavefront each
+constexpr int kTileThreads = 64 * kTileSeries;
+constexpr int kTileRows = kTile + 2 * (kHaloMax + 1);
+constexpr int kTileWords = kTileRows + kTileRows / kOwn + 1;   // one word of padding per kOwn rows
+static_assert(kTile / kOwn == 64, "one wavefront per series");
+__device__ __forceinline__ int tile_at(int k) { return k + (k >> 4); }
+
+// One elimination row: from the neighbour's relation s_n = g - h s (g, h in, cut
+// rows g = h = 0) and the row a s_n + dg s + c s_next = b to s = b' - c' s_next.
+struct Carry {
+    double h, g;   // c', d'
+    __device__ __forceinline__ double step(double a, double dg, double c, double b) {
+        const double inv = eob::refined_rcp(dg - a * h);
+        g = (b - a * g) * inv;
+        h = c * inv;
+        return inv;
+    }
+};
+
+__global__ __launch_bounds__(kTileThreads) void k_spline_build_tile(const double* __restrict__ dense, const double* __restrict__ knots,
+                                                                   const int* __restrict__ num_steps, int max_step,
+                                                                   double* __restrict__ coef) {
+    constexpr int G = kTileSeries;
+    __shared__ double dx[kTileWords], mq[G][kTileWords];
+    const int b = blockIdx.y;
+    const int len = num_steps[b];
+    const int base = blockIdx.x * kTile;
+    if (base >= len) return;
+    const int tid = threadIdx.x;
+    const double* T = dense + (size_t)b * max_step * 5;
+    const double* Y = knots + (size_t)b * max_step * G;
+    double* C = coef + (size_t)b * max_step * (4 * G);
+    if (len < 3) {
+        if (tid < G)
+            for (int i = 0; i < len; ++i) {
+                double* c = C + (size_t)(4 * G) * i + 4 * tid;
+                c[0] = Y[(size_t)G * i + tid];
+                c[1] = c[2] = c[3] = 0.0;
+            }
+        return;
+    }
+    // intervals lo .. top: what the lanes' halos can reach
+    const int lo = base - kHaloMax - 1 > 0 ? base - kHaloMax - 1 : 0;
+    const int top = base + kTile + kHaloMax < len - 2 ? base + kTile + kHaloMax : len - 2;
+    for (int k = tid; k <= top - lo; k += kTileThreads) {
+        const double* t = T + (size_t)5 * (lo + k);
+        const double* y = Y + (size_t)G * (lo + k);
+        const double d = t[5] - t[0];
+        dx[tile_at(k)] = d;
+#pragma unroll
+        for (int q = 0; q < G; ++q) mq[q][tile_at(k)] = eob::qdiv(y[G + q] - y[q], d);
+    }
+    __syncthreads();
+    const int q = tid >> 6, s0 = base + (tid & 63) * kOwn;
+    const bool on = s0 < len;
+    double x[kOwn + 1];
+    if (on) {
+        const double* m = mq[q];
+        const auto D = [&](int i) { return dx[tile_at(i - lo)]; };
+        const auto M = [&](int i) { return m[tile_at(i - lo)]; };
+        const int e0 = s0 + kOwn < len ? s0 + kOwn : len;
+        Carry dn, up;   // dn: s_{s0-1} = g - h s_{s0}; up: s_{e0} = g - h s_{e0-1}
+        // the not-a-knot rows at either end, for the lanes that reach them
+        double fb = 0.0, fdg = 1.0, fud = 0.0, lb = 0.0, ldg = 1.0, lld = 0.0;
+        if (s0 <= kHaloMax) {
+            const double p = D(0), r = D(1), u = M(0), v = M(1), e = p + r;
+            fb = ((p + 2 * e) * r * u + p * p * v) / e;
+            fud = e;
+            fdg = r;
+        }
+        if (e0 + kHaloMax >= len) {
+            const double p = D(len - 3), r = D(len - 2), u = M(len - 3), v = M(len - 2), e = p + r;
+            lb = (r * r * u + (2 * e + r) * p * v) / e;
+            ldg = p;
+            lld = e;
+        }
+        double d1 = 0.0, m1 = 0.0;   // interval s0 - 1
+#pragma unroll 1
+        for (int halo = kHalo;; halo = kHaloMax) {
+            const int i0 = s0 - halo > 0 ? s0 - halo : 0, i9 = e0 + halo < len ? e0 + halo : len;
+            double down = 0.0, above = 0.0;   // damping
+            dn.h = dn.g = up.h = up.g = 0.0;
+            double a1 = 0.0, am = 0.0, c2 = 0.0, cm = 0.0;
+            if (s0 > 0) {
+                if (i0 == 0) {
+                    a1 = D(0);
+                    am = M(0);
+                    dn.step(0.0, fdg, fud, fb);
+                } else {
+                    const double b1 = D(i0 - 1), bm = M(i0 - 1);
+                    a1 = D(i0);
+                    am = M(i0);
+                    down = a1 * dn.step(0.0, 2 * (b1 + a1), b1, 3.0 * (a1 * bm + b1 * am));
+                }
+            }
+            if (e0 < len) {
+                c2 = D(i9 - 2);
+                cm = M(i9 - 2);
+                if (i9 == len) {
+                    up.step(0.0, ldg, lld, lb);
+                } else {
+                    const double b2 = D(i9 - 1), bm = M(i9 - 1);
+                    above = c2 * up.step(0.0, 2 * (c2 + b2), b2, 3.0 * (b2 * cm + c2 * bm));
+                }
+            }
+            // row i below: intervals i - 1 (a1, am) and i; row j above: j - 1 and j (c2, cm)
+#pragma unroll 4
+            for (int k = 1; k < halo; ++k) {
+                const int i = i0 + k, j = i9 - 1 - k;
+                if (i < s0) {
+                    const double d2 = D(i), m2 = M(i);
+                    down *= d2 * dn.step(d2, 2 * (a1 + d2), a1, 3.0 * (d2 * am + a1 * m2));
+                    a1 = d2;
+                    am = m2;
+                }
+                if (j >= e0) {
+                    const double d0 = D(j - 1), m0 = M(j - 1);
+                    above *= d0 * up.step(d0, 2 * (d0 + c2), c2, 3.0 * (c2 * m0 + d0 * cm));
+                    c2 = d0;
+                    cm = m0;
+                }
+            }
+            d1 = a1;
+            m1 = am;
+            if ((fabs(down) < kDamped && fabs(above) < kDamped) || halo == kHaloMax) break;
+        }
+        // the lane's rows, then back through them
+        double pcs[kOwn], pds[kOwn];
+#pragma unroll
+        for (int j = 0; j < kOwn; ++j) {
+            const int i = s0 + j;
+            if (i < e0) {
+                const int k = i < len - 1 ? i : len - 2;
+                const double d2 = D(k), m2 = M(k);
+                const bool first = i == 0, last = i == len - 1;
+                const double a = first ? 0.0 : (last ? lld : d2), dg = first ? fdg : (last ? ldg : 2 * (d1 + d2));
+                const double c = first ? fud : (last ? 0.0 : d1), r = first ? fb : (last ? lb : 3.0 * (d2 * m1 + d1 * m2));
+                dn.step(a, dg, c, r);
+                d1 = d2;
+                m1 = m2;
+            }
+            pcs[j] = dn.h;   // past the end: the last row's
+            pds[j] = dn.g;
+        }
+        // row e0 - 1: s = g - h s_{e0} with s_{e0} = up.g - up.h s
+        double xi = (dn.g - dn.h * up.g) / (1.0 - dn.h * up.h);
+        double xn = up.g - up.h * xi;
+        x[kOwn] = xn;
+#pragma unroll
+        for (int j = kOwn - 1; j >= 0; --j) {
+            const int i = s0 + j;
+            if (i < e0 - 1) xi = pds[j] - pcs[j] * xn;
+            x[j] = xi;
+            if (i < e0) xn = xi;
+        }
+    }
+    __syncthreads();   // every lane has read the slopes of its halos
+    // the knot slopes take the intervals' place: row i at word i - base
+    if (on) {
+        const int c0 = (tid & 63) * kOwn;
+#pragma unroll
+        for (int j = 0; j < kOwn; ++j) mq[q][tile_at(c0 + j)] = x[j];
+        if ((tid & 63) == 63) mq[q][tile_at(kTile)] = x[kOwn];   // the row past the tile
+    }
+    __syncthreads();
+    const int rows = len - base < kTile ? len - base : kTile;
+    const int p = tid % G;
+    for (int j = tid / G; j < rows; j += kTileThreads / G) {
+        const int i = base + j;
+        const double* y = Y + (size_t)G * i + p;
+        const double yi = y[0];
+        double c1 = 0.0, c2 = 0.0, c3 = 0.0;
+        if (i < len - 1) {
+            const double xi = mq[p][tile_at(j)], xn = mq[p][tile_at(j + 1)];
+            const double dt = dx[tile_at(i - lo)], rt = eob::refined_rcp(dt);
+            const auto over = [&](double v) { const double w = v * rt; return fma(fma(-dt, w, v), rt, w); };   // v / dt
+            const double slope = over(y[G] - yi);
+            const double tt = over(xi + xn - 2 * slope);
+            c1 = xi;
+            c2 = over(slope - xi) - tt;
+            c3 = over(tt);
+        }
+        double* c = C + (size_t)(4 * G) * i + 4 * p;
+        c[0] = yi;
+        c[1] = c1;
+        c[2] = c2;
+        c[3] = c3;
+    }
+}
+
+// ------------------------------------------ any number of series: sweeps
+// The higher modes' series and those of r and pr.  These feed the
+// merger-ringdown attachment, whose discrete choices (the knot of the
+// frequency's peak, the attachment sample) turn on the last bits of the
+// coefficients for some binaries, so their order of operations is kept.
 //
 // One wavefront per binary builds all of them.  Each interpolant's slope
 // system is split into P <= 64 / nser chunks of >= kChunkMin rows, one lane
@@ -793,7 +1014,17 @@ size_t eobhip_spline_scratch_doubles(int n, int max_step) {
 
 int eobhip_spline_build_batched(const double* dense, const double* knots, const int* num_steps, int n, int max_step, double* coef,
                                 double* scratch, void* stream) {
-    return eobhip_spline_build_series(dense, knots, num_steps, n, max_step, 3, coef, scratch, stream);
+    (void)scratch;   // the tiles need none
+    EOBHIP_REQUIRE(n >= 0 && max_step >= 1, "bad sizes");
+    for (int b = 0; b < n; b += 65535) {   // the grid's second dimension
+        const int nb = n - b < 65535 ? n - b : 65535;
+        hipLaunchKernelGGL(k_spline_build_tile, dim3(blocks_for(max_step, kTile), nb), dim3(kTileThreads), 0, as_stream(stream),
+                           dense + (size_t)b * max_step * 5, knots + (size_t)b * max_step * 3, num_steps + b, max_step,
+                           coef + (size_t)b * max_step * 12);
+        const int rc = check_launch("spline_build");
+        if (rc) return rc;
+    }
+    return EOBHIP_OK;
 }
 
 size_t eobhip_spline_series_scratch_doubles(int n, int max_step, int nser) {

@@ -1,4 +1,5 @@
-"""The spline drop-in at the edges of the rows a lane owns and of the halos, against the same not-a-knot system solved in extended precision, on even,
+"""The tiled spline builders at the edges of their tiles, of the rows a lane owns
+and of the halos, against the same not-a-knot system solved in extended precision, on even,
 trajectory-like, random and graded knots ("steep": the short halo is not enough).
 (scipy's own coefficients are 1.7e-10 off the extended-precision ones where
 graded spacings jump back to 1, so they are no oracle for these knots.)"""
@@ -6,7 +7,8 @@ import numpy as np
 import pytest
 import torch
 
-from eobgpu_amd import pytdinterp
+from eobgpu_amd import pipeline as P, pytdinterp
+from eobgpu_amd._lib import call, lib
 
 pytestmark = pytest.mark.gpu
 
@@ -60,6 +62,33 @@ def exact_slopes_error(t, y, got, nser):
             worst = max(worst, float(np.max(np.abs(got[:-1, 4 * q + k] - c[k - 1][:, q]) * dx ** k) / scale))
         assert np.array_equal(got[:, 4 * q], y[:, q])
     return worst
+
+
+@pytest.mark.parametrize("kind", ["even", "step", "random", "graded", "steep"])
+@pytest.mark.parametrize("nser", [3])
+def test_batched_builder_tile_edges(dev, kind, nser):
+    lens = [4, 5, 15, 16, 17, 33, 63, 96, 97, 130, 1023, 1024, 1025, 1040, 1089, 2048, 2051, 3000]
+    ms = max(lens)
+    rng = np.random.default_rng(nser)
+    n = len(lens)
+    dense, y = np.zeros((n, ms, 5)), np.zeros((n, ms, nser))
+    for i, m in enumerate(lens):
+        t = knots_of(kind, m, rng)
+        dense[i, :m, 0] = t
+        for q in range(nser):
+            y[i, :m, q] = np.sin(3 * t / t[-1] + q) + 0.1 * np.cos(17 * t / t[-1])
+    d, k = torch.tensor(dense, device=dev), torch.tensor(y, device=dev)
+    ns = torch.tensor(lens, dtype=torch.int32, device=dev)
+    coef = torch.full((n, ms, 4 * nser), 7.0, dtype=torch.float64, device=dev)
+    scratch = torch.empty(int(lib().eobhip_spline_scratch_doubles(n, ms)), dtype=torch.float64, device=dev)
+    call("eobhip_spline_build_batched", d.data_ptr(), k.data_ptr(), ns.data_ptr(), n, ms, coef.data_ptr(), scratch.data_ptr(),
+         P.current_stream())
+    got = coef.cpu().numpy()
+    for i, m in enumerate(lens):
+        assert np.all(got[i, m:] == 7.0)            # nothing past the binary's rows
+        assert np.all(got[i, m - 1].reshape(nser, 4)[:, 1:] == 0.0)
+        # a backward-stable solve: rounding of the slopes, at most a few hundred ulp on the steepest grading
+        assert exact_slopes_error(dense[i, :m, 0], y[i, :m], got[i, :m], nser) < 1e-12
 
 
 @pytest.mark.parametrize("kind", ["even", "random", "graded", "steep"])
