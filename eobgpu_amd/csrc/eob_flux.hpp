@@ -320,8 +320,9 @@ EOB_HD void flux_setup(ModeCoef* mc, WaveCoef& wc, double m1, double m2, double 
 //   is evaluated per mode (the reference raises exp(-4 pi H Omega) to the m-th power,
 //   the same number within rounding)
 // (templated on the scalar so the FP64 operation count can be taken with a counting type)
+// As two factors, whose product is the summand.
 template <class T>
-EOB_HD T flux_mode(const ModeCoef& z, T v, T logv, T H, T Omega, T Heff, T pphi, T vPhi2) {
+EOB_HD void flux_mode_factors(const ModeCoef& z, T v, T logv, T H, T Omega, T Heff, T pphi, T vPhi2, T& lead, T& newton) {
     const T hk = H * (double)z.m * Omega;
     const T x = 4.0 * kPi * hk;
     const T Em = exp(-x);
@@ -352,8 +353,14 @@ EOB_HD T flux_mode(const ModeCoef& z, T v, T logv, T H, T Omega, T Heff, T pphi,
     T rpl = ipow15(rho, z.l);   // l <= 8 and l + eps <= 9
     rpl = (z.flags & 2) ? aux : rpl + aux;
     const T S = (z.flags & 1) ? Heff : v * pphi;
-    const T hN2 = z.N2 * ipow15(vPhi2, z.lpe);
-    return z.m2 * Omega * Omega * T2 * S * S * rpl * rpl * hN2;
+    newton = z.N2 * ipow15(vPhi2, z.lpe);
+    lead = z.m2 * Omega * Omega * T2 * S * S * rpl * rpl;
+}
+template <class T>
+EOB_HD T flux_mode(const ModeCoef& z, T v, T logv, T H, T Omega, T Heff, T pphi, T vPhi2) {
+    T lead, newton;
+    flux_mode_factors(z, v, logv, H, Omega, Heff, pphi, vPhi2, lead, newton);
+    return lead * newton;
 }
 
 }  // namespace eob

@@ -151,20 +151,145 @@ __device__ void rr_force_dropin(const ModeCoef* hm, const double* add, int n, in
     F[1] = -f_over_om;
 }
 
-__global__ __launch_bounds__(kBlock) void k_ode_dropin(const double* arg, double* k, const double* add, int n, const ModeCoef* modes,
-                                                       const int* idx) {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const HamCoef c = ham_from_add(add, n, i);
-        const double r = arg[i], pr = arg[2 * n + i], L = arg[3 * n + i];
-        const Dual d0 = ham_tangent(c, r, pr, L, 0);
-        const double dHdpr = ham_tangent(c, r, pr, L, 1).d;
-        const double dHdL = ham_tangent(c, r, pr, L, 2).d;
-        double F[2];
-        rr_force_dropin(modes + (size_t)idx[i] * kNumModes, add, n, i, c, r, pr, L, dHdL, F);
-        k[i] = dHdpr;
-        k[n + i] = dHdL;
-        k[2 * n + i] = -d0.d + F[0];
-        k[3 * n + i] = -0.0 + F[1];
+// ------------------------------------------- the same over a block's wavefronts
+// Right-hand sides of up to kDropMax systems by one block.  With a lane per
+// system each evaluation walked four or five passes of the Hamiltonian and the
+// 35 flux modes in turn (54 us, whatever the batch up to one chip of lanes).
+// Here the first wavefront takes H's passes for all of the block's systems, then
+// every (system, mode) pair is a thread's, and a lane per system adds its 35
+// modes in their order, so that the numbers round as the lane-per-system kernel's
+// (the error estimate of a step is a sum that cancels to its last bits).
+constexpr int kDropMax = 64;
+constexpr int kOdeWaves = 5, kIcWaves = 6;
+struct DropLds {
+    double r[kDropMax], pr[kDropMax], L[kDropMax];   // in this order (ham_grad)
+    double pass[kIcWaves][kDropMax];
+    double v[kDropMax], logv[kDropMax], Hreal[kDropMax], omega[kDropMax], Heff[kDropMax], vPhi2[kDropMax], eta_f[kDropMax], h22c[kDropMax];
+    double lead[kNumModes][kDropMax], newton[kNumModes][kDropMax];
+};
+
+// systems per block: few while that spreads the batch over the chip's 256 CUs
+// (never fewer than 4: their 140 (system, mode) pairs are one round of the
+// block), at most a lane each.  One attempted step through the three drop-ins,
+// lane per system before and blocks now: 16 systems 820 and 249 us, 2048 1060
+// and 281, 16384 1140 and 526; past one chip of lanes a lane per system catches
+// up (65536: 1770 and 1860).
+inline int drop_systems(int n) {
+    int s = 4;
+    while (s < kDropMax && (long long)s * 256 < n) s *= 2;
+    return s;
+}
+
+// Flux of the block's S systems from i0 on, from the states and H's passes in
+// `lds` (visible to the block).  Every thread calls it; valid on lane s of
+// wavefront 0.
+enum DropPass { kPassR, kPassPr, kPassOmega, kPassOmc, kPassH, kPassHrr = kPassR, kPassHrL = kPassH + 1 };
+__device__ __attribute__((noinline)) double block_flux(DropLds& lds, const ModeCoef* modes, const int* idx, const double* add, int n, int i0,
+                                                       int S) {
+    const int s = threadIdx.x;
+    const bool mine = s < S && i0 + s < n;
+    if (mine) {
+        const int i = i0 + s;
+        const double r = lds.r[s], omega = lds.pass[kPassOmega][s], omc = lds.pass[kPassOmc][s];
+        const double nu = nu_of(add[i], add[n + i]);
+        double eta_f = nu;
+        if (eta_f > 0.25 && eta_f < 0.25 + 1e-4) eta_f = 0.25;
+        const double Hreal = nu * lds.pass[kPassH][s];
+        const double v = cbrt(omega), logv = log(v);
+        const double vPhiIn = 1.0 / (omc * omc * (r * r * r));
+        const double vPhi = r * cbrt(vPhiIn) * omega;
+        lds.v[s] = v;
+        lds.logv[s] = logv;
+        lds.Hreal[s] = Hreal;
+        lds.omega[s] = omega;
+        lds.vPhi2[s] = vPhi * vPhi;
+        lds.Heff[s] = (Hreal * Hreal - 1.0) / (2.0 * eta_f) + 1.0;
+        lds.eta_f[s] = eta_f;
+        lds.h22c[s] = add[9 * n + i];
+    }
+    __syncthreads();
+    const int shift = __ffs(S) - 1;   // S is a power of two
+    for (int e = threadIdx.x; e < S * kNumModes; e += blockDim.x) {
+        const int q = e & (S - 1), mi = e >> shift, i = i0 + q;
+        if (i < n) {
+            ModeCoef z = modes[(size_t)(idx ? idx[i] : i) * kNumModes + mi];
+            const double pre = add[(10 + 2 * mi) * n + i], pim = add[(11 + 2 * mi) * n + i];
+            const double y = ylm_abs_eq(z.l - (z.lpe - z.l), z.m);
+            z.N2 = (pre * pre + pim * pim) * y * y;
+            if (mi == 1) z.c[10] = lds.h22c[q];
+            int fl = ((z.l + z.m) & 1) ? 0 : 1;
+            if (lds.eta_f[q] == 0.25 && (z.m & 1)) fl |= 2;
+            z.flags = fl;
+            flux_mode_factors(z, lds.v[q], lds.logv[q], lds.Hreal[q], lds.omega[q], lds.Heff[q], lds.L[q], lds.vPhi2[q], lds.lead[mi][q],
+                              lds.newton[mi][q]);
+        }
+    }
+    __syncthreads();
+    double sum = 0.0;
+    if (mine)
+        for (int mi = 0; mi < kNumModes; ++mi) sum += lds.lead[mi][s] * lds.newton[mi][s];
+    return sum / kPi / 8.0;
+}
+
+// H and its derivatives at the state and dH/dpphi at pr = 0, the passes of the
+// right-hand side.  A function of its own with its state read inside, so that it
+// is compiled with the coefficients in one basic block whoever calls it: the
+// compiler chooses which products of a block to fuse with their sums by what
+// else the block holds, and the lane-per-system kernel's rounding is kept.
+// (Passes on wavefronts of their own are 20% faster at 16 systems, but then
+// dH/dr rounds differently for one system in 2000.)
+__device__ __attribute__((noinline)) void ham_grad(const double* add, int n, int i, const double* at, double* out) {
+    const double r = at[0], pr = at[kDropMax], L = at[2 * kDropMax];
+    const HamCoef c = ham_from_add(add, n, i);
+    out[0] = ham_tangent(c, r, pr, L, 0).d;
+    out[kDropMax] = ham_tangent(c, r, pr, L, 1).d;
+    out[2 * kDropMax] = ham_tangent(c, r, pr, L, 2).d;
+    out[3 * kDropMax] = ham_tangent(c, r, pr, L, 3).d;
+    out[4 * kDropMax] = ham_eval<double>(c, r, pr, L);
+}
+// k1 .. k4 of the block's systems at the states in lds.r, pr, L (visible to the
+// block); nu is this lane's system's.  Valid on lane s of wavefront 0.
+__device__ __forceinline__ void block_rhs(DropLds& lds, double nu, const ModeCoef* modes, const int* idx,
+                                          const double* add, int n, int i0, int S, int s, int wave, bool on, double k[4]) {
+    if (on) {
+        if (wave == 0) ham_grad(add, n, i0 + s, lds.r + s, &lds.pass[kPassR][s]);
+    }
+    __syncthreads();
+    double flux = block_flux(lds, modes, idx, add, n, i0, S);
+    if (wave == 0 && on) {
+        const double pr = lds.pr[s], L = lds.L[s], omega = lds.pass[kPassOmega][s];
+        flux /= nu;
+        const double f_over_om = flux / omega;
+        k[0] = lds.pass[kPassPr][s];
+        k[1] = omega;
+        k[2] = fma(-pr / L, f_over_om, -lds.pass[kPassR][s]);
+        k[3] = -0.0 + -f_over_om;
+    }
+}
+
+__global__ __launch_bounds__(64 * kOdeWaves) void k_ode_dropin(const double* arg, double* k, const double* add, int n, const ModeCoef* modes,
+                                                               const int* idx, int S) {
+    __shared__ DropLds lds;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), s = threadIdx.x & 63;
+    const int i0 = blockIdx.x * S, i = i0 + s;
+    const bool on = s < S && i < n;
+    double nu = 1.0;
+    if (on) {
+        nu = nu_of(add[i], add[n + i]);
+        if (wave == 0) {
+            lds.r[s] = arg[i];
+            lds.pr[s] = arg[2 * n + i];
+            lds.L[s] = arg[3 * n + i];
+        }
+    }
+    __syncthreads();
+    double kk[4];
+    block_rhs(lds, nu, modes, idx, add, n, i0, S, s, wave, on, kk);
+    if (wave == 0 && on) {
+        k[i] = kk[0];
+        k[n + i] = kk[1];
+        k[2 * n + i] = kk[2];
+        k[3 * n + i] = kk[3];
     }
 }
 
@@ -281,29 +406,72 @@ __global__ __launch_bounds__(kBlock) void k_ic_diss(double* out, const double* p
     }
 }
 
-// root_find_scalar_all (src/EOB.cu:2712-2834), one binary per thread: false
-// position on IC_diss(pr) from start_bounds [2][n]; it stops when |IC_diss(c)| <
-// err or after max_iter steps.  The caller's args and additional args are read only.
-__global__ __launch_bounds__(kBlock) void k_root_find_scalar_all(double* pr_res, const double* bounds, const double* args,
-                                                                 const double* add, int max_iter, double err, int n,
-                                                                 const ModeCoef* modes) {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const HamCoef c = ham_from_add(add, n, i);
-        const ModeCoef* hm = modes + (size_t)i * kNumModes;
-        const double r = args[i], L = args[3 * n + i];
-        double a = bounds[i], b = bounds[n + i], g[4], F[2];
-        double fa = ic_diss_dev(hm, add, n, i, c, r, a, L, g, F);
-        double fb = ic_diss_dev(hm, add, n, i, c, r, b, L, g, F);
-        double cc = 0.0;
-        for (int it = 0; it < max_iter; ++it) {
-            cc = (a * fb - b * fa) / (fb - fa);
-            const double fc = ic_diss_dev(hm, add, n, i, c, r, cc, L, g, F);
-            if ((fb < 0.0 && fc < 0.0) || (fb >= 0.0 && fc >= 0.0)) { b = cc; fb = fc; }
-            else { a = cc; fa = fc; }
-            if (fabs(fc) < err) break;
+// root_find_scalar_all (src/EOB.cu:2712-2834): false position on IC_diss(pr) from
+// start_bounds [2][n]; it stops when |IC_diss(c)| < err or after max_iter steps.
+// The caller's args and additional args are read only.  S binaries per block,
+// IC_diss evaluated by its six wavefronts (the two second derivatives of H, its
+// tangents and its value side by side, then the flux modes); the block ends with its last binary.  1024 binaries: 320
+// us with a lane per binary, 53 us now.
+__global__ __launch_bounds__(64 * kIcWaves) void k_root_find_scalar_all(double* pr_res, const double* bounds, const double* args,
+                                                                        const double* add, int max_iter, double err, int n,
+                                                                        const ModeCoef* modes, int S) {
+    __shared__ DropLds lds;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), s = threadIdx.x & 63;
+    const int i0 = blockIdx.x * S, i = i0 + s;
+    const bool on = s < S && i < n, mine = on && wave == 0;
+    HamCoef c{};
+    double nu = 1.0, r = 1.0, L = 1.0, a = 0.0, b = 0.0, fa = 0.0, fb = 0.0, cc = 0.0;
+    if (on) {
+        c = ham_from_add(add, n, i);
+        nu = nu_of(add[i], add[n + i]);
+        r = args[i];
+        L = args[3 * n + i];
+        a = bounds[i];
+        b = bounds[n + i];
+        if (wave == 0) {
+            lds.r[s] = r;
+            lds.L[s] = L;
         }
-        pr_res[i] = cc;
     }
+    bool live = mine;
+    // evaluations 0 and 1 are the bounds', then one per step
+    for (long long ev = 0; ev < 2 + (long long)max_iter; ++ev) {
+        if (live) {
+            if (ev >= 2) cc = (a * fb - b * fa) / (fb - fa);
+            lds.pr[s] = ev == 0 ? a : (ev == 1 ? b : cc);
+        }
+        __syncthreads();
+        if (on) {
+            const double pr = lds.pr[s];
+            double x;
+            switch (wave) {
+                case kPassHrr: x = ham_second(c, r, pr, L, 0, 0); break;
+                case kPassPr: x = ham_tangent(c, r, pr, L, 1).d; break;
+                case kPassOmega: x = ham_tangent(c, r, pr, L, 2).d; break;
+                case kPassOmc: x = ham_tangent(c, r, pr, L, 3).d; break;
+                case kPassH: x = ham_eval<double>(c, r, pr, L); break;
+                default: x = ham_second(c, r, pr, L, 0, 3); break;
+            }
+            lds.pass[wave][s] = x;
+        }
+        __syncthreads();
+        double flux = block_flux(lds, modes, nullptr, add, n, i0, S);
+        if (live) {
+            flux /= nu;
+            const double F1 = -(flux / lds.pass[kPassOmega][s]);
+            const double dLdr = -lds.pass[kPassHrr][s] / lds.pass[kPassHrL][s];
+            const double fc = F1 / dLdr - lds.pass[kPassPr][s];
+            if (ev == 0) fa = fc;
+            else if (ev == 1) fb = fc;
+            else {
+                if ((fb < 0.0 && fc < 0.0) || (fb >= 0.0 && fc >= 0.0)) { b = cc; fb = fc; }
+                else { a = cc; fa = fc; }
+                if (fabs(fc) < err) live = false;
+            }
+        }
+        if (!__syncthreads_or(live)) break;
+    }
+    if (mine) pr_res[i] = cc;
 }
 
 __global__ __launch_bounds__(kBlock) void k_update_info(ModeCoef* modes, WaveCoef* wave, const double* m1, const double* m2,
@@ -358,23 +526,53 @@ __global__ __launch_bounds__(kBlock) void k_hlm_dropin(double* out, const double
 // ak_term = sum_j a_sj k_j accumulated from 0 in stage order; arg = solOld + h ak;
 // xCurrent = x + c_s h.  (src/DOPR853.cu:197-355, 381-516)
 struct StagePtrs {
-    const double* k[11];
+    double* k[12];   // where stage s leaves its k; later stages read it there
 };
 __constant__ double dA[12][12] = DOP_A;
-__global__ __launch_bounds__(kBlock) void k_stage_arg(double* arg, const double* solOld, const double* x, double* xCur, double* ak,
-                                                      const double* h, StagePtrs kp, int stage, int nargs, int n) {
-    for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < n; e += gridDim.x * blockDim.x) {
-        const double hh = h[e];
-        xCur[e] = x[e] + dC[stage] * hh;
-        for (int j = 0; j < nargs; ++j) {
+// All twelve stages of one attempted step for S systems per block: lane (s, j) of
+// the first wavefronts forms component j's argument, then block_rhs.  With two
+// launches per stage and a lane per system the 24 launches took 720 us for 16
+// systems; now one launch of 160 us.
+__global__ __launch_bounds__(64 * kOdeWaves) void k_dopr_steps(double* arg, const double* solOld, const double* x, double* xCur, double* ak,
+                                                               const double* h, StagePtrs kp, int n, const double* add,
+                                                               const ModeCoef* modes, const int* idx, int S) {
+    __shared__ DropLds lds;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), s = threadIdx.x & 63;
+    const int i0 = blockIdx.x * S, i = i0 + s;
+    const bool on = s < S && i < n;
+    double nu = 1.0, hh = 0.0;
+    if (on) {
+        nu = nu_of(add[i], add[n + i]);
+        hh = h[i];
+    }
+    for (int stage = 0; stage < 12; ++stage) {
+        if (on && wave < 4) {
             double acc = 0.0;
             for (int q = 0; q < stage; ++q) {
                 const double a = dA[stage][q];
-                if (a != 0.0) acc += a * kp.k[q][j * n + e];
+                if (a != 0.0) acc += a * kp.k[q][(size_t)wave * n + i];
             }
-            ak[j * n + e] = acc;
-            arg[j * n + e] = solOld[j * n + e] + hh * acc;
+            const double v = solOld[(size_t)wave * n + i] + hh * acc;
+            ak[(size_t)wave * n + i] = acc;
+            arg[(size_t)wave * n + i] = v;
+            if (wave == 0) {
+                xCur[i] = x[i] + dC[stage] * hh;
+                lds.r[s] = v;
+            }
+            if (wave == 2) lds.pr[s] = v;
+            if (wave == 3) lds.L[s] = v;
         }
+        __syncthreads();   // also: every read of this stage's k's is done before one is overwritten
+        double kk[4];
+        block_rhs(lds, nu, modes, idx, add, n, i0, S, s, wave, on, kk);
+        if (wave == 0 && on) {
+            double* o = kp.k[stage];
+            o[i] = kk[0];
+            o[n + i] = kk[1];
+            o[2 * n + i] = kk[2];
+            o[3 * n + i] = kk[3];
+        }
+        __syncthreads();   // the stage's k is in memory for the block's other wavefronts
     }
 }
 
@@ -1345,8 +1543,9 @@ int eobhip_seobnr_root_find_scalar_all(eobhip_seobnr_t h, double* pr_res, const 
     EOBHIP_REQUIRE(num_args == 4 && num_add_args == kNAdd, "root_find_scalar_all: 4 args and 80 additional args per binary");
     EOBHIP_REQUIRE(numBinAll >= 0 && numBinAll <= h->numSys && max_iter >= 0, "bad sizes");
     if (numBinAll == 0) return EOBHIP_OK;
-    hipLaunchKernelGGL(k_root_find_scalar_all, dim3(blocks_for(numBinAll, kBlock)), dim3(kBlock), 0, as_stream(stream), pr_res,
-                       start_bounds, argsIn, add, max_iter, err, numBinAll, h->modes);
+    const int S = drop_systems(numBinAll);
+    hipLaunchKernelGGL(k_root_find_scalar_all, dim3(blocks_for(numBinAll, S)), dim3(64 * kIcWaves), 0, as_stream(stream), pr_res,
+                       start_bounds, argsIn, add, max_iter, err, numBinAll, h->modes, S);
     return check_launch("root_find_scalar_all");
 }
 
@@ -1355,8 +1554,9 @@ int eobhip_seobnr_ODE_Ham_align_AD(eobhip_seobnr_t h, const double* x, const dou
     (void)x;
     EOBHIP_REQUIRE(h && h->allocated, "ODE_Ham_align_AD: update_information has not been called");
     if (numSys == 0) return EOBHIP_OK;
-    hipLaunchKernelGGL(k_ode_dropin, dim3(blocks_for(numSys, kBlock)), dim3(kBlock), 0, as_stream(stream), arg, k, add, numSys, h->modes,
-                       idx);
+    const int S = drop_systems(numSys);
+    hipLaunchKernelGGL(k_ode_dropin, dim3(blocks_for(numSys, S)), dim3(64 * kOdeWaves), 0, as_stream(stream), arg, k, add, numSys, h->modes,
+                       idx, S);
     return check_launch("ODE_Ham_align_AD");
 }
 
@@ -1388,20 +1588,13 @@ int eobhip_dormandPrinceSteps(double* x, double* xCurrent, double* solOld, doubl
     hipStream_t st = as_stream(stream);
     // stage s result buffers in reference order: stages 1..10 -> k1..k10, 11 -> k2, 12 -> k3
     double* outs[12] = {k1, k2, k3, k4, k5, k6, k7, k8, k9, k10, k2, k3};
+    // stage 12 reads stage 11 from k2 and stage 2 never enters it (a_12,2 = 0)
     StagePtrs kp;
-    const double* ins[11] = {k1, k2, k3, k4, k5, k6, k7, k8, k9, k10, k2};
-    for (int q = 0; q < 11; ++q) kp.k[q] = ins[q];
-    const unsigned nb = blocks_for(numEq, kBlock);
-    for (int s = 0; s < 12; ++s) {
-        // stage 12 reads stage 11 from k2 (ins[10]) and stage 2 never enters it (a_12,2 = 0)
-        hipLaunchKernelGGL(k_stage_arg, dim3(nb), dim3(kBlock), 0, st, arg, solOld, x, xCurrent, ak, h, kp, s, nargs, numEq);
-        int rc = check_launch("stage args");
-        if (rc) return rc;
-        hipLaunchKernelGGL(k_ode_dropin, dim3(nb), dim3(kBlock), 0, st, arg, outs[s], add, numEq, ode->modes, idx);
-        rc = check_launch("stage rhs");
-        if (rc) return rc;
-    }
-    return EOBHIP_OK;
+    for (int q = 0; q < 12; ++q) kp.k[q] = outs[q];
+    const int S = drop_systems(numEq);
+    hipLaunchKernelGGL(k_dopr_steps, dim3(blocks_for(numEq, S)), dim3(64 * kOdeWaves), 0, st, arg, solOld, x, xCurrent, ak, h, kp, numEq, add,
+                       ode->modes, idx, S);
+    return check_launch("dormandPrinceSteps");
 }
 
 int eobhip_error_tol(double* err, const double* solOld, double* solNew, const double* h, const double* k1, const double* k2,
