@@ -16,7 +16,7 @@
 
 #include "eob_fastmath.hpp"
 #include "eobhip_common.hpp"
-#include "knot_window.hpp"
+#include "resample.hpp"
 #include "spline_nak.hpp"
 
 using namespace eobhip_detail;
@@ -591,80 +591,37 @@ __global__ __launch_bounds__(kSplineLanes) void k_spline_build_seg(const double*
 
 // Uniform resample of h+ = amp * Re[(Re S + i Im S)(t) e^{-2 i phi(t)}] at
 // t_j = t_0 + j dT_M (dT_M = dt / (M MTSUN)), j < N_b = floor((t_last - t_0)/dT_M) + 1,
-// zero for N_b <= j < N.  Interval: searchsorted(t, t_j, 'right') - 1 over the knots
-// (eob/seobnrv4phm.py:241-272).  grid (blocks, binaries); a block takes spans of
-// kResSpan consecutive samples, stages the knot times of their intervals in LDS
-// (knot_window) and each thread searches there.
-constexpr int kResPerThread = 16;
-constexpr int kResSpan = kBlock * kResPerThread;
-constexpr int kResSearch = 4;   // samples per thread whose knot searches run together
-static_assert(kResPerThread % kResSearch == 0, "kResSearch divides kResPerThread");
+// zero for N_b <= j < N; hx is the imaginary part, the two series the reference
+// transforms (eob/seobnrv4phm.py:720, 742-744).  grid (blocks, binaries), a run
+// of samples per wavefront (resample.hpp).  Bound by the writes: 256 binaries x
+// 2^20 samples, 15% of them inside a template: h+ 593 us with knot windows per
+// block, 412 now (a fill of the same memory 340).
+// samples with a value: floor((t_last - t_0) / dT) + 1, at most N
+__device__ __forceinline__ long long series_samples(const double* T, int len, double dT, int N) {
+    if (len < 2) return 0;
+    const long long nb = (long long)((T[5 * (len - 1)] - T[0]) / dT) + 1;
+    return nb > N ? N : nb;
+}
+
 __global__ __launch_bounds__(kBlock) void k_resample_hplus(const double* __restrict__ dense, const double* __restrict__ coef,
                                                            const int* __restrict__ num_steps, const double* __restrict__ amp,
-                                                           const double* __restrict__ dT_M, int n, int max_step, int N,
+                                                           const double* __restrict__ dT_M, int max_step, int N,
                                                            double* __restrict__ hplus, int* __restrict__ nsamp,
                                                            double* __restrict__ hcross) {
     const int b = blockIdx.y;
     const int len = num_steps[b];
-    double* out = hplus + (size_t)b * N;
-    double* outc = hcross ? hcross + (size_t)b * N : nullptr;
-    if (len < 2) {
-        for (long long j = (long long)blockIdx.x * blockDim.x + threadIdx.x; j < N; j += (long long)gridDim.x * blockDim.x) {
-            out[j] = 0.0;
-            if (outc) outc[j] = 0.0;
-        }
-        if (blockIdx.x == 0 && threadIdx.x == 0) nsamp[b] = 0;
-        return;
-    }
     const double* T = dense + (size_t)b * max_step * 5;
-    const double* C = coef + (size_t)b * max_step * 12;
-    const double t0 = T[0], tl = T[5 * (len - 1)];
     const double dT = dT_M[b];
-    long long nb = (long long)((tl - t0) / dT) + 1;
-    if (nb > N) nb = N;
+    const long long nb = series_samples(T, len, dT, N);
     if (blockIdx.x == 0 && threadIdx.x == 0) nsamp[b] = (int)nb;
-    const double a = amp[b];
-    __shared__ KnotWindow<kBlock> win;
-    const long long nspan = ((long long)N + kResSpan - 1) / kResSpan;
-    for (long long sp0 = blockIdx.x; sp0 < nspan; sp0 += gridDim.x) {   // the same trip count on every thread
-        const long long j0 = sp0 * kResSpan;
-        if (j0 < nb) {
-            const long long jmax = (j0 + kResSpan < nb ? j0 + kResSpan : nb) - 1;
-            knot_window<kBlock>(win, T, 5, len, t0 + (double)j0 * dT, t0 + (double)jmax * dT);
-        }
-        for (int u0 = 0; u0 < kResPerThread; u0 += kResSearch) {
-            double tj[kResSearch];
-            int ind[kResSearch];
-#pragma unroll
-            for (int k = 0; k < kResSearch; ++k) tj[k] = t0 + (double)(j0 + (long long)(u0 + k) * kBlock + threadIdx.x) * dT;
-            if (j0 < nb) knot_intervals<kBlock, kResSearch>(win, T, 5, len, tj, ind);
-#pragma unroll
-            for (int k = 0; k < kResSearch; ++k) {
-                const long long j = j0 + (long long)(u0 + k) * kBlock + threadIdx.x;
-                if (j < N) {
-                    double val = 0.0, valc = 0.0;
-                    if (j < nb) {
-                        double tk, c[12];
-                        interval_row<12>(T, 5, C, ind[k], tk, c);
-                        const double x = tj[k] - tk;
-                        const double x2 = x * x, x3 = x2 * x;
-                        const double ph = c[0] + c[1] * x + c[2] * x2 + c[3] * x3;
-                        const double sr = c[4] + c[5] * x + c[6] * x2 + c[7] * x3;
-                        const double si = c[8] + c[9] * x + c[10] * x2 + c[11] * x3;
-                        double sp, cp;
-                        sincos(2.0 * ph, &sp, &cp);
-                        // the template (sr + i si)(cos 2ph - i sin 2ph); h+ and hx are its real and
-                        // imaginary parts, the series the reference transforms (eob/seobnrv4phm.py:720, 742-744)
-                        val = a * (sr * cp + si * sp);
-                        valc = a * (si * cp - sr * sp);
-                    }
-                    out[j] = val;
-                    if (outc) outc[j] = valc;
-                }
-            }
-        }
-        __syncthreads();   // the window is rewritten by the next span
-    }
+    const SeriesOut o{hplus + (size_t)b * N, hcross ? hcross + (size_t)b * N : nullptr, amp[b], nb, N};
+    const double* C = coef + (size_t)b * max_step * 12;
+    const double t0 = T[0];
+    for_runs(N, kBlock / 64, [&](long long j0) {
+        if (j0 < nb)
+            h22_rows(T, C, len, t0, dT, j0, nb, [&](long long j, const double (&re)[2], const double (&im)[2], bool full) { o.put(j, re, im, full); });
+        o.zeros(j0);
+    });
 }
 
 // Uniform resample of the mode sum h = amp sum_j S_j(t) e^{-i m_j phi(t)} (the
@@ -678,97 +635,77 @@ struct ModeMs {
     int nm;
     int m[15];
 };
-// One sample's mode sum: row holds the interval's coefficients (Re of each
-// mode, Im of each mode, phi; 4 per series).  e^{-i m phi} is m - 1 products
-// with e^{-i phi} (the products a table of the powers would hold, without a
-// per-mode select from the table).
+// One sample's sum from a row (Re of each mode, Im of each mode, phi; 4
+// coefficients per series).  e^{-i m phi} is m - 1 products with e^{-i phi} (the
+// products a table of the powers would hold, without a per-mode select from the
+// table).  NMT > 0: built for that many modes (the loop over modes unrolled); 0:
+// any.
 template <int NMT, class Ptr>
-__device__ __forceinline__ void modes_sample(Ptr row, double x, double x2, double x3, int nm, const ModeMs& mm, double& hr,
-                                             double& hi) {
-    Ptr cp = row + 4 * (2 * nm);
-    const double ph = cp[0] + cp[1] * x + cp[2] * x2 + cp[3] * x3;
+__device__ __forceinline__ void modes_sample(Ptr c, double x, int nm, const ModeMs& mm, double& hr, double& hi) {
+    const double x2 = x * x, x3 = x2 * x;
+    const auto cubic = [&](Ptr p) { return p[0] + p[1] * x + p[2] * x2 + p[3] * x3; };
     double sp, cph;
-    sincos(ph, &sp, &cph);
+    sincos_phase(cubic(c + 4 * (2 * nm)), &sp, &cph);
+    hr = hi = 0.0;
 #pragma unroll
     for (int q = 0; q < (NMT > 0 ? NMT : nm); ++q) {
-        Ptr cr = row + 4 * q;
-        Ptr ci = row + 4 * (nm + q);
-        const double sr = cr[0] + cr[1] * x + cr[2] * x2 + cr[3] * x3;
-        const double si = ci[0] + ci[1] * x + ci[2] * x2 + ci[3] * x3;
-        double pr_ = cph, pi_ = -sp;   // e^{-i phi}
+        const double re = cubic(c + 4 * q), im = cubic(c + 4 * (nm + q));
+        double pr = cph, pi = -sp;   // e^{-i phi}
         for (int k = 1; k < mm.m[q]; ++k) {
-            const double t = pr_ * cph + pi_ * sp;
-            pi_ = pi_ * cph - pr_ * sp;
-            pr_ = t;
+            const double t = pr * cph + pi * sp;
+            pi = pi * cph - pr * sp;
+            pr = t;
         }
-        hr += sr * pr_ - si * pi_;
-        hi += sr * pi_ + si * pr_;
+        hr += re * pr - im * pi;
+        hi += re * pi + im * pr;
     }
 }
 
-// NMT > 0: built for that many modes (the loop over modes unrolled); 0: any.
-// When all lanes of a wavefront sample one knot interval, its coefficient row
-// is read once through the scalar cache (constant address space: the table
-// is read-only while the kernel runs).
+// Rows are read through the scalar cache sample by sample (the 44 coefficients
+// of five modes do not fit the scalar registers).  Five modes of 512 binaries x
+// 2^20, 18% of the samples inside a template: 2470 us with knot windows per
+// block, 1519 now (the writes alone 1360).
 template <int NMT>
 __global__ __launch_bounds__(kBlock) void k_resample_modes(const double* __restrict__ dense, const double* __restrict__ coef,
                                                            const int* __restrict__ num_steps, const double* __restrict__ amp,
                                                            const double* __restrict__ dT_M, int max_step, int N, ModeMs mm,
                                                            double* __restrict__ hplus, double* __restrict__ hcross,
                                                            int* __restrict__ nsamp) {
-    typedef const __attribute__((address_space(4))) double* ConstPtr;
     const int b = blockIdx.y;
     const int len = num_steps[b];
-    const int nm = NMT > 0 ? NMT : mm.nm, S = 2 * nm + 1, cs = 4 * S;
-    double* out = hplus + (size_t)b * N;
-    double* outc = hcross + (size_t)b * N;
-    if (len < 2) {
-        for (long long j = (long long)blockIdx.x * blockDim.x + threadIdx.x; j < N; j += (long long)gridDim.x * blockDim.x) {
-            out[j] = 0.0;
-            outc[j] = 0.0;
-        }
-        if (blockIdx.x == 0 && threadIdx.x == 0) nsamp[b] = 0;
-        return;
-    }
+    const int nm = NMT > 0 ? NMT : mm.nm;
+    const int cs = 4 * (2 * nm + 1);
     const double* T = dense + (size_t)b * max_step * 5;
     const double* C = coef + (size_t)b * max_step * cs;
-    const double t0 = T[0], tl = T[5 * (len - 1)];
-    const double dT = dT_M[b];
-    long long nb = (long long)((tl - t0) / dT) + 1;
-    if (nb > N) nb = N;
+    const double dT = dT_M[b], t0 = T[0];
+    const long long nb = series_samples(T, len, dT, N);
     if (blockIdx.x == 0 && threadIdx.x == 0) nsamp[b] = (int)nb;
-    const double a = amp[b];
-    __shared__ KnotWindow<kBlock> win;
-    const long long nspan = ((long long)N + kResSpan - 1) / kResSpan;
-    for (long long sp0 = blockIdx.x; sp0 < nspan; sp0 += gridDim.x) {
-        const long long j0 = sp0 * kResSpan;
-        if (j0 < nb) {
-            const long long jmax = (j0 + kResSpan < nb ? j0 + kResSpan : nb) - 1;
-            knot_window<kBlock>(win, T, 5, len, t0 + (double)j0 * dT, t0 + (double)jmax * dT);
-        }
-        for (int u = 0; u < kResPerThread; ++u) {
-            const long long j = j0 + (long long)u * kBlock + threadIdx.x;
-            if (j >= N) break;
-            double hr = 0.0, hi = 0.0;
-            if (j < nb) {
-                const double tj = t0 + (double)j * dT;
-                const int ind = knot_interval<kBlock>(win, T, 5, len, tj);
-                const int i0 = __builtin_amdgcn_readfirstlane(ind);
-                if (__all(ind == i0)) {
-                    const double x = tj - ((ConstPtr)T)[5 * (size_t)i0];
-                    modes_sample<NMT>((ConstPtr)(C + (size_t)cs * i0), x, x * x, x * x * x, nm, mm, hr, hi);
-                } else {
-                    const double x = tj - T[5 * (size_t)ind];
-                    modes_sample<NMT>(C + (size_t)cs * ind, x, x * x, x * x * x, nm, mm, hr, hi);
-                }
-                hr *= a;
-                hi *= a;
-            }
-            out[j] = hr;
-            outc[j] = hi;
-        }
-        __syncthreads();   // the window is rewritten by the next span
-    }
+    const SeriesOut o{hplus + (size_t)b * N, hcross + (size_t)b * N, amp[b], nb, N};
+    for_runs(N, kBlock / 64, [&](long long j0) {
+        ConstPtr c = nullptr;
+        double tk = 0.0;
+        if (j0 < nb)
+            resample_rows(
+                T, len, j0, nb, [&](long long j) { return t0 + (double)j * dT; },
+                [&](int i) {
+                    c = (ConstPtr)(C + (size_t)cs * i);
+                    tk = ((ConstPtr)T)[5 * (size_t)i];
+                },
+                [&](long long j, double ta, double tb, bool full) {
+                    double re[2], im[2];
+                    modes_sample<NMT>(c, ta - tk, nm, mm, re[0], im[0]);
+                    modes_sample<NMT>(c, tb - tk, nm, mm, re[1], im[1]);
+                    o.put(j, re, im, full);
+                },
+                [&](long long j, double ta, double tb, int ia, int ib) {
+                    double re[2], im[2];
+                    one_by_one(ta, tb, ia, ib, re, im, [&](double t, int i, double& x, double& y) {
+                        modes_sample<NMT>(C + (size_t)cs * i, t - T[5 * (size_t)i], nm, mm, x, y);
+                    });
+                    o.put(j, re, im, false);
+                });
+        o.zeros(j0);
+    });
 }
 
 // TD2 (src/interpolate.cu:441-549), TDInterp_wrap2's kernel: per binary b and
@@ -1046,10 +983,9 @@ int eobhip_resample_hplus(const double* dense, const double* coef, const int* nu
                           int max_step, int N, double* hplus, int* nsamp, void* stream) {
     EOBHIP_REQUIRE(n >= 0 && N >= 1 && n <= 65535, "bad sizes");
     if (n == 0) return EOBHIP_OK;
-    int bx = (int)((N + (long long)kResSpan - 1) / kResSpan);
-    if (bx > 4096) bx = 4096;
-    hipLaunchKernelGGL(k_resample_hplus, dim3(bx, n), dim3(kBlock), 0, as_stream(stream), dense, coef, num_steps, amp, dT_M, n, max_step, N,
-                       hplus, nsamp, nullptr);
+    const int bx = resample_blocks(N, n);
+    hipLaunchKernelGGL(k_resample_hplus, dim3(bx, n), dim3(kBlock), 0, as_stream(stream), dense, coef, num_steps, amp, dT_M, max_step, N, hplus,
+                       nsamp, nullptr);
     return check_launch("resample_hplus");
 }
 
@@ -1065,8 +1001,7 @@ int eobhip_resample_modes(const double* dense, const double* coef, const int* nu
         mm.m[q] = ms[q];
     }
     if (n == 0) return EOBHIP_OK;
-    int bx = (int)((N + (long long)kResSpan - 1) / kResSpan);
-    if (bx > 4096) bx = 4096;
+    const int bx = resample_blocks(N, n);
     // built for the reference's five modes and for (2,2) alone; any other count runs the general build
     if (nm == 5)
         hipLaunchKernelGGL(k_resample_modes<5>, dim3(bx, n), dim3(kBlock), 0, as_stream(stream), dense, coef, num_steps, amp, dT_M,
@@ -1101,10 +1036,9 @@ int eobhip_resample_hpc(const double* dense, const double* coef, const int* num_
     EOBHIP_REQUIRE(n >= 0 && N >= 1 && n <= 65535, "bad sizes");
     EOBHIP_REQUIRE(hcross != nullptr, "hcross is required");
     if (n == 0) return EOBHIP_OK;
-    int bx = (int)((N + (long long)kResSpan - 1) / kResSpan);
-    if (bx > 4096) bx = 4096;
-    hipLaunchKernelGGL(k_resample_hplus, dim3(bx, n), dim3(kBlock), 0, as_stream(stream), dense, coef, num_steps, amp, dT_M, n, max_step, N,
-                       hplus, nsamp, hcross);
+    const int bx = resample_blocks(N, n);
+    hipLaunchKernelGGL(k_resample_hplus, dim3(bx, n), dim3(kBlock), 0, as_stream(stream), dense, coef, num_steps, amp, dT_M, max_step, N, hplus,
+                       nsamp, hcross);
     return check_launch("resample_hpc");
 }
 
