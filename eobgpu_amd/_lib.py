@@ -119,6 +119,7 @@ _SIGS.update({
     "eobhip_lik_sizes": [c_vp, c_vp, c_vp, c_int, c_int, c_int, c_int, c_vp, c_vp, c_vp],
     "eobhip_lik_partial_blocks": [c_int, ctypes.POINTER(c_int), ctypes.POINTER(c_int)],
     "eobhip_lik_resample": [c_vp] * 8 + [c_int, c_int, c_int, c_vp, c_vp, c_vp, c_vp],
+    "eobhip_lik_evaluate": [c_vp] * 8 + [c_int] * 4 + [c_vp, c_vp, c_int] + [c_vp] * 7 + [c_double, c_vp, c_vp, c_vp],
     "eobhip_lik_finish": [c_vp, c_vp, c_vp, c_int, c_int, c_int, c_vp, c_vp, c_vp, c_vp, c_double, c_vp, c_vp, c_vp],
 })
 _RESTYPES["eobhip_lik_bank_doubles"] = c_size

@@ -29,12 +29,13 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "eobhip_common.hpp"
+
 namespace eobhip_detail {
 
 constexpr int kFftThreads = 512;
 constexpr int kFftPoints = 16 * kFftThreads;
-constexpr int kFftMinLog2 = 10;      // N
-constexpr int kFftMaxLog2 = 21;
+constexpr int kFftMinLog2 = kRfftMinLog2, kFftMaxLog2 = kRfftMaxLog2;   // N
 constexpr int kFftOneMaxLog2 = 14;   // N whose H = N/2 points fit one block
 static_assert((1 << (kFftOneMaxLog2 - 1)) == kFftPoints, "one-kernel limit");
 
@@ -268,6 +269,42 @@ __device__ __forceinline__ void real_bins(const double2 (&v)[16], double* buf, i
         if (u == 8) zp = make_double2(self0 ? v[8].x : zp.x, self0 ? v[8].y : zp.y);
         use(u, real_bin(v[u], zp, cmul2(w0, w32(u))));
     }
+}
+
+// sum of |X_k|^2 w_k over the bins this thread's first 8 points give, k and H - k
+// of each pair from one (E, T): X_k = E + T, X_{H-k} = conj(E - T).  Every pair
+// of the block is some thread's (a thread's slots 8 .. 15 are its mates'), the
+// Nyquist bin is k = 0's partner, and slot 8 of `self0` is its own partner,
+// X = conj Z.  Half the exchange and products of real_bins.  weight(u) and
+// mirror(u): w at slot u's k and at H - k.
+template <class Wt, class Mi>
+__device__ __forceinline__ double real_norms(const double2 (&v)[16], double* buf, int mate, bool self0, double2 w0, const Wt& weight,
+                                             const Mi& mirror) {
+    double2* half = reinterpret_cast<double2*>(buf);
+    double wk[8], wm[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+        wk[u] = weight(u);
+        wm[u] = mirror(u);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 8; u < 16; ++u) half[(u - 8) * kFftThreads + threadIdx.x] = v[u];
+    __syncthreads();
+    double acc = self0 ? (v[8].x * v[8].x + v[8].y * v[8].y) * weight(8) : 0.0;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+        double2 zp = half[((self0 && u > 0) ? 8 - u : 7 - u) * kFftThreads + mate];
+        if (u == 0) zp = make_double2(self0 ? v[0].x : zp.x, self0 ? v[0].y : zp.y);
+        const double2 z = v[u], w = cmul2(w0, w32(u));
+        const double er = 0.5 * (z.x + zp.x), ei = 0.5 * (z.y - zp.y);
+        const double dr = 0.5 * (z.x - zp.x), di = 0.5 * (z.y + zp.y);
+        const double tr = w.x * di + w.y * dr, ti = -(w.x * dr - w.y * di);
+        const double ar = er + tr, ai = ei + ti, br = er - tr, bi = ei - ti;
+        acc += (ar * ar + ai * ai) * wk[u];
+        acc += (br * br + bi * bi) * wm[u];
+    }
+    return acc;
 }
 
 // Consecutive work on one XCD: block i runs on XCD i mod 8, and neighbouring

@@ -83,20 +83,18 @@ __global__ __launch_bounds__(kFftThreads) __attribute__((amdgpu_waves_per_eu(4))
     const auto addr = [&](int pos) { return rr * (H + H / 16) + pos + (pos >> 4); };
     const SplitTable tw{hi, lo};
     fft_stages<LH>(v, p, p, buf, tw, addr, addr, addr);
-    double acc = 0.0;
-    real_bins(v, buf, rr * per + ((per - p) & (per - 1)), p == 0, fft_unit((double)p * (0.5 / H)), [&](int u, double2 x) {
-        const int k = p + per * u;
-        if constexpr (kNorm) acc += (x.x * x.x + x.y * x.y) * nm.w[k];
-        else if (on) a.out[row * a.out_stride + k] = x;
-    });
-    if (p == 0) {
-        const double nyq = v[0].x - v[0].y;   // X_H
-        if constexpr (kNorm) acc += nyq * nyq * nm.w[H];
-        else if (on) a.out[row * a.out_stride + H] = make_double2(nyq, 0.0);
-    }
+    const int mate = rr * per + ((per - p) & (per - 1));
+    const double2 w0 = fft_unit((double)p * (0.5 / H));
     if constexpr (kNorm) {
+        const double acc = real_norms(v, buf, mate, p == 0, w0, [&](int u) { return nm.w[p + per * u]; },
+                                      [&](int u) { return nm.w[H - (p + per * u)]; });
         const double s = group_sum<per>(acc, buf);   // the first barrier inside is after every thread's reads of buf
         if (p == 0 && on) nm.partial[a.map[row] * nm.pstride] = s;
+    } else {
+        real_bins(v, buf, mate, p == 0, w0, [&](int u, double2 x) {
+            if (on) a.out[row * a.out_stride + p + per * u] = x;
+        });
+        if (p == 0 && on) a.out[row * a.out_stride + H] = make_double2(v[0].x - v[0].y, 0.0);   // X_H
     }
 }
 
@@ -168,20 +166,18 @@ __global__ __launch_bounds__(kFftThreads) __attribute__((amdgpu_waves_per_eu(4))
     // the partner H - k of k = ka + A kb: row A - ka, kb' = B - 1 - kb; rows 0
     // (kb' = B - kb) and A/2 are their own
     const int mate = (kl == 0 ? i : (i ^ C)) + C2 * (((ka == 0 ? per : per - 1) - p) & (per - 1));
-    const char* wt = reinterpret_cast<const char*>(nm.w);
-    double acc = 0.0;
-    real_bins(v, buf, mate, ka == 0 && p == 0, fft_unit((double)(ka + (long long)p * A) * (0.5 / (double)H)), [&](int u, double2 x) {
-        if constexpr (kNorm) acc += (x.x * x.x + x.y * x.y) * *reinterpret_cast<const double*>(wt + ((at + up * u) >> 1));
-        else *reinterpret_cast<double2*>(o + (at + up * u)) = x;
-    });
-    if (ka == 0 && p == 0) {
-        const double nyq = v[0].x - v[0].y;   // X_H
-        if constexpr (kNorm) acc += nyq * nyq * nm.w[H];
-        else *reinterpret_cast<double2*>(o + 16 * H) = make_double2(nyq, 0.0);
-    }
+    const double2 w0 = fft_unit((double)(ka + (long long)p * A) * (0.5 / (double)H));
+    const bool self0 = ka == 0 && p == 0;
     if constexpr (kNorm) {
+        const double* w = nm.w;
+        const unsigned k0 = (unsigned)ka + ((unsigned)p << LA), up = (unsigned)(per << LA);
+        const double acc = real_norms(v, buf, mate, self0, w0, [&](int u) { return w[k0 + up * u]; },
+                                      [&](int u) { return w[(unsigned)H - (k0 + up * u)]; });
         const double s = group_sum<kFftThreads>(acc, buf);
         if (t == 0) nm.partial[a.map[row] * nm.pstride + g] = s;
+    } else {
+        real_bins(v, buf, mate, self0, w0, [&](int u, double2 x) { *reinterpret_cast<double2*>(o + (at + up * u)) = x; });
+        if (self0) *reinterpret_cast<double2*>(o + 16 * H) = make_double2(v[0].x - v[0].y, 0.0);   // X_H
     }
 }
 
@@ -235,6 +231,14 @@ int rfft_own_log2(const void* in, const void* out, int n, int N) {
     const uintptr_t na = (uintptr_t)n * N * 8, nb = (uintptr_t)n * (N / 2 + 1) * 16;
     if (a < b + nb && b < a + na) return 0;
     return __builtin_ctz((unsigned)N);
+}
+
+int rfft_norm_partials(int log2N) { return log2N <= kFftOneMaxLog2 ? 1 : 1 << (log2N - kFftOneMaxLog2); }
+
+int rfft_weighted_norm(const double* in, long long in_stride, double* work, int n, int log2N, const int* count, const long long* map,
+                       const double* w, double* partial, int pstride, hipStream_t st) {
+    return launch_rows<true>(Rows{in, reinterpret_cast<double2*>(work), in_stride, 1LL << (log2N - 1), count, map, n}, Norm{w, partial, pstride},
+                             log2N, st);
 }
 
 int rfft_own(const double* in, double* out, int n, int log2N, hipStream_t st) {

@@ -19,17 +19,14 @@
 #include <hip/hip_runtime.h>
 
 #include "eobhip_common.hpp"
-#include "knot_window.hpp"
+#include "resample.hpp"
 
 using namespace eobhip_detail;
 
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kPerThread = 16;                 // resample: samples per thread per block
-constexpr int kSpan = kBlock * kPerThread;     // samples per block
-constexpr int kSearch = 4;                     // resample: samples per thread whose knot searches run together
-static_assert(kPerThread % kSearch == 0, "kSearch divides kPerThread");
+constexpr int kSpan = kRun * (kBlock / 64);    // resample: samples per block, a run per wavefront
 constexpr int kBinsPerThread = 8;              // hh: bins per thread per block
 constexpr int kBinSpan = kBlock * kBinsPerThread;
 
@@ -132,67 +129,48 @@ __global__ __launch_bounds__(kBlock) void k_lik_sizes(const double* __restrict__
 }
 
 // h+ = amp Re[S(t) e^{-2 i phi(t)}] from the spline coefficients (the uniform
-// resample of the full-length path) on j < M_b, zero for nsamp <= j < M_b;
-// per-block partial sums of h_j g_j.  grid (gx, n); a block covers kSpan
-// consecutive samples, stages the knot times of their intervals in LDS
-// (knot_window) and each thread searches there.
+// resample of the full-length path) and per-block partial sums of h_j g_j,
+// partial [n][pstride].  grid (blocks, rows), a run of samples per wavefront
+// (resample.hpp).  kSupport: row r is binary map[r], at hbuf + r stride, only its
+// support written (to the next even count; a block past it leaves at once).
+// Otherwise row b at hbuf + rowoff[b], zero for nsamp <= j < M_b.
+template <bool kSupport>
 __global__ __launch_bounds__(kBlock) void k_lik_resample(const double* __restrict__ dense, const double* __restrict__ coef,
                                                          const int* __restrict__ num_steps, const double* __restrict__ amp,
                                                          const double* __restrict__ dT_M, const int* __restrict__ nsamp,
-                                                         const int* __restrict__ mlog2, const long long* __restrict__ rowoff, int max_step,
+                                                         const int* __restrict__ mlog2, const long long* __restrict__ rowoff,
+                                                         const long long* __restrict__ map, long long stride, int max_step,
                                                          const double* __restrict__ g, double* __restrict__ hbuf,
-                                                         double* __restrict__ cross_partial) {
-    const int b = blockIdx.y;
-    const long long M = 1LL << mlog2[b];
-    const long long j0 = (long long)blockIdx.x * kSpan;
-    double* out = hbuf + rowoff[b];
+                                                         double* __restrict__ cross_partial, int pstride) {
+    const int b = kSupport ? (int)map[blockIdx.y] : blockIdx.y;
     const long long nb = nsamp[b];
+    if (kSupport && (long long)blockIdx.x * kSpan >= nb) return;
+    const long long M = kSupport ? (nb + 1) & ~1LL : 1LL << mlog2[b];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const long long j0 = (long long)blockIdx.x * kSpan + wave * kRun;
+    double* out = hbuf + (kSupport ? blockIdx.y * stride : rowoff[b]);
     double acc = 0.0;
-    __shared__ KnotWindow<kBlock> win;
-    if (j0 < M) {
-        const int len = num_steps[b];
+    if (j0 < nb) {
         const double* T = dense + (size_t)b * max_step * 5;
-        const double* C = coef + (size_t)b * max_step * 12;
-        const double dT = dT_M[b];
-        const double t0 = T[0];
-        if (j0 < nb) {
-            const long long jmax = (j0 + kSpan < nb ? j0 + kSpan : nb) - 1;   // last sample with a value in this block
-            knot_window<kBlock>(win, T, 5, len, t0 + (double)j0 * dT, t0 + (double)jmax * dT);
-        }
         const double a = amp[b];
-        for (int u0 = 0; u0 < kPerThread; u0 += kSearch) {
-            double tj[kSearch];
-            int ind[kSearch];
-#pragma unroll
-            for (int k = 0; k < kSearch; ++k) tj[k] = t0 + (double)(j0 + (long long)(u0 + k) * kBlock + threadIdx.x) * dT;
-            if (j0 < nb) knot_intervals<kBlock, kSearch>(win, T, 5, len, tj, ind);
-#pragma unroll
-            for (int k = 0; k < kSearch; ++k) {
-                const long long j = j0 + (long long)(u0 + k) * kBlock + threadIdx.x;
-                if (j < M) {
-                    double val = 0.0;
-                    if (j < nb) {
-                        double tk, c[12];
-                        interval_row<12>(T, 5, C, ind[k], tk, c);
-                        const double x = tj[k] - tk;
-                        const double x2 = x * x, x3 = x2 * x;
-                        const double ph = c[0] + c[1] * x + c[2] * x2 + c[3] * x3;
-                        const double sr = c[4] + c[5] * x + c[6] * x2 + c[7] * x3;
-                        const double si = c[8] + c[9] * x + c[10] * x2 + c[11] * x3;
-                        double sp, cp;
-                        sincos(2.0 * ph, &sp, &cp);
-                        val = a * (sr * cp + si * sp);
-                        acc += val * g[j];
-                    }
-                    out[j] = val;
-                }
-            }
-        }
+        h22_rows(T, coef + (size_t)b * max_step * 12, num_steps[b], T[0], dT_M[b], j0, nb,
+                 [&](long long j, const double (&re)[2], const double (&)[2], bool full) {
+                     const double ga = full || j < nb ? g[j] : 0.0, gb = full || j + 1 < nb ? g[j + 1] : 0.0;
+                     const double va = full || j < nb ? a * re[0] : 0.0, vb = full || j + 1 < nb ? a * re[1] : 0.0;
+                     acc += va * ga;
+                     acc += vb * gb;
+                     // the sum before the store: stores and loads share a counter, and a
+                     // wait for g after the store would wait for it as well
+                     asm volatile("" : "+v"(acc));
+                     store_pair<false>(out, j, M, va, vb);
+                 });
     }
-    // every thread of the block reaches the reduction's barrier (the window's
-    // barriers are taken by all threads or by none: j0 and nb are per block)
+    if constexpr (!kSupport) {
+        const long long done = j0 < nb ? (nb - j0 + kRow - 1) / kRow : 0;
+        for (long long r = done; r < kRunRows; ++r) store_pair<false>(out, j0 + r * kRow + 2 * lane, M, 0.0, 0.0);
+    }
     const double s = block_sum(acc);
-    if (threadIdx.x == 0) cross_partial[(size_t)b * gridDim.x + blockIdx.x] = s;
+    if (threadIdx.x == 0) cross_partial[(size_t)b * pstride + blockIdx.x] = s;
 }
 
 // per-block partial sums of |X_q|^2 W^(M)_q, q <= M/2; grid (gx2, n)
@@ -220,14 +198,19 @@ __global__ __launch_bounds__(kBlock) void k_lik_hh(const double2* __restrict__ X
     if (threadIdx.x == 0) hh_partial[(size_t)b * gridDim.x + blockIdx.x] = s;
 }
 
+// nsamp, mlog2 (both or neither): how many partials the support path leaves for
+// a template; otherwise all gx and gx2
 __global__ __launch_bounds__(64) void k_lik_final(const double* __restrict__ cross_partial, int gx, const double* __restrict__ hh_partial,
-                                                  int gx2, const double* __restrict__ dd, double df, int n, double* __restrict__ logl,
+                                                  int gx2, const int* __restrict__ nsamp, const int* __restrict__ mlog2,
+                                                  const double* __restrict__ dd, double df, int n, double* __restrict__ logl,
                                                   double* __restrict__ terms) {
     const int b = blockIdx.x;
     if (b >= n) return;
     double c = 0.0, h = 0.0;
-    for (int i = threadIdx.x; i < gx; i += 64) c += cross_partial[(size_t)b * gx + i];
-    for (int i = threadIdx.x; i < gx2; i += 64) h += hh_partial[(size_t)b * gx2 + i];
+    const int nc = nsamp ? (nsamp[b] + kSpan - 1) / kSpan : gx;
+    const int nh = mlog2 ? (mlog2[b] <= 14 ? 1 : 1 << (mlog2[b] - 14)) : gx2;
+    for (int i = threadIdx.x; i < nc; i += 64) c += cross_partial[(size_t)b * gx + i];
+    for (int i = threadIdx.x; i < nh; i += 64) h += hh_partial[(size_t)b * gx2 + i];
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) {
         c += __shfl_xor(c, off, 64);
@@ -380,8 +363,8 @@ int eobhip_lik_resample(const double* dense, const double* coef, const int* num_
     int gx, gx2;
     int rc = eobhip_lik_partial_blocks(max_mlog2, &gx, &gx2);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_lik_resample, dim3(gx, n), dim3(kBlock), 0, as_stream(stream), dense, coef, num_steps, amp, dT_M, nsamp, mlog2,
-                       rowoff, max_step, g, hbuf, cross_partial);
+    hipLaunchKernelGGL(k_lik_resample<false>, dim3(gx, n), dim3(kBlock), 0, as_stream(stream), dense, coef, num_steps, amp, dT_M, nsamp,
+                       mlog2, rowoff, nullptr, 0LL, max_step, g, hbuf, cross_partial, gx);
     return check_launch("lik_resample");
 }
 
@@ -397,7 +380,56 @@ int eobhip_lik_finish(const double* X, const long long* xoff, const int* mlog2, 
     hipLaunchKernelGGL(k_lik_hh, dim3(gx2, n), dim3(kBlock), 0, st, reinterpret_cast<const double2*>(X), xoff, mlog2, m_min_log2, bank,
                        hh_partial);
     if ((rc = check_launch("lik_hh"))) return rc;
-    hipLaunchKernelGGL(k_lik_final, dim3(n), dim3(64), 0, st, cross_partial, gx, hh_partial, gx2, dd, df, n, logl, terms);
+    hipLaunchKernelGGL(k_lik_final, dim3(n), dim3(64), 0, st, cross_partial, gx, hh_partial, gx2, nullptr, nullptr, dd, df, n, logl, terms);
+    return check_launch("lik_final");
+}
+
+// The second half of the likelihood in one call: per transform size (the
+// templates of a size are consecutive in `order`) the resample of the supports,
+// their transforms and the weighted norms, then log L.  Neither the samples
+// past a support nor the transforms are written: per template 8 L bytes of
+// samples and 8 M of the transform's intermediate go out and come back (M <=
+// 2^14: the samples only) instead of 8 M and the five or six passes of a plan.
+// 1024 templates of N = 2^20, M = 2^15 .. 2^20: the whole likelihood 5.75 ms with
+// plans per size, 2.10 in this form (88 us a size of resample, 235 of transforms
+// of the largest).
+int eobhip_lik_evaluate(const double* dense, const double* coef, const int* num_steps, const double* amp, const double* dT_M,
+                        const int* nsamp, const int* mlog2, const long long* order, int n, int max_step, int N, int nsizes,
+                        const int* size_log2, const int* size_count, int m_min_log2, const double* g, const double* bank, double* hbuf,
+                        double* work, double* cross_partial, double* hh_partial, const double* dd, double df, double* logl, double* terms,
+                        void* stream) {
+    const int L = log2_exact(N);
+    EOBHIP_REQUIRE(n >= 0 && n <= 65535 && max_step >= 1 && nsizes >= 0 && L >= 2, "bad sizes");
+    if (n == 0) return EOBHIP_OK;
+    int kmax = 0;
+    long long total = 0;
+    for (int q = 0; q < nsizes; ++q) {
+        EOBHIP_REQUIRE(size_log2[q] >= kRfftMinLog2 && size_log2[q] <= kRfftMaxLog2 && size_log2[q] >= m_min_log2 && size_log2[q] <= L,
+                       "lik_evaluate: transform size 2^%d outside 2^%d .. 2^%d", size_log2[q], kRfftMinLog2, kRfftMaxLog2);
+        EOBHIP_REQUIRE(size_count[q] >= 0, "lik_evaluate: negative count");
+        if (size_log2[q] > kmax) kmax = size_log2[q];
+        total += size_count[q];
+    }
+    EOBHIP_REQUIRE(total == n, "lik_evaluate: the sizes hold %lld of %d templates", total, n);
+    int gx, gx2;
+    int rc = eobhip_lik_partial_blocks(kmax, &gx, &gx2);
+    if (rc) return rc;
+    hipStream_t st = as_stream(stream);
+    for (int q = 0; q < nsizes; ++q) {
+        const int k = size_log2[q], rows = size_count[q];
+        if (rows == 0) continue;
+        // a support is at most half of M unless M is the whole segment
+        const long long stride = k < L ? 1LL << (k - 1) : 1LL << k;
+        hipLaunchKernelGGL(k_lik_resample<true>, dim3((unsigned)((stride + kSpan - 1) / kSpan), rows), dim3(kBlock), 0, st, dense, coef,
+                           num_steps, amp, dT_M, nsamp, mlog2, nullptr, order, stride, max_step, g, hbuf, cross_partial, gx);
+        if ((rc = check_launch("lik_resample"))) return rc;
+        rc = rfft_weighted_norm(hbuf, stride, work, rows, k, nsamp, order, bank + bank_offset(k, m_min_log2), hh_partial, gx2, st);
+        if (rc) return rc;
+        hbuf += stride * rows;
+        work += (2LL << (k - 1)) * rows;
+        order += rows;
+    }
+    hipLaunchKernelGGL(k_lik_final, dim3(n), dim3(64), 0, st, cross_partial, gx, hh_partial, gx2, nsamp, mlog2, dd, df, n, logl, terms);
     return check_launch("lik_final");
 }
 

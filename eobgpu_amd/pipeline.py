@@ -482,6 +482,8 @@ class SupportLikelihood:
     + ``fd_likelihood``) up to rounding; only the order of the sums differs.
     """
 
+    _OWN_LOG2 = (10, 21)   # transform sizes of the one-call second half (eobhip_lik_evaluate)
+
     def __init__(self, dtilde, N, df, f0=200.0, m_min_log2=10, device="cuda"):
         L = lib()
         self.N, self.df, self.f0, self.m_min = int(N), float(df), float(f0), int(m_min_log2)
@@ -538,15 +540,18 @@ class SupportLikelihood:
         return self.complete(self.begin(batch, total_mass_msun, dt, amp), out=out, terms=terms)
 
     def warm_transforms(self):
-        """Create the transform plans of every size (2^m_min .. N) and row chunk
-        (1, 2, 4, .. 64 rows) on the current stream -- plans are kept per stream
-        and size -- so that no later call on this stream spends host time
-        creating one (a call whose templates fall into new sizes or row counts
-        would otherwise)."""
+        """Create the transform plans of the sizes (2^m_min .. N) that the
+        library's own kernels do not take, for every row chunk (1, 2, 4, .. 64
+        rows) on the current stream -- plans are kept per stream and size -- so
+        that no later call on this stream spends host time creating one.  With
+        the default sizes there are none."""
         dev, chunk = self.device, 64
-        src = torch.zeros(chunk << self.log2N, dtype=torch.float64, device=dev)
-        dst = torch.empty(chunk * ((self.N >> 1) + 1), dtype=torch.complex128, device=dev)
-        for k in range(self.m_min, self.log2N + 1):
+        ks = [k for k in range(self.m_min, self.log2N + 1) if not self._OWN_LOG2[0] <= k <= self._OWN_LOG2[1]]
+        if not ks:
+            return
+        src = torch.zeros(chunk << ks[-1], dtype=torch.float64, device=dev)
+        dst = torch.empty(chunk * ((1 << ks[-1] >> 1) + 1), dtype=torch.complex128, device=dev)
+        for k in ks:
             rows = 1
             while rows <= chunk:
                 call("eobhip_rfft_batched", src.data_ptr(), dst.data_ptr(), rows, 1 << k, current_stream())
@@ -585,41 +590,50 @@ class SupportLikelihood:
         h["ready"].synchronize()
         ml = h["ml_host"].numpy().copy()
         order = np.argsort(ml, kind="stable")
-        rowoff = np.empty(n, dtype=np.int64)
-        xoff = np.empty(n, dtype=np.int64)
-        buckets = []
-        ph = px = 0
-        for k in np.unique(ml):
-            idx = order[ml[order] == k]
-            Mk = 1 << int(k)
-            buckets.append((Mk, ph, px, idx.size))
-            rowoff[idx] = ph + Mk * np.arange(idx.size)
-            xoff[idx] = px + (Mk // 2 + 1) * np.arange(idx.size)
-            ph += Mk * idx.size
-            px += (Mk // 2 + 1) * idx.size
+        sizes, counts = np.unique(ml, return_counts=True)
         kmax = int(ml.max()) if n else self.m_min
         gx, gx2 = ctypes.c_int(0), ctypes.c_int(0)
         call("eobhip_lik_partial_blocks", kmax, ctypes.byref(gx), ctypes.byref(gx2))
+        # the sizes the library's own transforms take go through one call that
+        # writes supports only and no transforms
+        one_call = n > 0 and sizes[0] >= self._OWN_LOG2[0] and sizes[-1] <= self._OWN_LOG2[1]
+        Mk = np.int64(1) << sizes.astype(np.int64)
+        hrow = np.where(sizes < self.log2N, Mk // 2, Mk) if one_call else Mk
+        xrow = Mk // 2 if one_call else Mk // 2 + 1
         with torch.cuda.stream(st):
             sp = current_stream()
-            w = self._buffers(n, ph, px, gx.value, gx2.value)
-            # row offsets then transform offsets, one contiguous copy
-            oh = w["offs_host"][:2 * n]
-            oh[:n].numpy()[:] = rowoff
-            oh[n:].numpy()[:] = xoff
-            offs = w["offs"][:2 * n]
-            offs.copy_(oh, non_blocking=True)
+            w = self._buffers(n, int((hrow * counts).sum()), int((xrow * counts).sum()), gx.value, gx2.value)
             hbuf, X, cross, hh = w["hbuf"], w["X"], w["cross"], w["hh"]
-            call("eobhip_lik_resample", batch.dense.data_ptr(), batch.coef.data_ptr(), batch.num_steps.data_ptr(),
-                 h["amp"].data_ptr(), h["dT_M"].data_ptr(), nsamp.data_ptr(), mlog2.data_ptr(), offs[:n].data_ptr(), n,
-                 batch.max_step, kmax, self.g.data_ptr(), hbuf.data_ptr(), cross.data_ptr(), sp)
-            for Mk, h0, x0, cnt in buckets:
-                call("eobhip_rfft_batched", hbuf.data_ptr() + 8 * h0, X.data_ptr() + 16 * x0, int(cnt), int(Mk), sp)
+            oh, offs = w["offs_host"], w["offs"]
             if out is None:
                 out = torch.empty(n, dtype=torch.float64, device=dev)
-            call("eobhip_lik_finish", X.data_ptr(), offs[n:].data_ptr(), mlog2.data_ptr(), n, kmax, self.m_min, self.bank.data_ptr(),
-                 cross.data_ptr(), hh.data_ptr(), self.dd.data_ptr(), self.df, out.data_ptr(),
-                 None if terms is None else terms.data_ptr(), sp)
+            if one_call:
+                oh[:n].numpy()[:] = order
+                offs[:n].copy_(oh[:n], non_blocking=True)
+                call("eobhip_lik_evaluate", batch.dense.data_ptr(), batch.coef.data_ptr(), batch.num_steps.data_ptr(),
+                     h["amp"].data_ptr(), h["dT_M"].data_ptr(), nsamp.data_ptr(), mlog2.data_ptr(), offs.data_ptr(), n, batch.max_step,
+                     self.N, len(sizes), _host_ints(sizes.tolist()), _host_ints(counts.tolist()), self.m_min, self.g.data_ptr(),
+                     self.bank.data_ptr(), hbuf.data_ptr(), X.data_ptr(), cross.data_ptr(), hh.data_ptr(), self.dd.data_ptr(), self.df,
+                     out.data_ptr(), None if terms is None else terms.data_ptr(), sp)
+            elif n:
+                # row offsets then transform offsets, one contiguous copy
+                first = np.concatenate([[0], np.cumsum(counts)])
+                h0 = np.concatenate([[0], np.cumsum(hrow * counts)])
+                x0 = np.concatenate([[0], np.cumsum(xrow * counts)])
+                a = oh[:2 * n].numpy()
+                for q, cnt in enumerate(counts):
+                    idx, r = order[first[q]:first[q + 1]], np.arange(cnt)
+                    a[idx] = h0[q] + hrow[q] * r
+                    a[n + idx] = x0[q] + xrow[q] * r
+                offs[:2 * n].copy_(oh[:2 * n], non_blocking=True)
+                call("eobhip_lik_resample", batch.dense.data_ptr(), batch.coef.data_ptr(), batch.num_steps.data_ptr(),
+                     h["amp"].data_ptr(), h["dT_M"].data_ptr(), nsamp.data_ptr(), mlog2.data_ptr(), offs[:n].data_ptr(), n,
+                     batch.max_step, kmax, self.g.data_ptr(), hbuf.data_ptr(), cross.data_ptr(), sp)
+                for q, cnt in enumerate(counts):
+                    call("eobhip_rfft_batched", hbuf.data_ptr() + 8 * int(h0[q]), X.data_ptr() + 16 * int(x0[q]), int(cnt), int(Mk[q]), sp)
+                call("eobhip_lik_finish", X.data_ptr(), offs[n:].data_ptr(), mlog2.data_ptr(), n, kmax, self.m_min, self.bank.data_ptr(),
+                     cross.data_ptr(), hh.data_ptr(), self.dd.data_ptr(), self.df, out.data_ptr(),
+                     None if terms is None else terms.data_ptr(), sp)
         self.nsamp, self.mlog2 = nsamp, mlog2
         self._tmp = (h["dT_M"], h["amp"])
         return out

@@ -363,6 +363,16 @@ int eobhip_lik_resample(const double* dense, const double* coef, const int* num_
 int eobhip_lik_finish(const double* X, const long long* xoff, const int* mlog2, int n, int max_mlog2, int m_min_log2,
                       const double* bank, const double* cross_partial, double* hh_partial, const double* dd, double df, double* logl,
                       double* terms, void* stream);
+/* resample, transforms, weighted norms and log L of n templates in one call: order [n] the
+ * templates by transform size, size_log2 / size_count (host, nsizes) the sizes in that order and
+ * how many templates have each (2^10 .. 2^21, the sizes eobhip_lik_sizes gave).  hbuf: per template
+ * M/2 doubles (M for M = N); work: M/2 complex; cross_partial, hh_partial as for
+ * eobhip_lik_resample and eobhip_lik_finish (eobhip_lik_partial_blocks of the largest size). */
+int eobhip_lik_evaluate(const double* dense, const double* coef, const int* num_steps, const double* amp, const double* dT_M,
+                        const int* nsamp, const int* mlog2, const long long* order, int n, int max_step, int N, int nsizes,
+                        const int* size_log2, const int* size_count, int m_min_log2, const double* g, const double* bank, double* hbuf,
+                        double* work, double* cross_partial, double* hh_partial, const double* dd, double df, double* logl, double* terms,
+                        void* stream);
 
 /* ---------------------------------------------------- merger-ringdown attachment
  * The fits of the NQC and ringdown attachment, evaluated elementwise on device
