@@ -150,10 +150,11 @@ __global__ __launch_bounds__(kBlock) void k_lik_resample(const double* __restric
     const long long j0 = (long long)blockIdx.x * kSpan + wave * kRun;
     double* out = hbuf + (kSupport ? blockIdx.y * stride : rowoff[b]);
     double acc = 0.0;
+    __shared__ H22Stage stages[kBlock / 64];
     if (j0 < nb) {
         const double* T = dense + (size_t)b * max_step * 5;
         const double a = amp[b];
-        h22_rows(T, coef + (size_t)b * max_step * 12, num_steps[b], T[0], dT_M[b], j0, nb,
+        h22_rows(stages[wave], T, coef + (size_t)b * max_step * 12, num_steps[b], T[0], dT_M[b], j0, nb,
                  [&](long long j, const double (&re)[2], const double (&)[2], bool full) {
                      const double ga = full || j < nb ? g[j] : 0.0, gb = full || j + 1 < nb ? g[j + 1] : 0.0;
                      const double va = full || j < nb ? a * re[0] : 0.0, vb = full || j + 1 < nb ? a * re[1] : 0.0;
@@ -391,7 +392,7 @@ int eobhip_lik_finish(const double* X, const long long* xoff, const int* mlog2, 
 // samples and 8 M of the transform's intermediate go out and come back (M <=
 // 2^14: the samples only) instead of 8 M and the five or six passes of a plan.
 // 1024 templates of N = 2^20, M = 2^15 .. 2^20: the whole likelihood 5.75 ms with
-// plans per size, 2.10 in this form (88 us a size of resample, 235 of transforms
+// plans per size, 2.00 in this form (73 us a size of resample, 235 of transforms
 // of the largest).
 int eobhip_lik_evaluate(const double* dense, const double* coef, const int* num_steps, const double* amp, const double* dT_M,
                         const int* nsamp, const int* mlog2, const long long* order, int n, int max_step, int N, int nsizes,

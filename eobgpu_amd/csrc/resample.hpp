@@ -4,13 +4,8 @@
 // time (two per lane, one 16-byte store per series), and keeps the knot
 // interval (searchsorted(t, t_j, 'right') - 1, eob/seobnrv4phm.py:241-272) it is
 // in.  Most rows of 128 lie in one interval: the row's last time against the next
-// knot decides that with one comparison, and the interval's coefficients are then
-// read once for the wavefront through the scalar cache.  A row that passes knots
-// reads up to 64 of them, one per lane, and each lane counts those at or before
-// its samples; only a row that passes many falls back to a bisection per
-// sample.  No LDS, no barriers: what a block waited for before (a window of
-// knots staged for 4096 samples, then a bisection of it per sample) was most of
-// these kernels' time.
+// knot decides that with one comparison.  The run's knots and table rows are
+// staged at its start, by and for the wavefront alone (no barriers).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -19,22 +14,24 @@
 namespace eobhip_detail {
 
 constexpr int kRow = 128;                 // samples per wavefront and step
-constexpr int kRunRows = 8;               // rows of a run
-constexpr int kFewKnots = 8;              // knots a row may pass before its lanes bisect
+constexpr int kRunRows = 4;               // rows of a run
 constexpr int kRun = kRow * kRunRows;     // samples per run
 
-// sin and cos of x: x - n pi/2 in two fused steps (the first exact for |n| <
-// 2^20), the Taylor series through r^17 and r^16 on |r| <= pi/4 (first omitted
-// terms below 2e-18), and the quadrant; the library's for larger x anywhere in
-// the wavefront.  Within 1e-16 absolute of it; the arguments here are phases of
-// 10 to 10^4 rad whose own rounding is 1e-15 to 1e-12.  About 40 instructions
-// against the library's 75.
+// sin and cos of x: x - n pi/2 in two fused steps (each exact but for its last
+// rounding: their terms cancel to below 1), the Taylor series through r^17 and
+// r^16 on |r| <= pi/4 (first omitted terms below 2e-18), and the quadrant.  Within
+// 1e-16 absolute for |x| < 2^50 (phases here are 10 to 10^5 rad, their own rounding
+// 1e-15 to 1e-11); larger x, of which a double no longer resolves the radian, are
+// taken down by the same step first and stay bounded.  About 40 instructions
+// against the library's 75, and 20 registers less for the kernel.
 __device__ __forceinline__ void sincos_phase(double x, double* s, double* c) {
-    if (__any(!(fabs(x) < 1.0e6))) {
-        sincos(x, s, c);
-        return;
-    }
     constexpr double kTwoOverPi = 0x1.45f306dc9c883p-1, kPio2Hi = 0x1.921fb54442d18p+0, kPio2Lo = 0x1.1a62633145c07p-54;
+    double quad = 0.0;
+    for (int it = 0; it < 24 && __any(!(fabs(x) < 0x1p45)); ++it) {
+        const double n = rint(x * kTwoOverPi);
+        x = fma(-n, kPio2Lo, fma(-n, kPio2Hi, x));
+        quad += fma(-4.0, floor(0.25 * n), n);
+    }
     const double n = rint(x * kTwoOverPi);
     const double r = fma(-n, kPio2Lo, fma(-n, kPio2Hi, x));
     const double z = r * r;
@@ -54,7 +51,7 @@ __device__ __forceinline__ void sincos_phase(double x, double* s, double* c) {
     q = fma(q, z, 1.0 / 24.0);
     q = fma(q, z, -0.5);
     const double cr = fma(q, z, 1.0);
-    const int k = (int)n;
+    const int k = (int)(fma(-4.0, floor(0.25 * n), n) + quad);
     const double a = (k & 1) ? cr : sr, b = (k & 1) ? sr : cr;
     *s = (k & 2) ? -a : a;
     *c = ((k + 1) & 2) ? -b : b;
@@ -92,72 +89,17 @@ __device__ __forceinline__ double lane_value(double v, int q) {
 
 typedef const __attribute__((address_space(4))) double* ConstPtr;
 
-// The rows of the run that starts at sample j0, as far as samples have a value
-// (j < jend; j0 < jend):
-//   time(j)                       the time of sample j
-//   enter(i)                      the wavefront is in interval i from here on (uniform)
-//   one(j, ta, tb, full)          a row in that interval: samples j, j + 1 of this lane;
-//                                 full: all of the row's samples are below jend
-//   each(j, ta, tb, ia, ib)       a row that passes knots: each sample's own interval
-// kLastApart: rows past the last knot go to each as well (its interval has a value
-// and no slope there).
-template <bool kLastApart = false, class Time, class Enter, class One, class Each>
-__device__ __forceinline__ void resample_rows(const double* __restrict__ T, int len, long long j0, long long jend, const Time& time,
-                                              const Enter& enter, const One& one, const Each& each) {
-    const int lane = threadIdx.x & 63;
-    int ind = wave_interval(T, len, time(j0));
-    for (int r = 0; r < kRunRows;) {
-        if (j0 + (long long)r * kRow >= jend) break;
-        const double next = ind + 1 < len ? ((ConstPtr)T)[5 * (size_t)(ind + 1)] : (kLastApart ? -HUGE_VAL : HUGE_VAL);
-        enter(ind);
-        double last = 0.0;
-        for (; r < kRunRows; ++r) {
-            const long long jr = j0 + (long long)r * kRow;
-            if (jr >= jend) return;
-            const bool full = jr + kRow <= jend;
-            last = time(full ? jr + kRow - 1 : jend - 1);
-            if (!__builtin_amdgcn_readfirstlane(last < next)) break;
-            const long long j = jr + 2 * lane;
-            one(j, time(j), time(j + 1), full);
-        }
-        if (r == kRunRows) break;
-        const long long j = j0 + (long long)r * kRow + 2 * lane;
-        const double ta = time(j), tb = time(j + 1);
-        const int k = ind + 1 + lane;
-        const double tk = k < len ? T[5 * (size_t)k] : HUGE_VAL;
-        const int passed = __popcll(__ballot(tk <= last));
-        int ia = ind, ib = ind;
-        if (passed <= kFewKnots) {
-            for (int q = 0; q < passed; ++q) {
-                const double x = lane_value(tk, q);
-                ia += x <= ta;
-                ib += x <= tb;
-            }
-            ind += passed;
-        } else {
-            // T[ind] <= every sample of the row (or ind = 0)
-            for (int m = len - ind; m > 1;) {
-                const int half = m >> 1;
-                ia = T[5 * (size_t)(ia + half)] <= ta ? ia + half : ia;
-                ib = T[5 * (size_t)(ib + half)] <= tb ? ib + half : ib;
-                m -= half;
-            }
-            ind = passed < 64 ? ind + passed : wave_interval(T, len, last);
-        }
-        each(j, ta, tb, ia, ib);
-        ++r;
-    }
-}
+// two consecutive doubles at any 8-byte boundary
+typedef double SamplePair __attribute__((ext_vector_type(2), aligned(8)));
 
-// A lane's two samples in turn, f(t, i, re, im) each: where a wavefront gathers
-// rows per lane, two samples' at once would double the registers of the whole
-// kernel.
+// A lane's two samples in turn, f(i, x, re, im) each: at once they would double the
+// registers of the whole kernel.
 template <class F>
-__device__ __forceinline__ void one_by_one(double ta, double tb, int ia, int ib, double (&re)[2], double (&im)[2], const F& f) {
+__device__ __forceinline__ void one_by_one(double xa, double xb, int ia, int ib, double (&re)[2], double (&im)[2], const F& f) {
 #pragma unroll 1
     for (int e = 0; e < 2; ++e) {
         double x, y;
-        f(e ? tb : ta, e ? ib : ia, x, y);
+        f(e ? ib : ia, e ? xb : xa, x, y);
         re[0] = e ? re[0] : x;
         im[0] = e ? im[0] : y;
         re[1] = x;
@@ -165,10 +107,120 @@ __device__ __forceinline__ void one_by_one(double ta, double tb, int ia, int ib,
     }
 }
 
+// A wavefront's LDS copy of R consecutive rows of a table, CS doubles each
+template <int CS, int R>
+struct StagedRows {
+    static constexpr int kRows = R;
+    __attribute__((aligned(16))) double c[R * CS];
+    // n <= R rows of `cs` <= CS doubles from src on
+    __device__ __forceinline__ void copy(const double* __restrict__ src, int n, int cs = CS) {
+        constexpr int kSteps = (R * CS + 127) / 128;
+        const int lane = threadIdx.x & 63;
+        SamplePair v[kSteps];
+#pragma unroll
+        for (int q = 0; q < kSteps; ++q) {
+            const int i = 2 * (lane + 64 * q);
+            if (i < n * cs) v[q] = *reinterpret_cast<const SamplePair*>(src + i);
+        }
+#pragma unroll
+        for (int q = 0; q < kSteps; ++q) {
+            const int i = 2 * (lane + 64 * q);
+            if (i < n * cs) *reinterpret_cast<double2*>(c + i) = make_double2(v[q].x, v[q].y);
+        }
+    }
+    __device__ __forceinline__ const double* row(int k) const { return c + k * CS; }
+    // row k of 4-coefficient series keeps its values and loses its slopes
+    __device__ __forceinline__ void flatten(int k, int cs = CS) {
+        for (int i = threadIdx.x & 63; i < cs; i += 64)
+            if (i & 3) c[k * cs + i] = 0.0;
+    }
+};
+
+// The rows of the run that starts at sample j0, as far as samples have a value
+// (j < jend; j0 < jend):
+//   time(j)                the time of sample j
+//   stage(i, n)            table rows i .. i + n - 1 (n <= R) into the wavefront's LDS
+//   near(k, x, re, im)     one sample at x past the knot of staged row k (per lane)
+//   far(i, x, re, im)      one sample from table row i (per lane), read from memory
+//   put(j, re, im, full)   a lane's samples j, j + 1 (full: all of the row's are below jend)
+// The run's knots (lane q holds the q-th after its first) and table rows are read
+// in two steps at its start; its rows then wait for no load.  Interval by interval
+// through the scalar cache, with gathers where a row passes a knot, the waits
+// (about 1 us each, four a row) were the time: 1024 templates' h+ for the likelihood
+// 880 us, 735 this way; the five modes with NQC factors of 512 binaries 3560, 3055.
+template <int R, class Time, class Stage, class Near, class Far, class Put>
+__device__ __forceinline__ void resample_rows(const double* __restrict__ T, int len, long long j0, long long jend, const Time& time,
+                                              const Stage& stage, const Near& near, const Far& far, const Put& put) {
+    static_assert(R <= 63, "a lane per knot");
+    const int lane = threadIdx.x & 63;
+    const double end = time((j0 + kRun < jend ? j0 + kRun : jend) - 1);
+    int ind = wave_interval(T, len, time(j0));
+    for (int r = 0; r < kRunRows;) {
+        if (j0 + (long long)r * kRow >= jend) break;
+        // staged: rows ind .. ind + cnt, local 0 .. cnt
+        const int kl = ind + 1 + lane;
+        const double tk = kl < len ? T[5 * (size_t)kl] : HUGE_VAL;
+        double t0 = ((ConstPtr)T)[5 * (size_t)ind];   // the current interval's knot
+        int cnt = __popcll(__ballot(kl < len && tk <= end));
+        cnt = cnt < R ? cnt : R - 1;
+        stage(ind, cnt + 1);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        int cur = 0;
+        double next = lane_value(tk, 0), last = 0.0;
+        long long j = 0;
+        double re[2], im[2];
+        bool covered = true;
+        for (; r < kRunRows; ++r) {
+            const long long jr = j0 + (long long)r * kRow;
+            if (jr >= jend) return;
+            const bool full = jr + kRow <= jend;
+            j = jr + 2 * lane;
+            last = time(full ? jr + kRow - 1 : jend - 1);
+            const double ta = time(j), tb = time(j + 1);
+            int ia = cur, ib = cur;
+            double xa = t0, xb = t0;
+            if (!__builtin_amdgcn_readfirstlane(last < next)) {
+                const int to = __popcll(__ballot(tk <= last));
+                covered = to <= cnt;
+                if (!covered) break;
+                for (; cur < to; ++cur) {
+                    t0 = lane_value(tk, cur);
+                    ia = t0 <= ta ? cur + 1 : ia;
+                    ib = t0 <= tb ? cur + 1 : ib;
+                    xa = t0 <= ta ? t0 : xa;
+                    xb = t0 <= tb ? t0 : xb;
+                }
+                next = lane_value(tk, cur);
+            }
+            one_by_one(ta - xa, tb - xb, ia, ib, re, im, near);
+            put(j, re, im, full);
+        }
+        if (covered) break;
+        if (cur > 0) {   // stage from here
+            ind += cur;
+            continue;
+        }
+        // the row passes more knots than are staged: T[ind] <= every sample of it (or ind = 0)
+        const double ta = time(j), tb = time(j + 1);
+        int ia = ind, ib = ind;
+        for (int m = len - ind; m > 1;) {
+            const int half = m >> 1;
+            ia = T[5 * (size_t)(ia + half)] <= ta ? ia + half : ia;
+            ib = T[5 * (size_t)(ib + half)] <= tb ? ib + half : ib;
+            m -= half;
+        }
+        one_by_one(ta - T[5 * (size_t)ia], tb - T[5 * (size_t)ib], ia, ib, re, im, far);
+        put(j, re, im, false);
+        ind = wave_interval(T, len, last);
+        ++r;
+    }
+}
+
 // Two consecutive samples of a series of N.  kStream: past the caches (a series
 // longer than they hold: 1682 us for the five-mode sum of 512 binaries x 2^20
 // against 2496 through them).
-typedef double SamplePair __attribute__((ext_vector_type(2), aligned(8)));
 template <bool kStream>
 __device__ __forceinline__ void store_pair(double* out, long long j, long long N, double a, double b) {
     if (j + 1 < N) {
@@ -194,36 +246,15 @@ __device__ __forceinline__ void h22_sample(const Row& c, double x, double& re, d
     im = si * cp - sr * sp;
 }
 
-// one interval's row of them and its knot, through the scalar cache (the tables
-// are read-only while the kernels run)
-struct H22Row {
-    double c[12], tk;
-    __device__ __forceinline__ void load(const double* T, const double* C, int i) {
-        const ConstPtr r = (ConstPtr)(C + (size_t)12 * i);
-#pragma unroll
-        for (int q = 0; q < 12; ++q) c[q] = r[q];
-        tk = ((ConstPtr)T)[5 * (size_t)i];
-    }
-};
-
 // h22 on the run of samples t0 + j dT from j0: put(j, re[2], im[2], full)
+typedef StagedRows<12, 16> H22Stage;
 template <class Put>
-__device__ __forceinline__ void h22_rows(const double* __restrict__ T, const double* __restrict__ C, int len, double t0, double dT, long long j0,
-                                         long long jend, const Put& put) {
-    H22Row row;
-    resample_rows(
-        T, len, j0, jend, [&](long long j) { return t0 + (double)j * dT; }, [&](int i) { row.load(T, C, i); },
-        [&](long long j, double ta, double tb, bool full) {
-            double re[2], im[2];
-            h22_sample(row.c, ta - row.tk, re[0], im[0]);
-            h22_sample(row.c, tb - row.tk, re[1], im[1]);
-            put(j, re, im, full);
-        },
-        [&](long long j, double ta, double tb, int ia, int ib) {
-            double re[2], im[2];
-            one_by_one(ta, tb, ia, ib, re, im, [&](double t, int i, double& x, double& y) { h22_sample(C + (size_t)12 * i, t - T[5 * (size_t)i], x, y); });
-            put(j, re, im, false);
-        });
+__device__ __forceinline__ void h22_rows(H22Stage& st, const double* __restrict__ T, const double* __restrict__ C, int len, double t0, double dT,
+                                         long long j0, long long jend, const Put& put) {
+    resample_rows<H22Stage::kRows>(
+        T, len, j0, jend, [&](long long j) { return t0 + (double)j * dT; }, [&](int i, int n) { st.copy(C + (size_t)12 * i, n); },
+        [&](int k, double x, double& re, double& im) { h22_sample(st.row(k), x, re, im); },
+        [&](int i, double x, double& re, double& im) { h22_sample(C + (size_t)12 * i, x, re, im); }, put);
 }
 
 // h+ and hx (hx may be null) of N samples, zero from nb on
@@ -247,7 +278,7 @@ struct SeriesOut {
     }
 };
 
-// A wavefront's runs of one binary's series (grid.x blocks of `waves` wavefronts): f(j0)
+// A wavefront's runs of one binary's series, f(j0); grid resample_grid
 template <class F>
 __device__ __forceinline__ void for_runs(long long N, int waves, const F& f) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -255,32 +286,41 @@ __device__ __forceinline__ void for_runs(long long N, int waves, const F& f) {
     for (long long run = (long long)blockIdx.x * waves + wave; run < nrun; run += (long long)gridDim.x * waves) f(run * kRun);
 }
 
-// Blocks (of four wavefronts) per binary: about 16384 in all (64 per CU), no
-// more, so that a wavefront takes several runs.  They are spread over the series
-// (run, run + the binary's wavefronts, ...), since the template's part costs more
-// than the zeros after it.  h+ of 256 binaries x 2^20 and the five-mode sum of
-// 512: a block per 4096 samples 540 and 2499 us, 16384 blocks 468 and 1682, 4096
-// blocks 501 and 1746; contiguous runs per block 772 and 3510.
-inline int resample_blocks(int N, int n) {
-    const int most = (int)((N + 4LL * kRun - 1) / (4LL * kRun)), want = (16384 + n - 1) / n;
-    return want < most ? want : most;
+// (blocks of four wavefronts, binaries): about 131072 blocks in all, no more, so
+// that a wavefront takes several runs.  They are spread over the series (run, run +
+// the binary's wavefronts, ...), since the template's part costs more than the
+// zeros after it.  h+ of 256 binaries x 2^20, the five-mode sum of 512 and the same
+// with its ringdown at 16384 Hz: 16384 blocks of runs of 8 rows 461, 1675 and 3165
+// us, 131072 of 4 rows 407, 1620 and 2990, 524288 409, 1581 and 3076; neighbouring
+// blocks on different binaries instead 480, 1690 and 3700 (writes all over
+// memory), contiguous runs per block slower by half.
+inline dim3 resample_grid(int N, int n) {
+    const int most = (int)((N + 4LL * kRun - 1) / (4LL * kRun)), want = (131072 + n - 1) / n;
+    return dim3(want < most ? want : most, n);
 }
 
-// The modes of a sum by falling m: mode q[k] is the k-th, down[k] = m[q[k-1]] -
-// m[q[k]] (0 for k = 0), down[nm] the last one's m.
 constexpr int kMaxModes = 15;
+
+// The modes of a sum by falling m, four bits each (two scalar registers a list,
+// where arrays would be loaded entry by entry): q(k) the k-th mode, down(k) =
+// m[q(k-1)] - m[q(k)] (0 for k = 0), down(nm) the last one's m.
 struct ModeOrder {
-    int q[kMaxModes], down[kMaxModes + 1];
+    unsigned long long qs = 0, downs = 0;
+    __device__ __forceinline__ int q(int k) const { return (int)(qs >> (4 * k)) & 15; }
+    __device__ __forceinline__ int down(int k) const { return (int)(downs >> (4 * k)) & 15; }
 };
-inline ModeOrder mode_order(const int* m, int nm) {
-    ModeOrder o{};
+inline ModeOrder mode_order(const int* m, int nm) {   // nm <= 15, 1 <= m <= 15
+    int q[16];
     for (int k = 0; k < nm; ++k) {
         int j = k;
-        for (; j > 0 && m[o.q[j - 1]] < m[k]; --j) o.q[j] = o.q[j - 1];
-        o.q[j] = k;
+        for (; j > 0 && m[q[j - 1]] < m[k]; --j) q[j] = q[j - 1];
+        q[j] = k;
     }
-    for (int k = 1; k < nm; ++k) o.down[k] = m[o.q[k - 1]] - m[o.q[k]];
-    o.down[nm] = m[o.q[nm - 1]];
+    ModeOrder o;
+    for (int k = 0; k < nm; ++k) {
+        o.qs |= (unsigned long long)q[k] << (4 * k);
+        o.downs |= (unsigned long long)(m[q[k]] - (k + 1 < nm ? m[q[k + 1]] : 0)) << (4 * (k + 1));
+    }
     return o;
 }
 

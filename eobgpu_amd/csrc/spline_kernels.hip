@@ -594,8 +594,8 @@ __global__ __launch_bounds__(kSplineLanes) void k_spline_build_seg(const double*
 // zero for N_b <= j < N; hx is the imaginary part, the two series the reference
 // transforms (eob/seobnrv4phm.py:720, 742-744).  grid (blocks, binaries), a run
 // of samples per wavefront (resample.hpp).  Bound by the writes: 256 binaries x
-// 2^20 samples, 15% of them inside a template: h+ 593 us with knot windows per
-// block, 412 now (a fill of the same memory 340).
+// 2^20 samples, 10% of them inside a template: h+ 593 us with knot windows per
+// block, 412 interval by interval, 373 now (a fill of the same memory 340).
 // samples with a value: floor((t_last - t_0) / dT) + 1, at most N
 __device__ __forceinline__ long long series_samples(const double* T, int len, double dT, int N) {
     if (len < 2) return 0;
@@ -617,9 +617,11 @@ __global__ __launch_bounds__(kBlock) void k_resample_hplus(const double* __restr
     const SeriesOut o{hplus + (size_t)b * N, hcross ? hcross + (size_t)b * N : nullptr, amp[b], nb, N};
     const double* C = coef + (size_t)b * max_step * 12;
     const double t0 = T[0];
+    __shared__ H22Stage stages[kBlock / 64];
+    H22Stage& st = stages[threadIdx.x >> 6];
     for_runs(N, kBlock / 64, [&](long long j0) {
         if (j0 < nb)
-            h22_rows(T, C, len, t0, dT, j0, nb, [&](long long j, const double (&re)[2], const double (&im)[2], bool full) { o.put(j, re, im, full); });
+            h22_rows(st, T, C, len, t0, dT, j0, nb, [&](long long j, const double (&re)[2], const double (&im)[2], bool full) { o.put(j, re, im, full); });
         o.zeros(j0);
     });
 }
@@ -631,49 +633,46 @@ __global__ __launch_bounds__(kBlock) void k_resample_hplus(const double* __restr
 // [n][max_step][4 (2 nm + 1)]: series j < nm Re S_j, nm + j Im S_j, 2 nm phi.
 // e^{-i m phi} is formed as the m-th power of e^{-i phi}.
 constexpr int kMaxModeM = 8;
-struct ModeMs {
-    int nm;
-    int m[15];
-};
 // One sample's sum from a row (Re of each mode, Im of each mode, phi; 4
-// coefficients per series).  e^{-i m phi} is m - 1 products with e^{-i phi} (the
-// products a table of the powers would hold, without a per-mode select from the
-// table).  NMT > 0: built for that many modes (the loop over modes unrolled); 0:
-// any.
-template <int NMT, class Ptr>
-__device__ __forceinline__ void modes_sample(Ptr c, double x, int nm, const ModeMs& mm, double& hr, double& hi) {
+// coefficients per series), by Horner's rule in e^{-i phi} over the modes by
+// falling m: a mode costs the products between its m and the next one's.
+template <class Ptr>
+__device__ __forceinline__ void modes_sample(Ptr c, double x, int nm, const ModeOrder& mo, double& hr, double& hi) {
     const double x2 = x * x, x3 = x2 * x;
     const auto cubic = [&](Ptr p) { return p[0] + p[1] * x + p[2] * x2 + p[3] * x3; };
     double sp, cph;
     sincos_phase(cubic(c + 4 * (2 * nm)), &sp, &cph);
-    hr = hi = 0.0;
-#pragma unroll
-    for (int q = 0; q < (NMT > 0 ? NMT : nm); ++q) {
-        const double re = cubic(c + 4 * q), im = cubic(c + 4 * (nm + q));
-        double pr = cph, pi = -sp;   // e^{-i phi}
-        for (int k = 1; k < mm.m[q]; ++k) {
-            const double t = pr * cph + pi * sp;
-            pi = pi * cph - pr * sp;
-            pr = t;
+    double r = 0.0, i = 0.0;
+    const auto turn = [&](int k) {
+        for (; k > 0; --k) {
+            const double t = r * cph + i * sp;
+            i = i * cph - r * sp;
+            r = t;
         }
-        hr += re * pr - im * pi;
-        hi += re * pi + im * pr;
+    };
+#pragma unroll 1
+    for (int k = 0; k < nm; ++k) {
+        const int q = mo.q(k);
+        turn(mo.down(k));
+        r += cubic(c + 4 * q);
+        i += cubic(c + 4 * (nm + q));
     }
+    turn(mo.down(nm));
+    hr = r;
+    hi = i;
 }
 
-// Rows are read through the scalar cache sample by sample (the 44 coefficients
-// of five modes do not fit the scalar registers).  Five modes of 512 binaries x
-// 2^20, 18% of the samples inside a template: 2470 us with knot windows per
-// block, 1519 now (the writes alone 1360).
-template <int NMT>
+// kModes: the most modes the staged rows have room for.  Five modes of 512 binaries
+// x 2^20, 10% of the samples inside a template: 2470 us with knot windows per block,
+// 1520 interval by interval, 1470 to 1570 now (the writes alone 1360).
+template <int kModes>
 __global__ __launch_bounds__(kBlock) void k_resample_modes(const double* __restrict__ dense, const double* __restrict__ coef,
                                                            const int* __restrict__ num_steps, const double* __restrict__ amp,
-                                                           const double* __restrict__ dT_M, int max_step, int N, ModeMs mm,
+                                                           const double* __restrict__ dT_M, int max_step, int N, int nm, ModeOrder mo,
                                                            double* __restrict__ hplus, double* __restrict__ hcross,
                                                            int* __restrict__ nsamp) {
     const int b = blockIdx.y;
     const int len = num_steps[b];
-    const int nm = NMT > 0 ? NMT : mm.nm;
     const int cs = 4 * (2 * nm + 1);
     const double* T = dense + (size_t)b * max_step * 5;
     const double* C = coef + (size_t)b * max_step * cs;
@@ -681,29 +680,16 @@ __global__ __launch_bounds__(kBlock) void k_resample_modes(const double* __restr
     const long long nb = series_samples(T, len, dT, N);
     if (blockIdx.x == 0 && threadIdx.x == 0) nsamp[b] = (int)nb;
     const SeriesOut o{hplus + (size_t)b * N, hcross + (size_t)b * N, amp[b], nb, N};
+    typedef StagedRows<4 * (2 * kModes + 1), 8> Stage;   // rows at their own stride cs
+    __shared__ Stage stages[kBlock / 64];
+    Stage& st = stages[threadIdx.x >> 6];
     for_runs(N, kBlock / 64, [&](long long j0) {
-        ConstPtr c = nullptr;
-        double tk = 0.0;
         if (j0 < nb)
-            resample_rows(
-                T, len, j0, nb, [&](long long j) { return t0 + (double)j * dT; },
-                [&](int i) {
-                    c = (ConstPtr)(C + (size_t)cs * i);
-                    tk = ((ConstPtr)T)[5 * (size_t)i];
-                },
-                [&](long long j, double ta, double tb, bool full) {
-                    double re[2], im[2];
-                    modes_sample<NMT>(c, ta - tk, nm, mm, re[0], im[0]);
-                    modes_sample<NMT>(c, tb - tk, nm, mm, re[1], im[1]);
-                    o.put(j, re, im, full);
-                },
-                [&](long long j, double ta, double tb, int ia, int ib) {
-                    double re[2], im[2];
-                    one_by_one(ta, tb, ia, ib, re, im, [&](double t, int i, double& x, double& y) {
-                        modes_sample<NMT>(C + (size_t)cs * i, t - T[5 * (size_t)i], nm, mm, x, y);
-                    });
-                    o.put(j, re, im, false);
-                });
+            resample_rows<Stage::kRows>(
+                T, len, j0, nb, [&](long long j) { return t0 + (double)j * dT; }, [&](int i, int n) { st.copy(C + (size_t)cs * i, n, cs); },
+                [&](int k, double x, double& re, double& im) { modes_sample(st.c + k * cs, x, nm, mo, re, im); },
+                [&](int i, double x, double& re, double& im) { modes_sample(C + (size_t)cs * i, x, nm, mo, re, im); },
+                [&](long long j, const double (&re)[2], const double (&im)[2], bool full) { o.put(j, re, im, full); });
         o.zeros(j0);
     });
 }
@@ -983,8 +969,7 @@ int eobhip_resample_hplus(const double* dense, const double* coef, const int* nu
                           int max_step, int N, double* hplus, int* nsamp, void* stream) {
     EOBHIP_REQUIRE(n >= 0 && N >= 1 && n <= 65535, "bad sizes");
     if (n == 0) return EOBHIP_OK;
-    const int bx = resample_blocks(N, n);
-    hipLaunchKernelGGL(k_resample_hplus, dim3(bx, n), dim3(kBlock), 0, as_stream(stream), dense, coef, num_steps, amp, dT_M, max_step, N, hplus,
+    hipLaunchKernelGGL(k_resample_hplus, resample_grid(N, n), dim3(kBlock), 0, as_stream(stream), dense, coef, num_steps, amp, dT_M, max_step, N, hplus,
                        nsamp, nullptr);
     return check_launch("resample_hplus");
 }
@@ -994,24 +979,11 @@ int eobhip_resample_modes(const double* dense, const double* coef, const int* nu
     EOBHIP_REQUIRE(n >= 0 && N >= 1 && n <= 65535, "bad sizes");
     EOBHIP_REQUIRE(nm >= 1 && nm <= 15, "nm must be 1 .. 15");
     EOBHIP_REQUIRE(hplus && hcross, "hplus and hcross are required");
-    ModeMs mm;
-    mm.nm = nm;
-    for (int q = 0; q < nm; ++q) {
-        EOBHIP_REQUIRE(ms[q] >= 1 && ms[q] <= kMaxModeM, "m must be 1 .. 8");
-        mm.m[q] = ms[q];
-    }
+    for (int q = 0; q < nm; ++q) EOBHIP_REQUIRE(ms[q] >= 1 && ms[q] <= kMaxModeM, "m must be 1 .. 8");
     if (n == 0) return EOBHIP_OK;
-    const int bx = resample_blocks(N, n);
-    // built for the reference's five modes and for (2,2) alone; any other count runs the general build
-    if (nm == 5)
-        hipLaunchKernelGGL(k_resample_modes<5>, dim3(bx, n), dim3(kBlock), 0, as_stream(stream), dense, coef, num_steps, amp, dT_M,
-                           max_step, N, mm, hplus, hcross, nsamp);
-    else if (nm == 1)
-        hipLaunchKernelGGL(k_resample_modes<1>, dim3(bx, n), dim3(kBlock), 0, as_stream(stream), dense, coef, num_steps, amp, dT_M,
-                           max_step, N, mm, hplus, hcross, nsamp);
-    else
-        hipLaunchKernelGGL(k_resample_modes<0>, dim3(bx, n), dim3(kBlock), 0, as_stream(stream), dense, coef, num_steps, amp, dT_M,
-                           max_step, N, mm, hplus, hcross, nsamp);
+    const auto kernel = nm <= 5 ? k_resample_modes<5> : k_resample_modes<kMaxModes>;
+    hipLaunchKernelGGL(kernel, resample_grid(N, n), dim3(kBlock), 0, as_stream(stream), dense, coef, num_steps, amp, dT_M, max_step,
+                       N, nm, mode_order(ms, nm), hplus, hcross, nsamp);
     return check_launch("resample_modes");
 }
 
@@ -1036,8 +1008,7 @@ int eobhip_resample_hpc(const double* dense, const double* coef, const int* num_
     EOBHIP_REQUIRE(n >= 0 && N >= 1 && n <= 65535, "bad sizes");
     EOBHIP_REQUIRE(hcross != nullptr, "hcross is required");
     if (n == 0) return EOBHIP_OK;
-    const int bx = resample_blocks(N, n);
-    hipLaunchKernelGGL(k_resample_hplus, dim3(bx, n), dim3(kBlock), 0, as_stream(stream), dense, coef, num_steps, amp, dT_M, max_step, N, hplus,
+    hipLaunchKernelGGL(k_resample_hplus, resample_grid(N, n), dim3(kBlock), 0, as_stream(stream), dense, coef, num_steps, amp, dT_M, max_step, N, hplus,
                        nsamp, hcross);
     return check_launch("resample_hpc");
 }
