@@ -421,28 +421,71 @@ IMR_HD double final_spin_hbr2016(double m1, double m2, double chi1, double chi2)
 constexpr int kLeaverAngDepth = 60;
 constexpr int kLeaverRadDepth = 300;   // n = 0 converged to 5e-15 up to a = 0.98
 
-// angular continued fraction beta_0 - alpha_0 gamma_1 / (beta_1 - ...)
-IMR_HD Cx leaver_angular_cf(Cx A, Cx c, int s, int m) {
+// angular terms: fraction beta_0 - alpha_0 gamma_1 / (beta_1 - ...)
+struct LeaverAng {
+    double k1, k12, s;   // k1, k1 + k2
+    Cx c, v;             // v: the part of beta without n
+};
+IMR_HD LeaverAng leaver_angular(Cx A, Cx c, int s, int m) {
     const double k1 = 0.5 * fabs((double)(m - s)), k2 = 0.5 * fabs((double)(m + s));
-    const Cx cc = c * c;
     // beta_n = n(n-1) + 2n(k1+k2+1-2c) - [2c(2k1+s+1) - (k1+k2)(k1+k2+1)] - [c^2 + s(s+1) + A]
-    auto beta = [&](int n) {
-        const double dn = n;
-        const Cx t = cx(dn * (dn - 1.0) + 2.0 * dn * (k1 + k2 + 1.0)) - (4.0 * dn) * c;
-        const Cx u = (2.0 * (2.0 * k1 + s + 1.0)) * c - (k1 + k2) * (k1 + k2 + 1.0);
-        return t - u - (cc + (double)(s * (s + 1)) + A);
-    };
-    auto alpha = [&](int n) { return cx(-2.0 * (n + 1.0) * (n + 2.0 * k1 + 1.0)); };
-    auto gamma = [&](int n) { return (2.0 * (n + k1 + k2 + s)) * c; };
-    Cx t = beta(kLeaverAngDepth);
-    for (int n = kLeaverAngDepth - 1; n >= 0; --n) t = beta(n) - alpha(n) * gamma(n + 1) / t;
-    return t;
+    const Cx u = (2.0 * (2.0 * k1 + s + 1.0)) * c - (k1 + k2) * (k1 + k2 + 1.0);
+    return LeaverAng{k1, k1 + k2, (double)s, c, u + (c * c + (double)(s * (s + 1)) + A)};
+}
+IMR_HD Cx leaver_beta(const LeaverAng& f, int n) {
+    const double dn = n;
+    return cx(dn * (dn - 1.0) + 2.0 * dn * (f.k12 + 1.0)) - (4.0 * dn) * f.c - f.v;
+}
+// alpha_n gamma_{n+1}
+IMR_HD Cx leaver_alpha_gamma(const LeaverAng& f, int n) {
+    return (-4.0 * (n + 1.0) * (n + 2.0 * f.k1 + 1.0) * (n + 1.0 + f.k12 + f.s)) * f.c;
 }
 
+// radial terms alpha_n = (n + 1)(n + c0), beta_n = -2 n^2 + (2 + c1) n + c3,
+// gamma_n = (n - 1)(n - 2) + c2 (n - 1) + c4 at omega for spin a (2 M = 1);
+// c0 + c1 + c2 = 2 i b omega
+struct LeaverRad {
+    Cx c0, c1, c2, c3, c4, c012;
+};
+IMR_HD LeaverRad leaver_radial(Cx w, double a, int s, int m, Cx A) {
+    const double b = sqrt(1.0 - 4.0 * a * a);
+    const Cx I = cx(0.0, 1.0);
+    const Cx wm = 0.5 * w - a * m;                // omega/2 - a m
+    const Cx iwm_b = (2.0 / b) * (I * wm);        // (2i/b)(omega/2 - a m)
+    LeaverRad f;
+    f.c0 = cx(1.0 - s) - I * w - iwm_b;
+    f.c1 = cx(-4.0) + (2.0 + b) * 2.0 * (I * w) + 2.0 * iwm_b;
+    f.c2 = cx(s + 3.0) - 3.0 * (I * w) + (-1.0) * iwm_b;
+    const Cx f4 = (4.0 * w + 2.0 * I) * wm * (1.0 / b);   // ((4 omega + 2i)/b)(omega/2 - a m)
+    f.c3 = w * w * (4.0 + 2.0 * b - a * a) - (2.0 * a * m) * w - (double)(s + 1) + (2.0 + b) * (I * w) - A + f4;
+    f.c4 = cx(s + 1.0) - 2.0 * (w * w) - (2.0 * s + 3.0) * (I * w) - f4;
+    f.c012 = (2.0 * b) * (I * w);
+    return f;
+}
+
+// The fractions from their last term back, a division per term
+struct LeaverSerial {
+    IMR_HD static Cx fraction(const LeaverAng& f) {
+        Cx t = leaver_beta(f, kLeaverAngDepth);
+        for (int n = kLeaverAngDepth - 1; n >= 0; --n) t = leaver_beta(f, n) - leaver_alpha_gamma(f, n) / t;
+        return t;
+    }
+    IMR_HD static Cx fraction(const LeaverRad& f) {
+        auto alpha = [&](int n) { const double d = n; return cx(d * d + d) + (f.c0 * d) + f.c0; };
+        auto beta = [&](int n) { const double d = n; return cx(-2.0 * d * d + 2.0 * d) + (f.c1 * d) + f.c3; };
+        auto gamma = [&](int n) { const double d = n; return cx(d * d - 3.0 * d + 2.0) + (f.c2 * d) + f.c4 - f.c2; };
+        Cx t = beta(kLeaverRadDepth);
+        for (int n = kLeaverRadDepth - 1; n >= 0; --n) t = beta(n) - alpha(n) * gamma(n + 1) / t;
+        return t;
+    }
+};
+
 // the separation constant nearest A0 (Newton with a complex-step-free secant)
+template <class Cf>
 IMR_HD Cx leaver_angular_solve(Cx A0, Cx c, int s, int m) {
+    const auto cf = [&](Cx A) { return Cf::fraction(leaver_angular(A, c, s, m)); };
     Cx a = A0, b = A0 + cx(1e-3, 1e-3);
-    Cx fa = leaver_angular_cf(a, c, s, m), fb = leaver_angular_cf(b, c, s, m);
+    Cx fa = cf(a), fb = cf(b);
     for (int it = 0; it < 60; ++it) {
         const Cx d = fb - fa;
         if (cabs2(d) == 0.0) break;
@@ -450,7 +493,7 @@ IMR_HD Cx leaver_angular_solve(Cx A0, Cx c, int s, int m) {
         a = b;
         fa = fb;
         b = nb;
-        fb = leaver_angular_cf(b, c, s, m);
+        fb = cf(b);
         if (cabs2(b - a) < 1e-28 * (1.0 + cabs2(b))) break;
     }
     return b;
@@ -458,24 +501,10 @@ IMR_HD Cx leaver_angular_solve(Cx A0, Cx c, int s, int m) {
 
 // radial continued fraction at omega for spin a (2 M = 1), with A solved from
 // the guess *A (updated)
+template <class Cf>
 IMR_HD Cx leaver_radial_cf(Cx w, double a, int s, int m, Cx* A) {
-    *A = leaver_angular_solve(*A, a * w, s, m);
-    const double b = sqrt(1.0 - 4.0 * a * a);
-    const Cx I = cx(0.0, 1.0);
-    const Cx wm = 0.5 * w - a * m;                // omega/2 - a m
-    const Cx iwm_b = (2.0 / b) * (I * wm);        // (2i/b)(omega/2 - a m)
-    const Cx c0 = cx(1.0 - s) - I * w - iwm_b;
-    const Cx c1 = cx(-4.0) + (2.0 + b) * 2.0 * (I * w) + 2.0 * iwm_b;
-    const Cx c2 = cx(s + 3.0) - 3.0 * (I * w) + (-1.0) * iwm_b;
-    const Cx f4 = (4.0 * w + 2.0 * I) * wm * (1.0 / b);   // ((4 omega + 2i)/b)(omega/2 - a m)
-    const Cx c3 = w * w * (4.0 + 2.0 * b - a * a) - (2.0 * a * m) * w - (double)(s + 1) + (2.0 + b) * (I * w) - *A + f4;
-    const Cx c4 = cx(s + 1.0) - 2.0 * (w * w) - (2.0 * s + 3.0) * (I * w) - f4;
-    auto alpha = [&](int n) { const double d = n; return cx(d * d + d) + (c0 * d) + c0; };
-    auto beta = [&](int n) { const double d = n; return cx(-2.0 * d * d + 2.0 * d) + (c1 * d) + c3; };
-    auto gamma = [&](int n) { const double d = n; return cx(d * d - 3.0 * d + 2.0) + (c2 * d) + c4 - c2; };
-    Cx t = beta(kLeaverRadDepth);
-    for (int n = kLeaverRadDepth - 1; n >= 0; --n) t = beta(n) - alpha(n) * gamma(n + 1) / t;
-    return t;
+    *A = leaver_angular_solve<Cf>(*A, a * w, s, m);
+    return Cf::fraction(leaver_radial(w, a, s, m, *A));
 }
 
 // The root of the radial continued fraction near w (Leaver units) at spin a,
@@ -483,12 +512,13 @@ IMR_HD Cx leaver_radial_cf(Cx w, double a, int s, int m, Cx* A) {
 struct QnmRoot {
     Cx w, A;
 };
+template <class Cf>
 IMR_HD QnmRoot leaver_refine(int m, double a, Cx w, Cx A, double dw) {
     const int s = -2;
     Cx x0 = w, x1 = w + cx(dw, -dw);
     Cx A0 = A, A1 = A;
-    Cx f0 = leaver_radial_cf(x0, a, s, m, &A0);
-    Cx f1 = leaver_radial_cf(x1, a, s, m, &A1);
+    Cx f0 = leaver_radial_cf<Cf>(x0, a, s, m, &A0);
+    Cx f1 = leaver_radial_cf<Cf>(x1, a, s, m, &A1);
     for (int it = 0; it < 50; ++it) {
         const Cx d = f1 - f0;
         if (cabs2(d) == 0.0) break;
@@ -497,7 +527,7 @@ IMR_HD QnmRoot leaver_refine(int m, double a, Cx w, Cx A, double dw) {
         f0 = f1;
         A0 = A1;
         x1 = x2;
-        f1 = leaver_radial_cf(x1, a, s, m, &A1);
+        f1 = leaver_radial_cf<Cf>(x1, a, s, m, &A1);
         if (cabs2(x1 - x0) < 1e-30 * (1.0 + cabs2(x1))) break;
     }
     return QnmRoot{x1, A1};
@@ -522,7 +552,7 @@ IMR_HD QnmRoot kerr_qnm_path(int l, int m, double af) {
         const double a = a_end * (double)k / nstep;
         const Cx guess = (k > 1) ? (2.0 * r.w - wprev) : r.w;   // linear extrapolation along the path
         wprev = r.w;
-        r = leaver_refine(m, a, guess, r.A, 1e-4);
+        r = leaver_refine<LeaverSerial>(m, a, guess, r.A, 1e-4);
     }
     return r;
 }

@@ -23,7 +23,7 @@
 
 #include "eobhip_common.hpp"
 #include "imr.hpp"
-#include "knot_window.hpp"
+#include "resample.hpp"
 #include "spline_nak.hpp"
 
 using namespace eobhip_detail;
@@ -95,6 +95,10 @@ __device__ __forceinline__ int knot_index(const double* __restrict__ T, int len,
 struct Piece {
     double x, x2, x3;
     bool last;
+    __device__ static Piece at(double x, bool last) {
+        const double x2 = x * x;
+        return Piece{x, x2, x2 * x, last};
+    }
     template <class Ptr>
     __device__ double v(Ptr c) const { return last ? c[0] : c[0] + c[1] * x + c[2] * x2 + c[3] * x3; }
     template <class Ptr>
@@ -234,8 +238,76 @@ __global__ void k_qnm_table() {
     o[3] = r.A.im;
 }
 
-// M omega_lm0 at spin af: from the table for the ringdown modes, |af| <= 0.99;
-// otherwise along the spin path from a = 0
+// The fractions by 16 lanes (the same value, bit for bit, on all of them).  t_n =
+// beta_n - alpha_n gamma_{n+1} / t_{n+1} is a Moebius map, so a lane multiplies the
+// 2 x 2 matrices of its run of terms (no divisions) and four exchanges multiply
+// the runs.  The radial maps are close to t -> -n^2 (2 + n^2 / t), whose products
+// cancel: they act on t + n^2 instead, where what is left of alpha_n gamma_{n+1} is
+// (n + 1)(c012 n^2 + e1 n + e0).  One secant step was 300 + 5 x 60 complex divisions
+// in turn; QNMs of 512 binaries x 5 modes 800 us, 109 now.  Roots for |a| <= 0.97
+// against extended precision: within 3.9e-15 (serial 1.9e-15, both near a = -0.97;
+// 5.1e-16 and 4.6e-16 up to 0.8, rms equal).
+constexpr int kQnmLanes = 16;
+struct Moebius {
+    Cx a, b, c, d;
+};
+__device__ __forceinline__ Cx mul_add(Cx x, Cx y, Cx z, Cx w) {
+    return imr::cx(x.re * y.re - x.im * y.im + z.re * w.re - z.im * w.im, x.re * y.im + x.im * y.re + z.re * w.im + z.im * w.re);
+}
+// by a power of two to the size of 1
+__device__ __forceinline__ void moebius_scale(Moebius& m) {
+    const double s = fmax(fmax(fmax(fabs(m.a.re), fabs(m.a.im)), fmax(fabs(m.b.re), fabs(m.b.im))),
+                          fmax(fmax(fabs(m.c.re), fabs(m.c.im)), fmax(fabs(m.d.re), fabs(m.d.im))));
+    const double f = s > 0.0 && s < 1e300 ? ldexp(1.0, -ilogb(s)) : 1.0;
+    m.a = f * m.a;
+    m.b = f * m.b;
+    m.c = f * m.c;
+    m.d = f * m.d;
+}
+__device__ __forceinline__ Cx shfl_xor_cx(Cx v, int off) { return imr::cx(__shfl_xor(v.re, off, 64), __shfl_xor(v.im, off, 64)); }
+// the lanes' product, applied to u
+__device__ __forceinline__ Cx moebius_apply(Moebius m, Cx u) {
+    moebius_scale(m);
+#pragma unroll
+    for (int off = 1; off < kQnmLanes; off <<= 1) {
+        const Moebius o{shfl_xor_cx(m.a, off), shfl_xor_cx(m.b, off), shfl_xor_cx(m.c, off), shfl_xor_cx(m.d, off)};
+        const bool up = threadIdx.x & off;
+        const Moebius l = up ? o : m, h = up ? m : o;
+        m = Moebius{mul_add(l.a, h.a, l.b, h.c), mul_add(l.a, h.b, l.b, h.d), mul_add(l.c, h.a, l.d, h.c), mul_add(l.c, h.b, l.d, h.d)};
+        moebius_scale(m);
+    }
+    return (m.a * u + m.b) / (m.c * u + m.d);
+}
+struct LeaverLanes {
+    __device__ static Cx fraction(const imr::LeaverAng& f) {
+        constexpr int D = imr::kLeaverAngDepth, per = (D + kQnmLanes - 1) / kQnmLanes;
+        const int lo = (int)(threadIdx.x % kQnmLanes) * per, hi = lo + per < D ? lo + per : D;
+        Moebius m{imr::cx(1.0), imr::cx(0.0), imr::cx(0.0), imr::cx(1.0)};
+#pragma unroll 1
+        for (int n = hi - 1; n >= lo; --n) {
+            const Cx be = imr::leaver_beta(f, n), g = -imr::leaver_alpha_gamma(f, n);
+            m = Moebius{mul_add(be, m.a, g, m.c), mul_add(be, m.b, g, m.d), m.a, m.b};
+        }
+        return moebius_apply(m, imr::leaver_beta(f, D));
+    }
+    __device__ static Cx fraction(const imr::LeaverRad& f) {
+        constexpr int D = imr::kLeaverRadDepth, per = (D + kQnmLanes - 1) / kQnmLanes;
+        const int lo = (int)(threadIdx.x % kQnmLanes) * per, hi = lo + per < D ? lo + per : D;
+        const Cx p = f.c1 + 2.0, e1 = p + f.c3 + f.c4 + f.c0 * (f.c2 - 1.0), e0 = f.c3 + f.c0 * f.c4;
+        Moebius m{imr::cx(1.0), imr::cx(0.0), imr::cx(0.0), imr::cx(1.0)};
+#pragma unroll 1
+        for (int n = hi - 1; n >= lo; --n) {
+            const double d = n, e = d + 1.0;
+            const Cx h = p * d + f.c3 - d * d, g = (-e) * ((f.c012 * d + e1) * d + e0);
+            m = Moebius{mul_add(h, m.a, g, m.c), mul_add(h, m.b, g, m.d), m.a - (e * e) * m.c, m.b - (e * e) * m.d};
+        }
+        const double d = D;
+        return moebius_apply(m, p * d + f.c3 - d * d);
+    }
+};
+
+// M omega_lm0 at spin af, by the kQnmLanes lanes of a group: from the table for the
+// ringdown modes, |af| <= 0.99; otherwise along the spin path from a = 0
 __device__ Cx kerr_qnm_fast(int l, int m, double af) {
     const int k = imr::rd_mode_index(l, m);
     if (k < 0 || !(fabs(af) <= 0.99)) return imr::kerr_qnm(l, m, af);
@@ -247,7 +319,7 @@ __device__ Cx kerr_qnm_fast(int l, int m, double af) {
     const double* p1 = g_qnm_tab[k][i + 1];
     const Cx w = imr::cx((1.0 - f) * p0[0] + f * p1[0], (1.0 - f) * p0[1] + f * p1[1]);
     const Cx A = imr::cx((1.0 - f) * p0[2] + f * p1[2], (1.0 - f) * p0[3] + f * p1[3]);
-    const imr::QnmRoot r = imr::leaver_refine(m, 0.5 * af, w, A, 1e-6);
+    const imr::QnmRoot r = imr::leaver_refine<LeaverLanes>(m, 0.5 * af, w, A, 1e-6);
     return imr::cx(0.5 * r.w.re, 0.5 * r.w.im);
 }
 
@@ -271,13 +343,13 @@ int ensure_qnm_table(void* stream) {
 }
 
 // ------------------------------------------------------------ QNMs per binary
-// Thread (b, j): j < nm the QNM of mode j, j == nm the (2,2) QNM that sets the
+// Lanes (b, j) of a group: j < nm the QNM of mode j, j == nm the (2,2) QNM that sets the
 // ringdown length (the reference's 30 damping times, :2463-2465 and :2514).
 // wl [n][nm] complex in lalsimulation's convention (omega_r + i / tau) in
 // units of the total mass; binf/bini as the enums.
 __global__ void k_imr_qnm(BinInputs in, const double* __restrict__ dense, const double* __restrict__ dT_M, int n, int max_step,
                           ImrModes mm, double* __restrict__ wl, double* __restrict__ binf, int* __restrict__ bini) {
-    const long long gid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long long gid = ((long long)blockIdx.x * blockDim.x + threadIdx.x) / kQnmLanes;
     const int per = mm.nm + 1;
     if (gid >= (long long)n * per) return;
     const int b = (int)(gid / per), j = (int)(gid % per);
@@ -287,6 +359,7 @@ __global__ void k_imr_qnm(BinInputs in, const double* __restrict__ dense, const 
     const double af = imr::final_spin_hbr2016(m1 / M, m2 / M, c1, c2);
     const int l = (j < mm.nm) ? mm.l[j] : 2, m = (j < mm.nm) ? mm.m[j] : 2;
     const Cx w = kerr_qnm_fast(l, m, af);
+    if (threadIdx.x % kQnmLanes != 0) return;
     const double wr = w.re / mf, wi = -w.im / mf;   // conj(omega) / M_f
     if (j < mm.nm) {
         wl[2 * ((size_t)b * mm.nm + j)] = wr;
@@ -506,23 +579,15 @@ __global__ __launch_bounds__(64) void k_imr_params(BinInputs in, const double* _
 
 // sin and cos of x: Taylor series through x^9 / x^10 when every active lane of
 // the wavefront has |x| < 1/16 (first omitted terms below 2.3e-20 relative),
-// through x^17 / x^18 for |x| < 1/2 (below 2e-23), the library's sincos
-// otherwise.  The NQC phase of the inspiral samples is small except near the
+// sincos_phase otherwise.  The NQC phase of the inspiral samples is small except near the
 // attachment.
 __device__ __forceinline__ void sincos_nqc(double x, double* s, double* c) {
-    const double ax = fabs(x);
-    if (__all(ax < 0.0625)) {
+    if (__all(fabs(x) < 0.0625)) {
         const double x2 = x * x;
         *s = x * (1.0 + x2 * (-1.0 / 6 + x2 * (1.0 / 120 + x2 * (-1.0 / 5040 + x2 * (1.0 / 362880)))));
         *c = 1.0 + x2 * (-0.5 + x2 * (1.0 / 24 + x2 * (-1.0 / 720 + x2 * (1.0 / 40320 + x2 * (-1.0 / 3628800)))));
-    } else if (ax < 0.5) {
-        const double x2 = x * x;
-        *s = x * (1.0 + x2 * (-1.0 / 6 + x2 * (1.0 / 120 + x2 * (-1.0 / 5040 + x2 * (1.0 / 362880 + x2 * (-1.0 / 39916800
-                 + x2 * (1.0 / 6227020800.0 + x2 * (-1.0 / 1307674368000.0 + x2 * (1.0 / 355687428096000.0)))))))));
-        *c = 1.0 + x2 * (-0.5 + x2 * (1.0 / 24 + x2 * (-1.0 / 720 + x2 * (1.0 / 40320 + x2 * (-1.0 / 3628800 + x2 * (1.0 / 479001600.0
-                 + x2 * (-1.0 / 87178291200.0 + x2 * (1.0 / 20922789888000.0 + x2 * (-1.0 / 6402373705728000.0)))))))));
     } else {
-        sincos(x, s, c);
+        sincos_phase(x, s, c);
     }
 }
 
@@ -530,125 +595,140 @@ __device__ __forceinline__ void sincos_nqc(double x, double* s, double* c) {
 // h_j = amp (sum over modes of h_lm NQC_lm (t_j) for j <= idx, of the ringdown
 // for idx < j < idx + nadd, 0 after), t_j = t_0 + j dT; hplus = Re, hcross = Im.
 constexpr int kImrBlock = 256;
-constexpr int kImrSpan = 2048;
 
-// One inspiral sample's sum over the NM modes: row holds the interval's
-// spline coefficients (Re of each mode, Im of each mode, phi), rpr those of r
-// and pr; nq the binary's NQC coefficients (5 per mode).  e^{-i m phi} is
-// formed from e^{-i phi} by m - 1 products (the same products as a table of
-// its powers, without selecting from the table per mode).
-template <int NM, class Ptr>
-__device__ __forceinline__ void imr_inspiral_sample(Ptr row, Ptr rpr, const Piece& p, const ImrModes& mm, const double* __restrict__ nq,
-                                                    double& hr, double& hi) {
-    const double phi = p.v(row + 4 * (2 * NM));
-    const double om = p.d(row + 4 * (2 * NM));
-    const double r = p.v(rpr), pr = p.v(rpr + 4);
-    const double sr = sqrt(r), rO = r * om;
-    const double P = pr * pr / (rO * rO);
-    const double ir = 1.0 / r, irs = 1.0 / (r * sr);
-    const double p1 = pr / rO, p3 = pr * pr * pr / rO;
-    double sp, cph;
-    sincos(phi, &sp, &cph);
-#pragma unroll
-    for (int q = 0; q < NM; ++q) {
-        const double re = p.v(row + 4 * q), im = p.v(row + 4 * (NM + q));
-        double pr_ = cph, pi_ = -sp;   // e^{-i phi}
-        for (int k = 1; k < mm.m[q]; ++k) {
-            const double t = pr_ * cph + pi_ * sp;
-            pi_ = pi_ * cph - pr_ * sp;
-            pr_ = t;
+// One inspiral sample's sum over the modes: row holds the interval's spline
+// coefficients (Re of each mode, Im of each mode, phi), rpr those of r and pr; nq
+// the binary's NQC coefficients (5 per mode).  sum_m h_m e^{-i m phi} by Horner's
+// rule in e^{-i phi} over the modes by falling m (mo): each mode then costs the
+// products between its m and the next one's, not m - 1 of its own.
+template <class Ptr>
+__device__ __forceinline__ void imr_inspiral_sample(Ptr row, Ptr rpr, const Piece& p, int nm, const ModeOrder& mo, const double* nq,
+                                                    double& re_out, double& im_out) {
+    const double om = p.d(row + 4 * (2 * nm)), r = p.v(rpr), pr = p.v(rpr + 4);
+    const double irO = 1.0 / (r * om);
+    const double p1 = pr * irO, p3 = pr * pr * p1, P = p1 * p1;
+    const double ir = om * irO, irs = ir * rsqrt(r);
+    double sp, cph, hr = 0.0, hi = 0.0;
+    sincos_phase(p.v(row + 4 * (2 * nm)), &sp, &cph);
+    const auto turn = [&](int k) {
+        for (; k > 0; --k) {
+            const double t = hr * cph + hi * sp;
+            hi = hi * cph - hr * sp;
+            hr = t;
         }
-        const double h_r = re * pr_ - im * pi_, h_i = re * pi_ + im * pr_;
+    };
+#pragma unroll 1
+    for (int k = 0; k < nm; ++k) {
+        const int q = mo.q(k);
+        const Ptr rq = row + 4 * q, iq = row + 4 * (nm + q);
         const double* c = nq + 5 * q;
-        const double mag = 1.0 + P * (c[0] + c[1] * ir + c[2] * irs);
         double sn, cn;
         sincos_nqc(c[3] * p1 + p3 * c[4], &sn, &cn);
-        const double fr = mag * cn, fi = mag * sn;
-        hr += h_r * fr - h_i * fi;
-        hi += h_r * fi + h_i * fr;
+        turn(mo.down(k));
+        const double mag = 1.0 + P * (c[0] + c[1] * ir + c[2] * irs);
+        const double re = p.v(rq), im = p.v(iq), fr = mag * cn, fi = mag * sn;
+        hr += re * fr - im * fi;
+        hi += re * fi + im * fr;
+    }
+    turn(mo.down(nm));
+    re_out = hr;
+    im_out = hi;
+}
+
+// samples of a template: inspiral 0 .. idx, ringdown to idx + nadd; 0: none
+__device__ __forceinline__ long long imr_samples(int idx, int nadd, int len) {
+    return (idx < 0 || len < 4) ? 0 : (long long)idx + (nadd > 0 ? nadd : 1);
+}
+
+// Ringdown samples (idx < j < idx + nadd), over the zeros of the inspiral's kernel:
+// a kernel of its own, since its functions would double that one's registers for
+// the few hundred samples of a binary.  grid (blocks, binaries).
+__global__ __launch_bounds__(kImrBlock) void k_imr_ringdown(const int* __restrict__ num_steps, const double* __restrict__ amp, int N, int nm,
+                                                            const double* __restrict__ rd, const double* __restrict__ binf,
+                                                            const int* __restrict__ bini, double* __restrict__ hplus,
+                                                            double* __restrict__ hcross) {
+    const int b = blockIdx.y;
+    const int idx = bini[(size_t)b * kBinICount + kBinIdx];
+    const long long end = imr_samples(idx, bini[(size_t)b * kBinICount + kBinNadd], num_steps[b]);
+    const double a = amp[b], t_match = binf[(size_t)b * kBinCount + kBinTMatch], dt = binf[(size_t)b * kBinCount + kBinDt];
+    const long long stop = end < N ? end : N;
+    for (long long j = (long long)idx + 1 + (long long)blockIdx.x * kImrBlock + threadIdx.x; j < stop; j += (long long)gridDim.x * kImrBlock) {
+        const double x = (t_match + (double)(j - idx) * dt) - t_match;
+        double hr = 0.0, hi = 0.0;
+        for (int q = 0; q < nm; ++q) {
+            const double* o = rd + ((size_t)b * nm + q) * kRdCount;
+            const double Alm = o[kRdC1c] * tanh(o[kRdC1f] * x + o[kRdC2f]) + o[kRdC2c];
+            const double philm = o[kRdPhi] - o[kRdD1c] * log((1.0 + o[kRdD2f] * exp(-o[kRdD1f] * x)) / (1.0 + o[kRdD2f]));
+            const double mod = o[kRdEta] * Alm * exp(-o[kRdWi] * x);
+            double s, c;
+            sincos(philm - o[kRdWr] * x, &s, &c);
+            hr += mod * c;
+            hi += mod * s;
+        }
+        hplus[(size_t)b * N + j] = a * hr;
+        hcross[(size_t)b * N + j] = a * hi;
     }
 }
 
-// grid (blocks, binaries); a block takes spans of kImrSpan samples, stages the
-// knot times of their inspiral part in LDS (knot_window) and searches there.
-// When all lanes of a wavefront sample one knot interval, its coefficient
-// rows are read once through the scalar cache (constant address space: the
-// tables are read-only while the kernel runs).
-template <int NM>
+// grid (blocks, binaries), runs of samples per wavefront (resample.hpp).  512
+// binaries x 2^20 samples at 16384 Hz, five modes, 32% of them inspiral: 6100 us
+// with knot windows per block, four divisions, a square root and ten complex
+// products a sample, 3055 now.  The arithmetic alone is 1540 (330 instructions a
+// sample at the FP64 rate) and the writes 1360: a binary's blocks run together, so
+// the two hardly overlap (taking the binaries in turn instead scatters the writes
+// and costs 3700).  Three wavefronts a SIMD; four (spills) or two samples at once
+// (two wavefronts) are no faster.
+// kModes: the most modes the staged rows have room for.
+template <int kModes>
 __global__ __launch_bounds__(kImrBlock) void k_imr_resample(const double* __restrict__ dense, const int* __restrict__ num_steps,
                                                             const double* __restrict__ coef, const double* __restrict__ rp,
                                                             const double* __restrict__ amp, const double* __restrict__ dT_M, int max_step,
-                                                            int N, ImrModes mm, const double* __restrict__ nqc, const double* __restrict__ rd,
-                                                            const double* __restrict__ binf, const int* __restrict__ bini,
-                                                            double* __restrict__ hplus, double* __restrict__ hcross, int* __restrict__ nsamp) {
-    typedef const __attribute__((address_space(4))) double* ConstPtr;
-    constexpr int cs = 4 * (2 * NM + 1);
+                                                            int N, int nm, ModeOrder mo, const double* __restrict__ nqc,
+                                                            const int* __restrict__ bini, double* __restrict__ hplus,
+                                                            double* __restrict__ hcross, int* __restrict__ nsamp) {
+    const int cs = 4 * (2 * nm + 1);
     const int b = blockIdx.y;
     const int len = num_steps[b];
     const int idx = bini[(size_t)b * kBinICount + kBinIdx];
     const int nadd = bini[(size_t)b * kBinICount + kBinNadd];
-    double* outp = hplus + (size_t)b * N;
-    double* outc = hcross + (size_t)b * N;
-    const long long nvalid = (idx < 0 || len < 4) ? 0 : (long long)idx + (nadd > 0 ? nadd : 1);
+    const long long nvalid = imr_samples(idx, nadd, len);
     if (blockIdx.x == 0 && threadIdx.x == 0) nsamp[b] = (int)(nvalid < N ? nvalid : N);
+    const long long jinsp = nvalid == 0 ? 0 : ((long long)idx + 1 < N ? (long long)idx + 1 : N);   // inspiral samples j < jinsp
     const double* T = dense + (size_t)b * max_step * 5;
     const double* C = coef + (size_t)b * max_step * cs;
     const double* RP = rp + (size_t)b * max_step * 8;
-    const double* nq = nqc + (size_t)b * NM * 5;
-    const double t0 = T[0];
-    const double dT = dT_M[b];
-    const double a = amp[b];
-    const double t_match = binf[(size_t)b * kBinCount + kBinTMatch];
-    const double dt = binf[(size_t)b * kBinCount + kBinDt];
-    __shared__ KnotWindow<kImrBlock> win;
-    const long long nspan = ((long long)N + kImrSpan - 1) / kImrSpan;
-    for (long long sp0 = blockIdx.x; sp0 < nspan; sp0 += gridDim.x) {
-        const long long j0 = sp0 * kImrSpan;
-        const long long jinsp = (long long)idx + 1 < N ? (long long)idx + 1 : N;   // inspiral samples j < jinsp
-        if (j0 < jinsp && nvalid > 0) {
-            const long long jmax = (j0 + kImrSpan < jinsp ? j0 + kImrSpan : jinsp) - 1;
-            knot_window<kImrBlock>(win, T, 5, len, grid_t(j0, dT, t0), grid_t(jmax, dT, t0));
-        }
-        for (int u = 0; u < kImrSpan / kImrBlock; ++u) {
-            const long long j = j0 + (long long)u * kImrBlock + threadIdx.x;
-            if (j >= N) break;
-            double hr = 0.0, hi = 0.0;
-            if (nvalid > 0 && j <= idx) {
-                const double tj = grid_t(j, dT, t0);
-                const int ind = knot_interval<kImrBlock>(win, T, 5, len, tj);
-                const int i0 = __builtin_amdgcn_readfirstlane(ind);
-                Piece p;
-                p.last = (ind == len - 1);
-                if (__all(ind == i0)) {
-                    p.x = tj - ((ConstPtr)T)[5 * (size_t)i0];
-                    p.x2 = p.x * p.x;
-                    p.x3 = p.x2 * p.x;
-                    imr_inspiral_sample<NM>((ConstPtr)(C + (size_t)cs * i0), (ConstPtr)(RP + (size_t)8 * i0), p, mm, nq, hr, hi);
-                } else {
-                    p.x = tj - T[5 * (size_t)ind];
-                    p.x2 = p.x * p.x;
-                    p.x3 = p.x2 * p.x;
-                    imr_inspiral_sample<NM>(C + (size_t)cs * ind, RP + (size_t)8 * ind, p, mm, nq, hr, hi);
-                }
-            } else if (nvalid > 0 && j < nvalid) {
-                const long long k = j - idx;
-                const double x = (t_match + (double)k * dt) - t_match;
-                for (int q = 0; q < NM; ++q) {
-                    const double* o = rd + ((size_t)b * NM + q) * kRdCount;
-                    const double Alm = o[kRdC1c] * tanh(o[kRdC1f] * x + o[kRdC2f]) + o[kRdC2c];
-                    const double philm = o[kRdPhi] - o[kRdD1c] * log((1.0 + o[kRdD2f] * exp(-o[kRdD1f] * x)) / (1.0 + o[kRdD2f]));
-                    const double mod = o[kRdEta] * Alm * exp(-o[kRdWi] * x);
-                    double s, c;
-                    sincos(philm - o[kRdWr] * x, &s, &c);
-                    hr += mod * c;
-                    hi += mod * s;
-                }
-            }
-            outp[j] = a * hr;
-            outc[j] = a * hi;
-        }
-        __syncthreads();   // the window is rewritten by the next span
-    }
+    const double t0 = T[0], dT = dT_M[b];
+    const SeriesOut o{hplus + (size_t)b * N, hcross + (size_t)b * N, amp[b], jinsp, N};
+    struct Stage {
+        StagedRows<4 * (2 * kModes + 1), 8> modes;   // rows at their own stride cs
+        StagedRows<8, 8> rp;
+        double nq[5 * kModes];
+    };
+    __shared__ Stage stages[kImrBlock / 64];
+    Stage& st = stages[threadIdx.x >> 6];
+    if ((int)(threadIdx.x & 63) < 5 * nm) st.nq[threadIdx.x & 63] = nqc[(size_t)b * nm * 5 + (threadIdx.x & 63)];
+    for_runs(N, kImrBlock / 64, [&](long long j0) {
+        if (j0 < jinsp)
+            resample_rows<8>(
+                T, len, j0, jinsp, [&](long long j) { return grid_t(j, dT, t0); },
+                [&](int i, int n) {
+                    st.modes.copy(C + (size_t)cs * i, n, cs);
+                    st.rp.copy(RP + (size_t)8 * i, n);
+                    if (i + n == len) {   // the last knot's interval: its value, no slope
+                        __builtin_amdgcn_wave_barrier();
+                        st.modes.flatten(n - 1, cs);
+                        st.rp.flatten(n - 1);
+                    }
+                },
+                [&](int k, double x, double& re, double& im) {
+                    imr_inspiral_sample(st.modes.c + k * cs, st.rp.c + 8 * k, Piece::at(x, false), nm, mo, st.nq, re, im);
+                },
+                [&](int i, double x, double& re, double& im) {
+                    imr_inspiral_sample(C + (size_t)cs * i, RP + (size_t)8 * i, Piece::at(x, i == len - 1), nm, mo, st.nq, re, im);
+                },
+                [&](long long j, const double (&re)[2], const double (&im)[2], bool full) { o.put(j, re, im, full); });
+        o.zeros(j0);
+    });
 }
 
 // ---------------------------------------------------------- drop-in fits
@@ -679,9 +759,10 @@ __global__ void k_imr_fit(int which, int l, int m, const double* __restrict__ x1
 }
 
 __global__ void k_kerr_qnm(int l, int m, const double* __restrict__ af, int n, double* __restrict__ out) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const long long i = ((long long)blockIdx.x * blockDim.x + threadIdx.x) / kQnmLanes;
     if (i >= n) return;
     const Cx w = kerr_qnm_fast(l, m, af[i]);
+    if (threadIdx.x % kQnmLanes != 0) return;
     out[2 * i] = w.re;
     out[2 * i + 1] = w.im;
 }
@@ -715,7 +796,7 @@ int eobhip_kerr_qnm(int l, int m, const double* af, int n, double* omega, void* 
     if (n == 0) return EOBHIP_OK;
     const int rc = ensure_qnm_table(stream);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_kerr_qnm, dim3(blocks_for(n, 64)), dim3(64), 0, as_stream(stream), l, m, af, n, omega);
+    hipLaunchKernelGGL(k_kerr_qnm, dim3(blocks_for(n, 64 / kQnmLanes)), dim3(64), 0, as_stream(stream), l, m, af, n, omega);
     return check_launch("kerr_qnm");
 }
 
@@ -731,7 +812,7 @@ int eobhip_imr_params(const double* m1, const double* m2, const double* chi1, co
     if (rc) return rc;
     const BinInputs in{m1, m2, chi1, chi2};
     const long long nq = (long long)n * (nm + 1);
-    hipLaunchKernelGGL(k_imr_qnm, dim3(blocks_for(nq, 64)), dim3(64), 0, as_stream(stream), in, dense, dT_M, n, max_step, mm, qnm, binf,
+    hipLaunchKernelGGL(k_imr_qnm, dim3(blocks_for(nq, 64 / kQnmLanes)), dim3(64), 0, as_stream(stream), in, dense, dT_M, n, max_step, mm, qnm, binf,
                        bini);
     rc = check_launch("imr_qnm");
     if (rc) return rc;
@@ -749,29 +830,15 @@ int eobhip_imr_resample(const double* dense, const int* num_steps, const double*
     if (rc) return rc;
     EOBHIP_REQUIRE(n >= 0 && n <= 65535 && N >= 1, "bad sizes");
     if (n == 0) return EOBHIP_OK;
-    int bx = (int)((N + (long long)kImrSpan - 1) / kImrSpan);
-    if (bx > 4096) bx = 4096;
-    const dim3 grid(bx, n), block(kImrBlock);
+    const dim3 grid = resample_grid(N, n), block(kImrBlock);
     hipStream_t st = as_stream(stream);
-#define EOBHIP_IMR_RESAMPLE(NM)                                                                                                             \
-    case NM:                                                                                                                              \
-        hipLaunchKernelGGL(k_imr_resample<NM>, grid, block, 0, st, dense, num_steps, coef, rp_coef, amp, dT_M, max_step, N, mm, nqc, rd,  \
-                           binf, bini, hplus, hcross, nsamp);                                                                             \
-        break;
-    switch (nm) {
-        EOBHIP_IMR_RESAMPLE(1)
-        EOBHIP_IMR_RESAMPLE(2)
-        EOBHIP_IMR_RESAMPLE(3)
-        EOBHIP_IMR_RESAMPLE(4)
-        EOBHIP_IMR_RESAMPLE(5)
-        EOBHIP_IMR_RESAMPLE(6)
-        EOBHIP_IMR_RESAMPLE(7)
-        EOBHIP_IMR_RESAMPLE(8)
-        default: break;   // make_modes has checked 1 <= nm <= kImrMaxModes
-    }
-    static_assert(kImrMaxModes == 8, "one instantiation per mode count");
-#undef EOBHIP_IMR_RESAMPLE
-    return check_launch("imr_resample");
+    static_assert(kImrMaxModes == 8, "room for every mode");
+    const auto kernel = nm <= 5 ? k_imr_resample<5> : k_imr_resample<8>;
+    hipLaunchKernelGGL(kernel, grid, block, 0, st, dense, num_steps, coef, rp_coef, amp, dT_M, max_step, N, nm, mode_order(mm.m, nm), nqc, bini,
+                       hplus, hcross, nsamp);
+    if ((rc = check_launch("imr_resample"))) return rc;
+    hipLaunchKernelGGL(k_imr_ringdown, dim3(4, n), block, 0, st, num_steps, amp, N, nm, rd, binf, bini, hplus, hcross);
+    return check_launch("imr_ringdown");
 }
 
 size_t eobhip_imr_rd_doubles(void) { return kRdCount; }
