@@ -27,6 +27,8 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr int kSpan = kRun * (kBlock / 64);    // resample: samples per block, a run per wavefront
+constexpr int kSpanLog2 = __builtin_ctz(kSpan);
+static_assert(1 << kSpanLog2 == kSpan);
 constexpr int kBinsPerThread = 8;              // hh: bins per thread per block
 constexpr int kBinSpan = kBlock * kBinsPerThread;
 
@@ -128,27 +130,51 @@ __global__ __launch_bounds__(kBlock) void k_lik_sizes(const double* __restrict__
     mlog2[b] = k;
 }
 
+// The support path's sample buffer: rows [first[q], first[q + 1]) of `order` are
+// binaries of one transform size, 2^lstride[q] samples apart from offset[q] on;
+// block[q] is the size's first block, 2^(lstride - log2 kSpan) (at least 1) a row.
+constexpr int kLikSizes = kRfftMaxLog2 - kRfftMinLog2 + 1;
+struct LikRows {
+    int count;
+    int first[kLikSizes + 1], block[kLikSizes + 1], lstride[kLikSizes];
+    long long offset[kLikSizes];
+    const long long* order;
+};
+
 // h+ = amp Re[S(t) e^{-2 i phi(t)}] from the spline coefficients (the uniform
 // resample of the full-length path) and per-block partial sums of h_j g_j,
 // partial [n][pstride].  grid (blocks, rows), a run of samples per wavefront
-// (resample.hpp).  kSupport: row r is binary map[r], at hbuf + r stride, only its
-// support written (to the next even count; a block past it leaves at once).
-// Otherwise row b at hbuf + rowoff[b], zero for nsamp <= j < M_b.
+// (resample.hpp).  kSupport: row r is binary order[r], only its support written (to
+// the next even count; a block past it leaves at once); all sizes in one launch,
+// the longest templates first, and a block index over what the sizes hold (ten
+// launches of 73 us, each with its own slow end; 616 in one; with the grid of
+// the longest for every row 729).  Otherwise row b at hbuf + rowoff[b], zero for nsamp <= j < M_b.
 template <bool kSupport>
 __global__ __launch_bounds__(kBlock) void k_lik_resample(const double* __restrict__ dense, const double* __restrict__ coef,
                                                          const int* __restrict__ num_steps, const double* __restrict__ amp,
                                                          const double* __restrict__ dT_M, const int* __restrict__ nsamp,
-                                                         const int* __restrict__ mlog2, const long long* __restrict__ rowoff,
-                                                         const long long* __restrict__ map, long long stride, int max_step,
-                                                         const double* __restrict__ g, double* __restrict__ hbuf,
+                                                         const int* __restrict__ mlog2, const long long* __restrict__ rowoff, LikRows rows,
+                                                         int max_step, const double* __restrict__ g, double* __restrict__ hbuf,
                                                          double* __restrict__ cross_partial, int pstride) {
-    const int b = kSupport ? (int)map[blockIdx.y] : blockIdx.y;
+    int b = blockIdx.y, bx = blockIdx.x;
+    double* out = hbuf;
+    if constexpr (kSupport) {
+        const int id = gridDim.x - 1 - blockIdx.x;
+        int q = 0;
+        while (q + 1 < rows.count && id >= rows.block[q + 1]) ++q;
+        const int lb = rows.lstride[q] > kSpanLog2 ? rows.lstride[q] - kSpanLog2 : 0;
+        const int r = (id - rows.block[q]) >> lb;
+        bx = (id - rows.block[q]) & ((1 << lb) - 1);
+        b = (int)rows.order[rows.first[q] + r];
+        out += rows.offset[q] + ((long long)r << rows.lstride[q]);
+    } else {
+        out += rowoff[b];
+    }
     const long long nb = nsamp[b];
-    if (kSupport && (long long)blockIdx.x * kSpan >= nb) return;
+    if (kSupport && (long long)bx * kSpan >= nb) return;
     const long long M = kSupport ? (nb + 1) & ~1LL : 1LL << mlog2[b];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const long long j0 = (long long)blockIdx.x * kSpan + wave * kRun;
-    double* out = hbuf + (kSupport ? blockIdx.y * stride : rowoff[b]);
+    const long long j0 = (long long)bx * kSpan + wave * kRun;
     double acc = 0.0;
     __shared__ H22Stage stages[kBlock / 64];
     if (j0 < nb) {
@@ -171,7 +197,7 @@ __global__ __launch_bounds__(kBlock) void k_lik_resample(const double* __restric
         for (long long r = done; r < kRunRows; ++r) store_pair<false>(out, j0 + r * kRow + 2 * lane, M, 0.0, 0.0);
     }
     const double s = block_sum(acc);
-    if (threadIdx.x == 0) cross_partial[(size_t)b * pstride + blockIdx.x] = s;
+    if (threadIdx.x == 0) cross_partial[(size_t)b * pstride + bx] = s;
 }
 
 // per-block partial sums of |X_q|^2 W^(M)_q, q <= M/2; grid (gx2, n)
@@ -365,7 +391,7 @@ int eobhip_lik_resample(const double* dense, const double* coef, const int* num_
     int rc = eobhip_lik_partial_blocks(max_mlog2, &gx, &gx2);
     if (rc) return rc;
     hipLaunchKernelGGL(k_lik_resample<false>, dim3(gx, n), dim3(kBlock), 0, as_stream(stream), dense, coef, num_steps, amp, dT_M, nsamp,
-                       mlog2, rowoff, nullptr, 0LL, max_step, g, hbuf, cross_partial, gx);
+                       mlog2, rowoff, LikRows{}, max_step, g, hbuf, cross_partial, gx);
     return check_launch("lik_resample");
 }
 
@@ -392,7 +418,7 @@ int eobhip_lik_finish(const double* X, const long long* xoff, const int* mlog2, 
 // samples and 8 M of the transform's intermediate go out and come back (M <=
 // 2^14: the samples only) instead of 8 M and the five or six passes of a plan.
 // 1024 templates of N = 2^20, M = 2^15 .. 2^20: the whole likelihood 5.75 ms with
-// plans per size, 2.00 in this form (73 us a size of resample, 235 of transforms
+// plans per size, 1.81 in this form (0.62 of it the resample, 0.24 each pass
 // of the largest).
 int eobhip_lik_evaluate(const double* dense, const double* coef, const int* num_steps, const double* amp, const double* dT_M,
                         const int* nsamp, const int* mlog2, const long long* order, int n, int max_step, int N, int nsizes,
@@ -402,33 +428,43 @@ int eobhip_lik_evaluate(const double* dense, const double* coef, const int* num_
     const int L = log2_exact(N);
     EOBHIP_REQUIRE(n >= 0 && n <= 65535 && max_step >= 1 && nsizes >= 0 && L >= 2, "bad sizes");
     if (n == 0) return EOBHIP_OK;
-    int kmax = 0;
-    long long total = 0;
+    LikRows sizes{};
+    sizes.order = order;
+    int kmax = 0, logs[kLikSizes];
+    long long total = 0, samples = 0, blocks = 0;
     for (int q = 0; q < nsizes; ++q) {
         EOBHIP_REQUIRE(size_log2[q] >= kRfftMinLog2 && size_log2[q] <= kRfftMaxLog2 && size_log2[q] >= m_min_log2 && size_log2[q] <= L,
                        "lik_evaluate: transform size 2^%d outside 2^%d .. 2^%d", size_log2[q], kRfftMinLog2, kRfftMaxLog2);
         EOBHIP_REQUIRE(size_count[q] >= 0, "lik_evaluate: negative count");
-        if (size_log2[q] > kmax) kmax = size_log2[q];
+        if (size_count[q] == 0) continue;
+        EOBHIP_REQUIRE(sizes.count < kLikSizes, "lik_evaluate: a size twice");
+        // a support is at most half of M unless M is the whole segment
+        const int k = size_log2[q], ls = k < L ? k - 1 : k;
+        logs[sizes.count] = k;
+        sizes.first[sizes.count] = (int)total;
+        sizes.offset[sizes.count] = samples;
+        sizes.lstride[sizes.count] = ls;
+        sizes.block[sizes.count] = (int)blocks;
+        samples += (long long)size_count[q] << ls;
+        blocks += (long long)size_count[q] << (ls > kSpanLog2 ? ls - kSpanLog2 : 0);
         total += size_count[q];
+        sizes.first[++sizes.count] = (int)total;
+        if (k > kmax) kmax = k;
     }
     EOBHIP_REQUIRE(total == n, "lik_evaluate: the sizes hold %lld of %d templates", total, n);
     int gx, gx2;
     int rc = eobhip_lik_partial_blocks(kmax, &gx, &gx2);
     if (rc) return rc;
     hipStream_t st = as_stream(stream);
-    for (int q = 0; q < nsizes; ++q) {
-        const int k = size_log2[q], rows = size_count[q];
-        if (rows == 0) continue;
-        // a support is at most half of M unless M is the whole segment
-        const long long stride = k < L ? 1LL << (k - 1) : 1LL << k;
-        hipLaunchKernelGGL(k_lik_resample<true>, dim3((unsigned)((stride + kSpan - 1) / kSpan), rows), dim3(kBlock), 0, st, dense, coef,
-                           num_steps, amp, dT_M, nsamp, mlog2, nullptr, order, stride, max_step, g, hbuf, cross_partial, gx);
-        if ((rc = check_launch("lik_resample"))) return rc;
-        rc = rfft_weighted_norm(hbuf, stride, work, rows, k, nsamp, order, bank + bank_offset(k, m_min_log2), hh_partial, gx2, st);
+    hipLaunchKernelGGL(k_lik_resample<true>, dim3((unsigned)blocks), dim3(kBlock), 0, st, dense, coef, num_steps, amp,
+                       dT_M, nsamp, mlog2, nullptr, sizes, max_step, g, hbuf, cross_partial, gx);
+    if ((rc = check_launch("lik_resample"))) return rc;
+    for (int q = 0; q < sizes.count; ++q) {
+        const int k = logs[q], rows = sizes.first[q + 1] - sizes.first[q];
+        rc = rfft_weighted_norm(hbuf + sizes.offset[q], 1LL << sizes.lstride[q], work, rows, k, nsamp, order + sizes.first[q],
+                                bank + bank_offset(k, m_min_log2), hh_partial, gx2, st);
         if (rc) return rc;
-        hbuf += stride * rows;
         work += (2LL << (k - 1)) * rows;
-        order += rows;
     }
     hipLaunchKernelGGL(k_lik_final, dim3(n), dim3(64), 0, st, cross_partial, gx, hh_partial, gx2, nsamp, mlog2, dd, df, n, logl, terms);
     return check_launch("lik_final");
