@@ -605,9 +605,10 @@ template <class Ptr>
 __device__ __forceinline__ void imr_inspiral_sample(Ptr row, Ptr rpr, const Piece& p, int nm, const ModeOrder& mo, const double* nq,
                                                     double& re_out, double& im_out) {
     const double om = p.d(row + 4 * (2 * nm)), r = p.v(rpr), pr = p.v(rpr + 4);
-    const double irO = 1.0 / (r * om);
-    const double p1 = pr * irO, p3 = pr * pr * p1, P = p1 * p1;
-    const double ir = om * irO, irs = ir * rsqrt(r);
+    // each rounded once: the NQC coefficients come from nearly singular solves and
+    // cancel in the sums below by up to eight digits
+    const double rO = r * om, ir = 1.0 / r, irs = 1.0 / (r * sqrt(r));
+    const double p1 = pr / rO, p3 = pr * pr * pr / rO, P = p1 * p1;
     double sp, cph, hr = 0.0, hi = 0.0;
     sincos_phase(p.v(row + 4 * (2 * nm)), &sp, &cph);
     const auto turn = [&](int k) {
@@ -672,11 +673,12 @@ __global__ __launch_bounds__(kImrBlock) void k_imr_ringdown(const int* __restric
 
 // grid (blocks, binaries), runs of samples per wavefront (resample.hpp).  512
 // binaries x 2^20 samples at 16384 Hz, five modes, 32% of them inspiral: 6100 us
-// with knot windows per block, four divisions, a square root and ten complex
-// products a sample, 3055 now.  The arithmetic alone is 1540 (330 instructions a
-// sample at the FP64 rate) and the writes 1360: a binary's blocks run together, so
+// with knot windows per block and ten complex products a sample, 3350 now.  The
+// arithmetic alone is about 1750 (375 instructions a sample at the FP64 rate; with
+// one shared reciprocal for its four divisions and the root 1540 and 3055, but an
+// ulp or two off where the NQC sums cancel) and the writes 1360: a binary's blocks run together, so
 // the two hardly overlap (taking the binaries in turn instead scatters the writes
-// and costs 3700).  Three wavefronts a SIMD; four (spills) or two samples at once
+// and costs a fifth more).  Three wavefronts a SIMD; four (spills) or two samples at once
 // (two wavefronts) are no faster.
 // kModes: the most modes the staged rows have room for.
 template <int kModes>

@@ -147,7 +147,7 @@ struct StagedRows {
 // in two steps at its start; its rows then wait for no load.  Interval by interval
 // through the scalar cache, with gathers where a row passes a knot, the waits
 // (about 1 us each, four a row) were the time: 1024 templates' h+ for the likelihood
-// 880 us, 735 this way; the five modes with NQC factors of 512 binaries 3560, 3055.
+// 880 us, 735 this way; the five modes with NQC factors of 512 binaries 3560, 3060.
 template <int R, class Time, class Stage, class Near, class Far, class Put>
 __device__ __forceinline__ void resample_rows(const double* __restrict__ T, int len, long long j0, long long jend, const Time& time,
                                               const Stage& stage, const Near& near, const Far& far, const Put& put) {

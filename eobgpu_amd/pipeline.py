@@ -1142,7 +1142,7 @@ class GraphPass:
 
     def capture(self):
         """Record the pass (after one eager pass on the same stream, which creates
-        the transform plans the pass uses)."""
+        the transform plans the pass uses, if its N needs any)."""
         self.run_eager()
         torch.cuda.synchronize(self.device)
         g = torch.cuda.CUDAGraph()

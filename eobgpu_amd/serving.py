@@ -251,8 +251,9 @@ class Server:
         return sum(p.capacity * p.bytes_per_binary() for p in self.pools)
 
     def warm(self):
-        """Create the FFT plans of every row-chunk size on every stream (plan
-        creation allocates device memory, which is kept out of the served path)."""
+        """One transform of every row-chunk size on every stream: for an N outside
+        the library's own kernels (2^10 .. 2^21) that creates the plans (plan creation
+        allocates device memory, which is kept out of the served path)."""
         rows = 2 * 64 - 1      # 64 + 32 + 16 + 8 + 4 + 2 + 1
         h = torch.zeros((rows, self.N), dtype=torch.float64, device=self.device)
         ht = torch.empty((rows, self.N // 2 + 1), dtype=torch.complex128, device=self.device)
