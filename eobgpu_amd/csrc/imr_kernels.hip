@@ -579,16 +579,17 @@ __global__ __launch_bounds__(64) void k_imr_params(BinInputs in, const double* _
 
 // sin and cos of x: Taylor series through x^9 / x^10 when every active lane of
 // the wavefront has |x| < 1/16 (first omitted terms below 2.3e-20 relative),
-// sincos_phase otherwise.  The NQC phase of the inspiral samples is small except near the
+// sincos_of otherwise.  The NQC phase of the inspiral samples is small except near the
 // attachment.
-__device__ __forceinline__ void sincos_nqc(double x, double* s, double* c) {
+template <SamplePath P>
+__device__ __forceinline__ bool sincos_nqc(double x, double* s, double* c) {
     if (__all(fabs(x) < 0.0625)) {
         const double x2 = x * x;
         *s = x * (1.0 + x2 * (-1.0 / 6 + x2 * (1.0 / 120 + x2 * (-1.0 / 5040 + x2 * (1.0 / 362880)))));
         *c = 1.0 + x2 * (-0.5 + x2 * (1.0 / 24 + x2 * (-1.0 / 720 + x2 * (1.0 / 40320 + x2 * (-1.0 / 3628800)))));
-    } else {
-        sincos_phase(x, s, c);
+        return true;
     }
+    return sincos_of<P>(x, *s, *c);
 }
 
 // ------------------------------------------------------- the IMR template
@@ -601,8 +602,8 @@ constexpr int kImrBlock = 256;
 // the binary's NQC coefficients (5 per mode).  sum_m h_m e^{-i m phi} by Horner's
 // rule in e^{-i phi} over the modes by falling m (mo): each mode then costs the
 // products between its m and the next one's, not m - 1 of its own.
-template <class Ptr>
-__device__ __forceinline__ void imr_inspiral_sample(Ptr row, Ptr rpr, const Piece& p, int nm, const ModeOrder& mo, const double* nq,
+template <SamplePath kPath, class Ptr>
+__device__ __forceinline__ bool imr_inspiral_sample(Ptr row, Ptr rpr, const Piece& p, int nm, const ModeOrder& mo, const double* nq,
                                                     double& re_out, double& im_out) {
     const double om = p.d(row + 4 * (2 * nm)), r = p.v(rpr), pr = p.v(rpr + 4);
     // each rounded once: the NQC coefficients come from nearly singular solves and
@@ -610,7 +611,7 @@ __device__ __forceinline__ void imr_inspiral_sample(Ptr row, Ptr rpr, const Piec
     const double rO = r * om, ir = 1.0 / r, irs = 1.0 / (r * sqrt(r));
     const double p1 = pr / rO, p3 = pr * pr * pr / rO, P = p1 * p1;
     double sp, cph, hr = 0.0, hi = 0.0;
-    sincos_phase(p.v(row + 4 * (2 * nm)), &sp, &cph);
+    bool good = sincos_of<kPath>(p.v(row + 4 * (2 * nm)), sp, cph);
     const auto turn = [&](int k) {
         for (; k > 0; --k) {
             const double t = hr * cph + hi * sp;
@@ -624,7 +625,7 @@ __device__ __forceinline__ void imr_inspiral_sample(Ptr row, Ptr rpr, const Piec
         const Ptr rq = row + 4 * q, iq = row + 4 * (nm + q);
         const double* c = nq + 5 * q;
         double sn, cn;
-        sincos_nqc(c[3] * p1 + p3 * c[4], &sn, &cn);
+        good &= sincos_nqc<kPath>(c[3] * p1 + p3 * c[4], &sn, &cn);
         turn(mo.down(k));
         const double mag = 1.0 + P * (c[0] + c[1] * ir + c[2] * irs);
         const double re = p.v(rq), im = p.v(iq), fr = mag * cn, fi = mag * sn;
@@ -634,6 +635,7 @@ __device__ __forceinline__ void imr_inspiral_sample(Ptr row, Ptr rpr, const Piec
     turn(mo.down(nm));
     re_out = hr;
     im_out = hi;
+    return good;
 }
 
 // samples of a template: inspiral 0 .. idx, ringdown to idx + nadd; 0: none
@@ -723,10 +725,10 @@ __global__ __launch_bounds__(kImrBlock) void k_imr_resample(const double* __rest
                     }
                 },
                 [&](int k, double x, double& re, double& im) {
-                    imr_inspiral_sample(st.modes.c + k * cs, st.rp.c + 8 * k, Piece::at(x, false), nm, mo, st.nq, re, im);
+                    return imr_inspiral_sample<kNear>(st.modes.c + k * cs, st.rp.c + 8 * k, Piece::at(x, false), nm, mo, st.nq, re, im);
                 },
                 [&](int i, double x, double& re, double& im) {
-                    imr_inspiral_sample(C + (size_t)cs * i, RP + (size_t)8 * i, Piece::at(x, i == len - 1), nm, mo, st.nq, re, im);
+                    return imr_inspiral_sample<kFar>(C + (size_t)cs * i, RP + (size_t)8 * i, Piece::at(x, i == len - 1), nm, mo, st.nq, re, im);
                 },
                 [&](long long j, const double (&re)[2], const double (&im)[2], bool full) { o.put(j, re, im, full); });
         o.zeros(j0);

@@ -17,46 +17,6 @@ constexpr int kRow = 128;                 // samples per wavefront and step
 constexpr int kRunRows = 4;               // rows of a run
 constexpr int kRun = kRow * kRunRows;     // samples per run
 
-// sin and cos of x: x - n pi/2 in two fused steps (each exact but for its last
-// rounding: their terms cancel to below 1), the Taylor series through r^17 and
-// r^16 on |r| <= pi/4 (first omitted terms below 2e-18), and the quadrant.  Within
-// 1e-16 absolute for |x| < 2^50 (phases here are 10 to 10^5 rad, their own rounding
-// 1e-15 to 1e-11); larger x, of which a double no longer resolves the radian, are
-// taken down by the same step first and stay bounded.  About 40 instructions
-// against the library's 75, and 20 registers less for the kernel.
-__device__ __forceinline__ void sincos_phase(double x, double* s, double* c) {
-    constexpr double kTwoOverPi = 0x1.45f306dc9c883p-1, kPio2Hi = 0x1.921fb54442d18p+0, kPio2Lo = 0x1.1a62633145c07p-54;
-    double quad = 0.0;
-    for (int it = 0; it < 24 && __any(!(fabs(x) < 0x1p45)); ++it) {
-        const double n = rint(x * kTwoOverPi);
-        x = fma(-n, kPio2Lo, fma(-n, kPio2Hi, x));
-        quad += fma(-4.0, floor(0.25 * n), n);
-    }
-    const double n = rint(x * kTwoOverPi);
-    const double r = fma(-n, kPio2Lo, fma(-n, kPio2Hi, x));
-    const double z = r * r;
-    double p = fma(z, 1.0 / 355687428096000.0, -1.0 / 1307674368000.0);
-    p = fma(p, z, 1.0 / 6227020800.0);
-    p = fma(p, z, -1.0 / 39916800.0);
-    p = fma(p, z, 1.0 / 362880.0);
-    p = fma(p, z, -1.0 / 5040.0);
-    p = fma(p, z, 1.0 / 120.0);
-    p = fma(p, z, -1.0 / 6.0);
-    const double sr = fma(r * z, p, r);
-    double q = fma(z, 1.0 / 20922789888000.0, -1.0 / 87178291200.0);
-    q = fma(q, z, 1.0 / 479001600.0);
-    q = fma(q, z, -1.0 / 3628800.0);
-    q = fma(q, z, 1.0 / 40320.0);
-    q = fma(q, z, -1.0 / 720.0);
-    q = fma(q, z, 1.0 / 24.0);
-    q = fma(q, z, -0.5);
-    const double cr = fma(q, z, 1.0);
-    const int k = (int)(fma(-4.0, floor(0.25 * n), n) + quad);
-    const double a = (k & 1) ? cr : sr, b = (k & 1) ? sr : cr;
-    *s = (k & 2) ? -a : a;
-    *c = ((k + 1) & 2) ? -b : b;
-}
-
 // searchsorted(T, t, 'right') - 1, at least 0, for a wavefront-uniform t: 64
 // knots are compared at once.  T: knot times at stride 5, sorted, len >= 1.
 __device__ __forceinline__ int wave_interval(const double* __restrict__ T, int len, double t) {
@@ -93,18 +53,32 @@ typedef const __attribute__((address_space(4))) double* ConstPtr;
 typedef double SamplePair __attribute__((ext_vector_type(2), aligned(8)));
 
 // A lane's two samples in turn, f(i, x, re, im) each: at once they would double the
-// registers of the whole kernel.
+// registers of the whole kernel.  Whether f was true for both.
 template <class F>
-__device__ __forceinline__ void one_by_one(double xa, double xb, int ia, int ib, double (&re)[2], double (&im)[2], const F& f) {
+__device__ __forceinline__ bool one_by_one(double xa, double xb, int ia, int ib, double (&re)[2], double (&im)[2], const F& f) {
+    bool good = true;
 #pragma unroll 1
     for (int e = 0; e < 2; ++e) {
         double x, y;
-        f(e ? ib : ia, e ? xb : xa, x, y);
+        good &= f(e ? ib : ia, e ? xb : xa, x, y);
         re[0] = e ? re[0] : x;
         im[0] = e ? im[0] : y;
         re[1] = x;
         im[1] = y;
     }
+    return good;
+}
+
+// How a sample's sine and cosine are taken: kNear only for |x| < 2^49 (false for the
+// others), kFar for any.  The hot loop takes kNear alone and a row with a larger
+// phase goes the general way: with the large reduction inside the loop the
+// likelihood of 1024 templates takes 5% longer.
+enum SamplePath { kNear, kFar };
+template <SamplePath P>
+__device__ __forceinline__ bool sincos_of(double x, double& s, double& c) {
+    if constexpr (P == kNear) return eob::sincos_bounded(x, s, c);
+    eob::sincos_phase(x, s, c);
+    return true;
 }
 
 // A wavefront's LDS copy of R consecutive rows of a table, CS doubles each
@@ -140,7 +114,8 @@ struct StagedRows {
 // (j < jend; j0 < jend):
 //   time(j)                the time of sample j
 //   stage(i, n)            table rows i .. i + n - 1 (n <= R) into the wavefront's LDS
-//   near(k, x, re, im)     one sample at x past the knot of staged row k (per lane)
+//   near(k, x, re, im)     one sample at x past the knot of staged row k (per lane); false
+//                          if the row needs far
 //   far(i, x, re, im)      one sample from table row i (per lane), read from memory
 //   put(j, re, im, full)   a lane's samples j, j + 1 (full: all of the row's are below jend)
 // The run's knots (lane q holds the q-th after its first) and table rows are read
@@ -171,7 +146,7 @@ __device__ __forceinline__ void resample_rows(const double* __restrict__ T, int 
         double next = lane_value(tk, 0), last = 0.0;
         long long j = 0;
         double re[2], im[2];
-        bool covered = true;
+        bool covered = true, large = false;
         for (; r < kRunRows; ++r) {
             const long long jr = j0 + (long long)r * kRow;
             if (jr >= jend) return;
@@ -194,15 +169,17 @@ __device__ __forceinline__ void resample_rows(const double* __restrict__ T, int 
                 }
                 next = lane_value(tk, cur);
             }
-            one_by_one(ta - xa, tb - xb, ia, ib, re, im, near);
+            large = __any(!one_by_one(ta - xa, tb - xb, ia, ib, re, im, near));
+            if (large) break;
             put(j, re, im, full);
         }
-        if (covered) break;
-        if (cur > 0) {   // stage from here
+        if (covered && !large) break;
+        if (!large && cur > 0) {   // stage from here
             ind += cur;
             continue;
         }
-        // the row passes more knots than are staged: T[ind] <= every sample of it (or ind = 0)
+        // the row passes more knots than are staged, or has a phase that near leaves out: T[ind]
+        // <= every sample of it (or ind = 0)
         const double ta = time(j), tb = time(j + 1);
         int ia = ind, ib = ind;
         for (int m = len - ind; m > 1;) {
@@ -234,16 +211,17 @@ __device__ __forceinline__ void store_pair(double* out, long long j, long long N
 
 // h22 = S e^{-2 i phi} at x past the knot of a row of the (2,2) splines (phi,
 // Re S, Im S; 4 coefficients each)
-template <class Row>
-__device__ __forceinline__ void h22_sample(const Row& c, double x, double& re, double& im) {
+template <SamplePath P, class Row>
+__device__ __forceinline__ bool h22_sample(const Row& c, double x, double& re, double& im) {
     const double x2 = x * x, x3 = x2 * x;
     const double ph = c[0] + c[1] * x + c[2] * x2 + c[3] * x3;
     const double sr = c[4] + c[5] * x + c[6] * x2 + c[7] * x3;
     const double si = c[8] + c[9] * x + c[10] * x2 + c[11] * x3;
     double sp, cp;
-    sincos_phase(2.0 * ph, &sp, &cp);
+    const bool good = sincos_of<P>(2.0 * ph, sp, cp);
     re = sr * cp + si * sp;
     im = si * cp - sr * sp;
+    return good;
 }
 
 // h22 on the run of samples t0 + j dT from j0: put(j, re[2], im[2], full)
@@ -253,8 +231,8 @@ __device__ __forceinline__ void h22_rows(H22Stage& st, const double* __restrict_
                                          long long j0, long long jend, const Put& put) {
     resample_rows<H22Stage::kRows>(
         T, len, j0, jend, [&](long long j) { return t0 + (double)j * dT; }, [&](int i, int n) { st.copy(C + (size_t)12 * i, n); },
-        [&](int k, double x, double& re, double& im) { h22_sample(st.row(k), x, re, im); },
-        [&](int i, double x, double& re, double& im) { h22_sample(C + (size_t)12 * i, x, re, im); }, put);
+        [&](int k, double x, double& re, double& im) { return h22_sample<kNear>(st.row(k), x, re, im); },
+        [&](int i, double x, double& re, double& im) { return h22_sample<kFar>(C + (size_t)12 * i, x, re, im); }, put);
 }
 
 // h+ and hx (hx may be null) of N samples, zero from nb on

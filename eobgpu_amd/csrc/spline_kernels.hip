@@ -636,12 +636,12 @@ constexpr int kMaxModeM = 8;
 // One sample's sum from a row (Re of each mode, Im of each mode, phi; 4
 // coefficients per series), by Horner's rule in e^{-i phi} over the modes by
 // falling m: a mode costs the products between its m and the next one's.
-template <class Ptr>
-__device__ __forceinline__ void modes_sample(Ptr c, double x, int nm, const ModeOrder& mo, double& hr, double& hi) {
+template <SamplePath P, class Ptr>
+__device__ __forceinline__ bool modes_sample(Ptr c, double x, int nm, const ModeOrder& mo, double& hr, double& hi) {
     const double x2 = x * x, x3 = x2 * x;
     const auto cubic = [&](Ptr p) { return p[0] + p[1] * x + p[2] * x2 + p[3] * x3; };
     double sp, cph;
-    sincos_phase(cubic(c + 4 * (2 * nm)), &sp, &cph);
+    const bool good = sincos_of<P>(cubic(c + 4 * (2 * nm)), sp, cph);
     double r = 0.0, i = 0.0;
     const auto turn = [&](int k) {
         for (; k > 0; --k) {
@@ -660,6 +660,7 @@ __device__ __forceinline__ void modes_sample(Ptr c, double x, int nm, const Mode
     turn(mo.down(nm));
     hr = r;
     hi = i;
+    return good;
 }
 
 // kModes: the most modes the staged rows have room for.  Five modes of 512 binaries
@@ -687,8 +688,8 @@ __global__ __launch_bounds__(kBlock) void k_resample_modes(const double* __restr
         if (j0 < nb)
             resample_rows<Stage::kRows>(
                 T, len, j0, nb, [&](long long j) { return t0 + (double)j * dT; }, [&](int i, int n) { st.copy(C + (size_t)cs * i, n, cs); },
-                [&](int k, double x, double& re, double& im) { modes_sample(st.c + k * cs, x, nm, mo, re, im); },
-                [&](int i, double x, double& re, double& im) { modes_sample(C + (size_t)cs * i, x, nm, mo, re, im); },
+                [&](int k, double x, double& re, double& im) { return modes_sample<kNear>(st.c + k * cs, x, nm, mo, re, im); },
+                [&](int i, double x, double& re, double& im) { return modes_sample<kFar>(C + (size_t)cs * i, x, nm, mo, re, im); },
                 [&](long long j, const double (&re)[2], const double (&im)[2], bool full) { o.put(j, re, im, full); });
         o.zeros(j0);
     });
