@@ -463,6 +463,15 @@ IMR_HD LeaverRad leaver_radial(Cx w, double a, int s, int m, Cx A) {
     return f;
 }
 
+// t_0 of the radial fraction from t_n, a division per term
+IMR_HD Cx leaver_radial_down(const LeaverRad& f, Cx t, int n) {
+    auto alpha = [&](int n) { const double d = n; return cx(d * d + d) + (f.c0 * d) + f.c0; };
+    auto beta = [&](int n) { const double d = n; return cx(-2.0 * d * d + 2.0 * d) + (f.c1 * d) + f.c3; };
+    auto gamma = [&](int n) { const double d = n; return cx(d * d - 3.0 * d + 2.0) + (f.c2 * d) + f.c4 - f.c2; };
+    for (--n; n >= 0; --n) t = beta(n) - alpha(n) * gamma(n + 1) / t;
+    return t;
+}
+
 // The fractions from their last term back, a division per term
 struct LeaverSerial {
     IMR_HD static Cx fraction(const LeaverAng& f) {
@@ -471,12 +480,8 @@ struct LeaverSerial {
         return t;
     }
     IMR_HD static Cx fraction(const LeaverRad& f) {
-        auto alpha = [&](int n) { const double d = n; return cx(d * d + d) + (f.c0 * d) + f.c0; };
-        auto beta = [&](int n) { const double d = n; return cx(-2.0 * d * d + 2.0 * d) + (f.c1 * d) + f.c3; };
-        auto gamma = [&](int n) { const double d = n; return cx(d * d - 3.0 * d + 2.0) + (f.c2 * d) + f.c4 - f.c2; };
-        Cx t = beta(kLeaverRadDepth);
-        for (int n = kLeaverRadDepth - 1; n >= 0; --n) t = beta(n) - alpha(n) * gamma(n + 1) / t;
-        return t;
+        const double d = kLeaverRadDepth;
+        return leaver_radial_down(f, cx(-2.0 * d * d + 2.0 * d) + (f.c1 * d) + f.c3, kLeaverRadDepth);
     }
 };
 
@@ -511,6 +516,7 @@ IMR_HD Cx leaver_radial_cf(Cx w, double a, int s, int m, Cx* A) {
 // with the separation constant followed from A: secant steps from w.
 struct QnmRoot {
     Cx w, A;
+    Cx slope;   // dw / df of the last step that was well above rounding
 };
 template <class Cf>
 IMR_HD QnmRoot leaver_refine(int m, double a, Cx w, Cx A, double dw) {
@@ -518,10 +524,11 @@ IMR_HD QnmRoot leaver_refine(int m, double a, Cx w, Cx A, double dw) {
     Cx x0 = w, x1 = w + cx(dw, -dw);
     Cx A0 = A, A1 = A;
     Cx f0 = leaver_radial_cf<Cf>(x0, a, s, m, &A0);
-    Cx f1 = leaver_radial_cf<Cf>(x1, a, s, m, &A1);
+    Cx f1 = leaver_radial_cf<Cf>(x1, a, s, m, &A1), slope = cx(0.0);
     for (int it = 0; it < 50; ++it) {
         const Cx d = f1 - f0;
         if (cabs2(d) == 0.0) break;
+        if (cabs2(x1 - x0) > 1e-20) slope = (x1 - x0) / d;
         const Cx x2 = x1 - f1 * (x1 - x0) / d;
         x0 = x1;
         f0 = f1;
@@ -530,7 +537,7 @@ IMR_HD QnmRoot leaver_refine(int m, double a, Cx w, Cx A, double dw) {
         f1 = leaver_radial_cf<Cf>(x1, a, s, m, &A1);
         if (cabs2(x1 - x0) < 1e-30 * (1.0 + cabs2(x1))) break;
     }
-    return QnmRoot{x1, A1};
+    return QnmRoot{x1, A1, slope};
 }
 
 // The fundamental (l, m) root at spin af (units of M, |af| <= 0.9999) followed
