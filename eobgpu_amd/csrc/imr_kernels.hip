@@ -20,6 +20,7 @@
 #include <hip/hip_runtime.h>
 
 #include <mutex>
+#include <type_traits>
 
 #include "eobhip_common.hpp"
 #include "imr.hpp"
@@ -319,11 +320,10 @@ struct LeaverLanes {
 
 constexpr int kLowTerms = 40;
 
-// M omega_lm0 at spin af, by the kQnmLanes lanes of a group: from the table for the
-// ringdown modes, |af| <= 0.99; otherwise along the spin path from a = 0
-__device__ Cx kerr_qnm_fast(int l, int m, double af) {
-    const int k = imr::rd_mode_index(l, m);
-    if (k < 0 || !(fabs(af) <= 0.99)) return imr::kerr_qnm(l, m, af);
+// M omega_lm0 at spin |af| <= 0.99 of a ringdown mode, from the table's guess; Cf
+// LeaverLanes: by the kQnmLanes lanes of a group
+template <class Cf>
+__device__ Cx kerr_qnm_table(int k, int m, double af) {
     const double x = (af - kQnmA0) / kQnmDa;
     int i = (int)floor(x);
     i = i < 0 ? 0 : (i > kQnmGrid - 2 ? kQnmGrid - 2 : i);
@@ -332,23 +332,55 @@ __device__ Cx kerr_qnm_fast(int l, int m, double af) {
     const double* p1 = g_qnm_tab[k][i + 1];
     const Cx w = imr::cx((1.0 - f) * p0[0] + f * p1[0], (1.0 - f) * p0[1] + f * p1[1]);
     const Cx A = imr::cx((1.0 - f) * p0[2] + f * p1[2], (1.0 - f) * p0[3] + f * p1[3]);
-    imr::QnmRoot r = imr::leaver_refine<LeaverLanes>(m, 0.5 * af, w, A, 1e-6);
-    if (fabs(af) >= 0.8) {
-        const double a = 0.5 * af;
-        const int steps = fabs(af) < 0.97 ? 2 : 4;
-        Cx sum = imr::cx(0.0);
+    imr::QnmRoot r = imr::leaver_refine<Cf>(m, 0.5 * af, w, A, 1e-6);
+    if constexpr (std::is_same_v<Cf, LeaverLanes>) {
+        if (fabs(af) >= 0.8) {
+            const double a = 0.5 * af;
+            const int steps = fabs(af) < 0.97 ? 2 : 4;
+            Cx sum = imr::cx(0.0);
 #pragma unroll 1
-        for (int k = 0; k < steps; ++k) {
-            if (k) r.A = imr::leaver_angular_solve<LeaverLanes>(r.A, a * r.w, -2, m);
-            const imr::LeaverRad f = imr::leaver_radial(r.w, a, -2, m, r.A);
-            const Cx t = LeaverLanes::radial_from<kLowTerms>(f) - (double)(kLowTerms * kLowTerms);
-            r.w = r.w - r.slope * imr::leaver_radial_down(f, t, kLowTerms);
-            sum = sum + r.w;
+            for (int k = 0; k < steps; ++k) {
+                if (k) r.A = imr::leaver_angular_solve<LeaverLanes>(r.A, a * r.w, -2, m);
+                const imr::LeaverRad f = imr::leaver_radial(r.w, a, -2, m, r.A);
+                const Cx t = LeaverLanes::radial_from<kLowTerms>(f) - (double)(kLowTerms * kLowTerms);
+                r.w = r.w - r.slope * imr::leaver_radial_down(f, t, kLowTerms);
+                sum = sum + r.w;
+            }
+            r.w = (1.0 / steps) * sum;
         }
-        r.w = (1.0 / steps) * sum;
     }
     return imr::cx(0.5 * r.w.re, 0.5 * r.w.im);
 }
+
+// How a launch of blocks of 64 threads shares n roots: in its first `groups` blocks a
+// group of kQnmLanes lanes per root that the table serves, in the others a lane per
+// root for what is left: roots without a table (the spin path from a = 0, where a
+// group's lanes would all walk the same path) and, with no groups, all.  Up to
+// kQnmGrouped roots the groups are faster, since a root's chain is the time: (2,2),
+// 4096 roots 118 us by groups and 785 by lanes, 65536 926 and 771, 262144 3444 and 2036.
+// Without a table, 65536 roots 16.5 ms a lane each and 101 by groups.
+constexpr long long kQnmGrouped = 49152;
+struct QnmSplit {
+    unsigned groups;
+    static QnmSplit of(long long n, bool table) { return QnmSplit{table && n <= kQnmGrouped ? blocks_for(n, 64 / kQnmLanes) : 0u}; }
+    unsigned blocks(long long n) const { return groups + blocks_for(n, 64); }
+    __device__ __forceinline__ bool grouped() const { return blockIdx.x < groups; }
+    __device__ __forceinline__ long long root() const {
+        return grouped() ? ((long long)blockIdx.x * 64 + threadIdx.x) / kQnmLanes : (long long)(blockIdx.x - groups) * 64 + threadIdx.x;
+    }
+    // M omega_lm0 at spin af; true on the one lane that has it
+    __device__ __forceinline__ bool omega(int l, int m, double af, Cx& w) const {
+        const int k = imr::rd_mode_index(l, m);
+        const bool table = k >= 0 && fabs(af) <= 0.99;
+        if (grouped()) {
+            if (table) w = kerr_qnm_table<LeaverLanes>(k, m, af);
+            return table && threadIdx.x % kQnmLanes == 0;
+        }
+        if (table && groups) return false;
+        w = table ? kerr_qnm_table<imr::LeaverSerial>(k, m, af) : imr::kerr_qnm(l, m, af);
+        return true;
+    }
+};
 
 // fill the table on the current device once (stream-ordered, then waited for,
 // so that launches on any stream see it)
@@ -370,13 +402,13 @@ int ensure_qnm_table(void* stream) {
 }
 
 // ------------------------------------------------------------ QNMs per binary
-// Lanes (b, j) of a group: j < nm the QNM of mode j, j == nm the (2,2) QNM that sets the
+// Root (b, j): j < nm the QNM of mode j, j == nm the (2,2) QNM that sets the
 // ringdown length (the reference's 30 damping times, :2463-2465 and :2514).
 // wl [n][nm] complex in lalsimulation's convention (omega_r + i / tau) in
 // units of the total mass; binf/bini as the enums.
 __global__ void k_imr_qnm(BinInputs in, const double* __restrict__ dense, const double* __restrict__ dT_M, int n, int max_step,
-                          ImrModes mm, double* __restrict__ wl, double* __restrict__ binf, int* __restrict__ bini) {
-    const long long gid = ((long long)blockIdx.x * blockDim.x + threadIdx.x) / kQnmLanes;
+                          ImrModes mm, QnmSplit split, double* __restrict__ wl, double* __restrict__ binf, int* __restrict__ bini) {
+    const long long gid = split.root();
     const int per = mm.nm + 1;
     if (gid >= (long long)n * per) return;
     const int b = (int)(gid / per), j = (int)(gid % per);
@@ -385,8 +417,8 @@ __global__ void k_imr_qnm(BinInputs in, const double* __restrict__ dense, const 
     const double mf = imr::final_mass_seobnrv4(m1 / M, m2 / M, c1, c2);
     const double af = imr::final_spin_hbr2016(m1 / M, m2 / M, c1, c2);
     const int l = (j < mm.nm) ? mm.l[j] : 2, m = (j < mm.nm) ? mm.m[j] : 2;
-    const Cx w = kerr_qnm_fast(l, m, af);
-    if (threadIdx.x % kQnmLanes != 0) return;
+    Cx w;
+    if (!split.omega(l, m, af, w)) return;
     const double wr = w.re / mf, wi = -w.im / mf;   // conj(omega) / M_f
     if (j < mm.nm) {
         wl[2 * ((size_t)b * mm.nm + j)] = wr;
@@ -789,11 +821,11 @@ __global__ void k_imr_fit(int which, int l, int m, const double* __restrict__ x1
     out[i] = v;
 }
 
-__global__ void k_kerr_qnm(int l, int m, const double* __restrict__ af, int n, double* __restrict__ out) {
-    const long long i = ((long long)blockIdx.x * blockDim.x + threadIdx.x) / kQnmLanes;
+__global__ void k_kerr_qnm(int l, int m, const double* __restrict__ af, int n, QnmSplit split, double* __restrict__ out) {
+    const long long i = split.root();
     if (i >= n) return;
-    const Cx w = kerr_qnm_fast(l, m, af[i]);
-    if (threadIdx.x % kQnmLanes != 0) return;
+    Cx w;
+    if (!split.omega(l, m, af[i], w)) return;
     out[2 * i] = w.re;
     out[2 * i + 1] = w.im;
 }
@@ -827,7 +859,8 @@ int eobhip_kerr_qnm(int l, int m, const double* af, int n, double* omega, void* 
     if (n == 0) return EOBHIP_OK;
     const int rc = ensure_qnm_table(stream);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_kerr_qnm, dim3(blocks_for(n, 64 / kQnmLanes)), dim3(64), 0, as_stream(stream), l, m, af, n, omega);
+    const QnmSplit split = QnmSplit::of(n, imr::rd_mode_index(l, m) >= 0);
+    hipLaunchKernelGGL(k_kerr_qnm, dim3(split.blocks(n)), dim3(64), 0, as_stream(stream), l, m, af, n, split, omega);
     return check_launch("kerr_qnm");
 }
 
@@ -843,8 +876,8 @@ int eobhip_imr_params(const double* m1, const double* m2, const double* chi1, co
     if (rc) return rc;
     const BinInputs in{m1, m2, chi1, chi2};
     const long long nq = (long long)n * (nm + 1);
-    hipLaunchKernelGGL(k_imr_qnm, dim3(blocks_for(nq, 64 / kQnmLanes)), dim3(64), 0, as_stream(stream), in, dense, dT_M, n, max_step, mm, qnm, binf,
-                       bini);
+    const QnmSplit split = QnmSplit::of(nq, true);
+    hipLaunchKernelGGL(k_imr_qnm, dim3(split.blocks(nq)), dim3(64), 0, as_stream(stream), in, dense, dT_M, n, max_step, mm, split, qnm, binf, bini);
     rc = check_launch("imr_qnm");
     if (rc) return rc;
     EOBHIP_REQUIRE((long long)n * nm < (1LL << 31), "too many (binary, mode) pairs");
