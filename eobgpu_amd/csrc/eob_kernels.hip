@@ -168,12 +168,18 @@ struct DropLds {
     double lead[kNumModes][kDropMax], newton[kNumModes][kDropMax];
 };
 
+// Batches from these sizes on take a lane per system (k_*_lanes), which fill the chip
+// by themselves and have no wavefronts waiting through H.  Blocks and lanes, us: one
+// right-hand side of 32768 systems 108 and 115, 49152 156 and 126, 262144 723 and 483;
+// the scalar root of 32768 356 and 421, 49152 536 and 477, 262144 2649 and 2034; a
+// step's twelve stages of 49152 1349 and 1530, 65536 1791 and 1691, 262144 7116 and 5962.
+constexpr int kRhsLanes = 36864, kRootLanes = 43008, kStepLanes = 59392;
+
 // systems per block: few while that spreads the batch over the chip's 256 CUs
 // (never fewer than 4: their 140 (system, mode) pairs are one round of the
 // block), at most a lane each.  One attempted step through the three drop-ins,
 // lane per system before and blocks now: 16 systems 820 and 249 us, 2048 1060
-// and 281, 16384 1140 and 526; past one chip of lanes a lane per system catches
-// up (65536: 1770 and 1860).
+// and 281, 16384 1140 and 526.
 inline int drop_systems(int n) {
     int s = 4;
     while (s < kDropMax && (long long)s * 256 < n) s *= 2;
@@ -264,6 +270,24 @@ __device__ __forceinline__ void block_rhs(DropLds& lds, double nu, const ModeCoe
         k[1] = omega;
         k[2] = fma(-pr / L, f_over_om, -lds.pass[kPassR][s]);
         k[3] = -0.0 + -f_over_om;
+    }
+}
+
+// one system per lane
+__global__ __launch_bounds__(kBlock) void k_ode_dropin_lanes(const double* arg, double* k, const double* add, int n, const ModeCoef* modes,
+                                                             const int* idx) {
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+        const HamCoef c = ham_from_add(add, n, i);
+        const double r = arg[i], pr = arg[2 * n + i], L = arg[3 * n + i];
+        const Dual d0 = ham_tangent(c, r, pr, L, 0);
+        const double dHdpr = ham_tangent(c, r, pr, L, 1).d;
+        const double dHdL = ham_tangent(c, r, pr, L, 2).d;
+        double F[2];
+        rr_force_dropin(modes + (size_t)idx[i] * kNumModes, add, n, i, c, r, pr, L, dHdL, F);
+        k[i] = dHdpr;
+        k[n + i] = dHdL;
+        k[2 * n + i] = -d0.d + F[0];
+        k[3 * n + i] = -0.0 + F[1];
     }
 }
 
@@ -474,6 +498,29 @@ __global__ __launch_bounds__(64 * kIcWaves) void k_root_find_scalar_all(double* 
     if (mine) pr_res[i] = cc;
 }
 
+// one binary per lane
+__global__ __launch_bounds__(kBlock) void k_root_find_scalar_lanes(double* pr_res, const double* bounds, const double* args,
+                                                                   const double* add, int max_iter, double err, int n,
+                                                                   const ModeCoef* modes) {
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+        const HamCoef c = ham_from_add(add, n, i);
+        const ModeCoef* hm = modes + (size_t)i * kNumModes;
+        const double r = args[i], L = args[3 * n + i];
+        double a = bounds[i], b = bounds[n + i], g[4], F[2];
+        double fa = ic_diss_dev(hm, add, n, i, c, r, a, L, g, F);
+        double fb = ic_diss_dev(hm, add, n, i, c, r, b, L, g, F);
+        double cc = 0.0;
+        for (int it = 0; it < max_iter; ++it) {
+            cc = (a * fb - b * fa) / (fb - fa);
+            const double fc = ic_diss_dev(hm, add, n, i, c, r, cc, L, g, F);
+            if ((fb < 0.0 && fc < 0.0) || (fb >= 0.0 && fc >= 0.0)) { b = cc; fb = fc; }
+            else { a = cc; fa = fc; }
+            if (fabs(fc) < err) break;
+        }
+        pr_res[i] = cc;
+    }
+}
+
 __global__ __launch_bounds__(kBlock) void k_update_info(ModeCoef* modes, WaveCoef* wave, const double* m1, const double* m2,
                                                         const double* eta, const double* a, const double* chiS, const double* chiA,
                                                         int use_hm, int n) {
@@ -529,6 +576,24 @@ struct StagePtrs {
     double* k[12];   // where stage s leaves its k; later stages read it there
 };
 __constant__ double dA[12][12] = DOP_A;
+// a stage's arguments, one system per lane
+__global__ __launch_bounds__(kBlock) void k_stage_arg(double* arg, const double* solOld, const double* x, double* xCur, double* ak,
+                                                      const double* h, StagePtrs kp, int stage, int n) {
+    for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < n; e += gridDim.x * blockDim.x) {
+        const double hh = h[e];
+        xCur[e] = x[e] + dC[stage] * hh;
+        for (int j = 0; j < 4; ++j) {
+            double acc = 0.0;
+            for (int q = 0; q < stage; ++q) {
+                const double a = dA[stage][q];
+                if (a != 0.0) acc += a * kp.k[q][(size_t)j * n + e];
+            }
+            ak[(size_t)j * n + e] = acc;
+            arg[(size_t)j * n + e] = solOld[(size_t)j * n + e] + hh * acc;
+        }
+    }
+}
+
 // All twelve stages of one attempted step for S systems per block: lane (s, j) of
 // the first wavefronts forms component j's argument, then block_rhs.  With two
 // launches per stage and a lane per system the 24 launches took 720 us for 16
@@ -1543,6 +1608,11 @@ int eobhip_seobnr_root_find_scalar_all(eobhip_seobnr_t h, double* pr_res, const 
     EOBHIP_REQUIRE(num_args == 4 && num_add_args == kNAdd, "root_find_scalar_all: 4 args and 80 additional args per binary");
     EOBHIP_REQUIRE(numBinAll >= 0 && numBinAll <= h->numSys && max_iter >= 0, "bad sizes");
     if (numBinAll == 0) return EOBHIP_OK;
+    if (numBinAll >= kRootLanes) {
+        hipLaunchKernelGGL(k_root_find_scalar_lanes, dim3(blocks_for(numBinAll, kBlock)), dim3(kBlock), 0, as_stream(stream), pr_res,
+                           start_bounds, argsIn, add, max_iter, err, numBinAll, h->modes);
+        return check_launch("root_find_scalar_all");
+    }
     const int S = drop_systems(numBinAll);
     hipLaunchKernelGGL(k_root_find_scalar_all, dim3(blocks_for(numBinAll, S)), dim3(64 * kIcWaves), 0, as_stream(stream), pr_res,
                        start_bounds, argsIn, add, max_iter, err, numBinAll, h->modes, S);
@@ -1554,6 +1624,11 @@ int eobhip_seobnr_ODE_Ham_align_AD(eobhip_seobnr_t h, const double* x, const dou
     (void)x;
     EOBHIP_REQUIRE(h && h->allocated, "ODE_Ham_align_AD: update_information has not been called");
     if (numSys == 0) return EOBHIP_OK;
+    if (numSys >= kRhsLanes) {
+        hipLaunchKernelGGL(k_ode_dropin_lanes, dim3(blocks_for(numSys, kBlock)), dim3(kBlock), 0, as_stream(stream), arg, k, add, numSys,
+                           h->modes, idx);
+        return check_launch("ODE_Ham_align_AD");
+    }
     const int S = drop_systems(numSys);
     hipLaunchKernelGGL(k_ode_dropin, dim3(blocks_for(numSys, S)), dim3(64 * kOdeWaves), 0, as_stream(stream), arg, k, add, numSys, h->modes,
                        idx, S);
@@ -1591,6 +1666,18 @@ int eobhip_dormandPrinceSteps(double* x, double* xCurrent, double* solOld, doubl
     // stage 12 reads stage 11 from k2 and stage 2 never enters it (a_12,2 = 0)
     StagePtrs kp;
     for (int q = 0; q < 12; ++q) kp.k[q] = outs[q];
+    if (numEq >= kStepLanes) {
+        const unsigned nb = blocks_for(numEq, kBlock);
+        for (int s = 0; s < 12; ++s) {
+            hipLaunchKernelGGL(k_stage_arg, dim3(nb), dim3(kBlock), 0, st, arg, solOld, x, xCurrent, ak, h, kp, s, numEq);
+            int rc = check_launch("stage args");
+            if (rc) return rc;
+            hipLaunchKernelGGL(k_ode_dropin_lanes, dim3(nb), dim3(kBlock), 0, st, arg, outs[s], add, numEq, ode->modes, idx);
+            rc = check_launch("stage rhs");
+            if (rc) return rc;
+        }
+        return EOBHIP_OK;
+    }
     const int S = drop_systems(numEq);
     hipLaunchKernelGGL(k_dopr_steps, dim3(blocks_for(numEq, S)), dim3(64 * kOdeWaves), 0, st, arg, solOld, x, xCurrent, ak, h, kp, numEq, add,
                        ode->modes, idx, S);
