@@ -18,6 +18,12 @@
 //                  H - k, so X follows in the block.  It reads and writes the
 //                  same index set {q A + ka}, so the output row itself is the
 //                  only intermediate and no workspace is needed.
+// A batch too small to fill the chip is bound by one block's latency: its blocks are
+// smaller (a wavefront for rows of 2^10 and 2^11, 128 threads for the two kernels,
+// which also take rows of 2^14 then).  us, with blocks of kFftThreads for every batch,
+// now, and hipFFT's plan: one row of 2^11 9.4, 6.1, 7.2, of 2^14 12.2, 9.4, 11.8, of
+// 2^15 15.0, 10.1, 12.9, of 2^18 17.9, 11.9, 16.4; 32 rows of 2^11 10.3, 6.3, 6.5; up
+// to 64 rows of 2^10 9.0, 5.8, 5.5.
 // Measured on 256 rows of 2^20 samples: 1.77 ms, the two passes at 4.85 TB/s
 // (a large copy reaches 4.97) against 4.62 ms for hipFFT's plan (three
 // transposes, two transforms and the real step); 4096 rows of 2^10: 20 us
@@ -33,7 +39,7 @@
 
 namespace eobhip_detail {
 
-constexpr int kFftThreads = 512;
+constexpr int kFftThreads = 512;   // the most
 constexpr int kFftPoints = 16 * kFftThreads;
 constexpr int kFftMinLog2 = kRfftMinLog2, kFftMaxLog2 = kRfftMaxLog2;   // N
 constexpr int kFftOneMaxLog2 = 14;   // N whose H = N/2 points fit one block
@@ -192,7 +198,7 @@ __device__ __forceinline__ void stage_bfly(double2 (&v)[16]) {
     for (int m = 0; m < 16 / R; ++m) bfly<R>(v, m);
 }
 
-// The stages of a length-2^LN transform (LN = 7 .. 13) whose points are in v
+// The stages of a length-2^LN transform (LN = 6 .. 13) whose points are in v
 // (point p + (n/16) u in slot u).  addr(pos) places a point of this thread's
 // transform in the exchange buffer; before the last stage the thread may turn
 // to point p2 of another transform of the block, placed by addr2 (the same
@@ -204,7 +210,7 @@ __device__ __forceinline__ void fft_stages(double2 (&v)[16], int p, int p2, doub
     constexpr int q16 = (1 << LN) / 16;
     constexpr int full = (LN % 4 == 0) ? LN / 4 : LN / 4 + 1;   // stages
     constexpr int RL = (LN % 4 == 0) ? 16 : (1 << (LN % 4));    // last radix
-    static_assert(full >= 2 && full <= 4, "7 <= LN <= 13");
+    static_assert(full >= 2 && full <= 4, "5 <= LN <= 13");
     bfly<16>(v, 0);
     if constexpr (full > 2) {
         lds_exchange(v, buf, [&](int u) { return addr(stage_out(p, 1, u)); }, [&](int u) { return addr(p + q16 * u); });
@@ -246,26 +252,26 @@ __device__ __forceinline__ double2 w32(int u) {
 // (or, where `self0`, with its own slot 16 - u, slots 0 and 8 with themselves).
 // Half the slots go through LDS at a time as whole complex values, so that no
 // second set of 16 is held in registers.  w0 is W_N^k of slot 0; use(u, X).
-template <class Use>
+template <int T, class Use>
 __device__ __forceinline__ void real_bins(const double2 (&v)[16], double* buf, int mate, bool self0, double2 w0, const Use& use) {
     double2* half = reinterpret_cast<double2*>(buf);   // 8 values per thread
     __syncthreads();
 #pragma unroll
-    for (int u = 8; u < 16; ++u) half[(u - 8) * kFftThreads + threadIdx.x] = v[u];
+    for (int u = 8; u < 16; ++u) half[(u - 8) * T + threadIdx.x] = v[u];
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-        double2 zp = half[((self0 && u > 0) ? 8 - u : 7 - u) * kFftThreads + mate];
+        double2 zp = half[((self0 && u > 0) ? 8 - u : 7 - u) * T + mate];
         if (u == 0) zp = make_double2(self0 ? v[0].x : zp.x, self0 ? v[0].y : zp.y);
         use(u, real_bin(v[u], zp, cmul2(w0, w32(u))));
     }
     __syncthreads();
 #pragma unroll
-    for (int u = 0; u < 8; ++u) half[u * kFftThreads + threadIdx.x] = v[u];
+    for (int u = 0; u < 8; ++u) half[u * T + threadIdx.x] = v[u];
     __syncthreads();
 #pragma unroll
     for (int u = 8; u < 16; ++u) {
-        double2 zp = half[((self0 && u > 8) ? 16 - u : 15 - u) * kFftThreads + mate];
+        double2 zp = half[((self0 && u > 8) ? 16 - u : 15 - u) * T + mate];
         if (u == 8) zp = make_double2(self0 ? v[8].x : zp.x, self0 ? v[8].y : zp.y);
         use(u, real_bin(v[u], zp, cmul2(w0, w32(u))));
     }
@@ -277,7 +283,7 @@ __device__ __forceinline__ void real_bins(const double2 (&v)[16], double* buf, i
 // Nyquist bin is k = 0's partner, and slot 8 of `self0` is its own partner,
 // X = conj Z.  Half the exchange and products of real_bins.  weight(u) and
 // mirror(u): w at slot u's k and at H - k.
-template <class Wt, class Mi>
+template <int T, class Wt, class Mi>
 __device__ __forceinline__ double real_norms(const double2 (&v)[16], double* buf, int mate, bool self0, double2 w0, const Wt& weight,
                                              const Mi& mirror) {
     double2* half = reinterpret_cast<double2*>(buf);
@@ -289,12 +295,12 @@ __device__ __forceinline__ double real_norms(const double2 (&v)[16], double* buf
     }
     __syncthreads();
 #pragma unroll
-    for (int u = 8; u < 16; ++u) half[(u - 8) * kFftThreads + threadIdx.x] = v[u];
+    for (int u = 8; u < 16; ++u) half[(u - 8) * T + threadIdx.x] = v[u];
     __syncthreads();
     double acc = self0 ? (v[8].x * v[8].x + v[8].y * v[8].y) * weight(8) : 0.0;
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-        double2 zp = half[((self0 && u > 0) ? 8 - u : 7 - u) * kFftThreads + mate];
+        double2 zp = half[((self0 && u > 0) ? 8 - u : 7 - u) * T + mate];
         if (u == 0) zp = make_double2(self0 ? v[0].x : zp.x, self0 ? v[0].y : zp.y);
         const double2 z = v[u], w = cmul2(w0, w32(u));
         const double er = 0.5 * (z.x + zp.x), ei = 0.5 * (z.y - zp.y);
