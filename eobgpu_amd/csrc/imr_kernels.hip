@@ -655,6 +655,7 @@ __device__ __forceinline__ bool sincos_nqc(double x, double* s, double* c) {
 // h_j = amp (sum over modes of h_lm NQC_lm (t_j) for j <= idx, of the ringdown
 // for idx < j < idx + nadd, 0 after), t_j = t_0 + j dT; hplus = Re, hcross = Im.
 constexpr int kImrBlock = 256;
+constexpr int kRingBlocks = 4;   // blocks on a binary's ringdown
 
 // One inspiral sample's sum over the modes: row holds the interval's spline
 // coefficients (Re of each mode, Im of each mode, phi), rpr those of r and pr; nq
@@ -702,23 +703,17 @@ __device__ __forceinline__ long long imr_samples(int idx, int nadd, int len) {
     return (idx < 0 || len < 4) ? 0 : (long long)idx + (nadd > 0 ? nadd : 1);
 }
 
-// Ringdown samples (idx < j < idx + nadd), over the zeros of the inspiral's kernel:
-// a kernel of its own, since its functions would double that one's registers for
-// the few hundred samples of a binary.  grid (blocks, binaries).
-__global__ __launch_bounds__(kImrBlock) void k_imr_ringdown(const int* __restrict__ num_steps, const double* __restrict__ amp, int N, int nm,
-                                                            const double* __restrict__ rd, const double* __restrict__ binf,
-                                                            const int* __restrict__ bini, double* __restrict__ hplus,
-                                                            double* __restrict__ hcross) {
-    const int b = blockIdx.y;
-    const int idx = bini[(size_t)b * kBinICount + kBinIdx];
-    const long long end = imr_samples(idx, bini[(size_t)b * kBinICount + kBinNadd], num_steps[b]);
-    const double a = amp[b], t_match = binf[(size_t)b * kBinCount + kBinTMatch], dt = binf[(size_t)b * kBinCount + kBinDt];
-    const long long stop = end < N ? end : N;
-    for (long long j = (long long)idx + 1 + (long long)blockIdx.x * kImrBlock + threadIdx.x; j < stop; j += (long long)gridDim.x * kImrBlock) {
+// The ringdown of a binary (rd: its modes' rows of kRdCount), the sum over the modes
+// at sample j > idx
+struct Ringdown {
+    const double* rd;
+    double t_match, dt;
+    long long idx;
+    __device__ __forceinline__ void sample(long long j, int nm, double& hr, double& hi) const {
         const double x = (t_match + (double)(j - idx) * dt) - t_match;
-        double hr = 0.0, hi = 0.0;
+        hr = hi = 0.0;
         for (int q = 0; q < nm; ++q) {
-            const double* o = rd + ((size_t)b * nm + q) * kRdCount;
+            const double* o = rd + (size_t)q * kRdCount;
             const double Alm = o[kRdC1c] * tanh(o[kRdC1f] * x + o[kRdC2f]) + o[kRdC2c];
             const double philm = o[kRdPhi] - o[kRdD1c] * log((1.0 + o[kRdD2f] * exp(-o[kRdD1f] * x)) / (1.0 + o[kRdD2f]));
             const double mod = o[kRdEta] * Alm * exp(-o[kRdWi] * x);
@@ -727,10 +722,8 @@ __global__ __launch_bounds__(kImrBlock) void k_imr_ringdown(const int* __restric
             hr += mod * c;
             hi += mod * s;
         }
-        hplus[(size_t)b * N + j] = a * hr;
-        hcross[(size_t)b * N + j] = a * hi;
     }
-}
+};
 
 // grid (blocks, binaries), runs of samples per wavefront (resample.hpp).  512
 // binaries x 2^20 samples at 16384 Hz, five modes, 32% of them inspiral: 6100 us
@@ -741,12 +734,19 @@ __global__ __launch_bounds__(kImrBlock) void k_imr_ringdown(const int* __restric
 // the two hardly overlap (taking the binaries in turn instead scatters the writes
 // and costs a fifth more).  Three wavefronts a SIMD; four (spills) or two samples at once
 // (two wavefronts) are no faster.
+//
+// A binary's last kRingBlocks blocks take its ringdown, which the others leave out.
+// (Its few hundred samples in a launch of their own: 20 us for 17 where one binary
+// of 2^18 samples and one mode is the batch, 34 for 28 with five modes, 280 for 260
+// with 256 binaries of 2^16; by the lanes that would write zeros there: 23, 47 and 386.)
+//
 // kModes: the most modes the staged rows have room for.
 template <int kModes>
 __global__ __launch_bounds__(kImrBlock) void k_imr_resample(const double* __restrict__ dense, const int* __restrict__ num_steps,
                                                             const double* __restrict__ coef, const double* __restrict__ rp,
                                                             const double* __restrict__ amp, const double* __restrict__ dT_M, int max_step,
                                                             int N, int nm, ModeOrder mo, const double* __restrict__ nqc,
+                                                            const double* __restrict__ rd, const double* __restrict__ binf,
                                                             const int* __restrict__ bini, double* __restrict__ hplus,
                                                             double* __restrict__ hcross, int* __restrict__ nsamp) {
     const int cs = 4 * (2 * nm + 1);
@@ -761,7 +761,20 @@ __global__ __launch_bounds__(kImrBlock) void k_imr_resample(const double* __rest
     const double* C = coef + (size_t)b * max_step * cs;
     const double* RP = rp + (size_t)b * max_step * 8;
     const double t0 = T[0], dT = dT_M[b];
-    const SeriesOut o{hplus + (size_t)b * N, hcross + (size_t)b * N, amp[b], jinsp, N};
+    const long long stop = nvalid < N ? nvalid : N;
+    const SeriesOut<true> o{hplus + (size_t)b * N, hcross + (size_t)b * N, amp[b], jinsp, N, stop};   // nvalid >= idx + 1, or 0
+    const unsigned blocks = gridDim.x - kRingBlocks;
+    if (blockIdx.x >= blocks) {
+        const double t_match = binf[(size_t)b * kBinCount + kBinTMatch], dt = binf[(size_t)b * kBinCount + kBinDt];
+        const Ringdown ring{rd + (size_t)b * nm * kRdCount, t_match, dt, idx};
+        for (long long j = idx + 1 + (long long)(blockIdx.x - blocks) * kImrBlock + threadIdx.x; j < stop; j += kRingBlocks * kImrBlock) {
+            double hr, hi;
+            ring.sample(j, nm, hr, hi);
+            o.out[j] = o.a * hr;
+            o.outc[j] = o.a * hi;
+        }
+        return;
+    }
     struct Stage {
         StagedRows<4 * (2 * kModes + 1), 8> modes;   // rows at their own stride cs
         StagedRows<8, 8> rp;
@@ -770,7 +783,7 @@ __global__ __launch_bounds__(kImrBlock) void k_imr_resample(const double* __rest
     __shared__ Stage stages[kImrBlock / 64];
     Stage& st = stages[threadIdx.x >> 6];
     if ((int)(threadIdx.x & 63) < 5 * nm) st.nq[threadIdx.x & 63] = nqc[(size_t)b * nm * 5 + (threadIdx.x & 63)];
-    for_runs(N, kImrBlock / 64, [&](long long j0) {
+    for_runs(N, kImrBlock / 64, blocks, [&](long long j0) {
         if (j0 < jinsp)
             resample_rows<8>(
                 T, len, j0, jinsp, [&](long long j) { return grid_t(j, dT, t0); },
@@ -894,15 +907,15 @@ int eobhip_imr_resample(const double* dense, const int* num_steps, const double*
     if (rc) return rc;
     EOBHIP_REQUIRE(n >= 0 && n <= 65535 && N >= 1, "bad sizes");
     if (n == 0) return EOBHIP_OK;
-    const dim3 grid = resample_grid(N, n), block(kImrBlock);
+    dim3 grid = resample_grid(N, n);
+    const dim3 block(kImrBlock);
     hipStream_t st = as_stream(stream);
     static_assert(kImrMaxModes == 8, "room for every mode");
+    grid.x += kRingBlocks;
     const auto kernel = nm <= 5 ? k_imr_resample<5> : k_imr_resample<8>;
-    hipLaunchKernelGGL(kernel, grid, block, 0, st, dense, num_steps, coef, rp_coef, amp, dT_M, max_step, N, nm, mode_order(mm.m, nm), nqc, bini,
-                       hplus, hcross, nsamp);
-    if ((rc = check_launch("imr_resample"))) return rc;
-    hipLaunchKernelGGL(k_imr_ringdown, dim3(4, n), block, 0, st, num_steps, amp, N, nm, rd, binf, bini, hplus, hcross);
-    return check_launch("imr_ringdown");
+    hipLaunchKernelGGL(kernel, grid, block, 0, st, dense, num_steps, coef, rp_coef, amp, dT_M, max_step, N, nm, mode_order(mm.m, nm), nqc, rd, binf,
+                       bini, hplus, hcross, nsamp);
+    return check_launch("imr_resample");
 }
 
 size_t eobhip_imr_rd_doubles(void) { return kRdCount; }

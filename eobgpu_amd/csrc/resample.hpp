@@ -235,33 +235,43 @@ __device__ __forceinline__ void h22_rows(H22Stage& st, const double* __restrict_
         [&](int i, double x, double& re, double& im) { return h22_sample<kFar>(C + (size_t)12 * i, x, re, im); }, put);
 }
 
-// h+ and hx (hx may be null) of N samples, zero from nb on
+// h+ and hx (hx may be null) of N samples, zero from nb on.  kHole: but samples nb <= j <
+// hole are left as they are.
+template <bool kHole = false>
 struct SeriesOut {
     double *out, *outc;
     double a;
-    long long nb, N;
+    long long nb, N, hole = 0;
+    __device__ __forceinline__ void pair(double* o, long long j, double x, double y) const {
+        if (!kHole || j + 1 < nb || j >= hole) {
+            store_pair<true>(o, j, N, x, y);
+        } else {
+            if (j < nb && j < N) o[j] = x;
+            if (j + 1 >= hole && j + 1 < N) o[j + 1] = y;
+        }
+    }
     __device__ __forceinline__ void put(long long j, const double (&re)[2], const double (&im)[2], bool full) const {
         const bool va = full || j < nb, vb = full || j + 1 < nb;
-        store_pair<true>(out, j, N, va ? a * re[0] : 0.0, vb ? a * re[1] : 0.0);
-        if (outc) store_pair<true>(outc, j, N, va ? a * im[0] : 0.0, vb ? a * im[1] : 0.0);
+        pair(out, j, va ? a * re[0] : 0.0, vb ? a * re[1] : 0.0);
+        if (outc) pair(outc, j, va ? a * im[0] : 0.0, vb ? a * im[1] : 0.0);
     }
     // the run's rows without a sample below nb
     __device__ __forceinline__ void zeros(long long j0) const {
         const long long k = nb > j0 ? (nb - j0 + kRow - 1) / kRow : 0;
         for (int r = k < kRunRows ? (int)k : kRunRows; r < kRunRows; ++r) {
             const long long j = j0 + (long long)r * kRow + 2 * (threadIdx.x & 63);
-            store_pair<true>(out, j, N, 0.0, 0.0);
-            if (outc) store_pair<true>(outc, j, N, 0.0, 0.0);
+            pair(out, j, 0.0, 0.0);
+            if (outc) pair(outc, j, 0.0, 0.0);
         }
     }
 };
 
-// A wavefront's runs of one binary's series, f(j0); grid resample_grid
+// A wavefront's runs of one binary's series by `blocks` blocks, f(j0); grid resample_grid
 template <class F>
-__device__ __forceinline__ void for_runs(long long N, int waves, const F& f) {
+__device__ __forceinline__ void for_runs(long long N, int waves, unsigned blocks, const F& f) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const long long nrun = (N + kRun - 1) / kRun;
-    for (long long run = (long long)blockIdx.x * waves + wave; run < nrun; run += (long long)gridDim.x * waves) f(run * kRun);
+    for (long long run = (long long)blockIdx.x * waves + wave; run < nrun; run += (long long)blocks * waves) f(run * kRun);
 }
 
 // (blocks of four wavefronts, binaries): about 131072 blocks in all, no more, so

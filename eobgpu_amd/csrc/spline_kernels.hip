@@ -614,12 +614,12 @@ __global__ __launch_bounds__(kBlock) void k_resample_hplus(const double* __restr
     const double dT = dT_M[b];
     const long long nb = series_samples(T, len, dT, N);
     if (blockIdx.x == 0 && threadIdx.x == 0) nsamp[b] = (int)nb;
-    const SeriesOut o{hplus + (size_t)b * N, hcross ? hcross + (size_t)b * N : nullptr, amp[b], nb, N};
+    const SeriesOut<> o{hplus + (size_t)b * N, hcross ? hcross + (size_t)b * N : nullptr, amp[b], nb, N};
     const double* C = coef + (size_t)b * max_step * 12;
     const double t0 = T[0];
     __shared__ H22Stage stages[kBlock / 64];
     H22Stage& st = stages[threadIdx.x >> 6];
-    for_runs(N, kBlock / 64, [&](long long j0) {
+    for_runs(N, kBlock / 64, gridDim.x, [&](long long j0) {
         if (j0 < nb)
             h22_rows(st, T, C, len, t0, dT, j0, nb, [&](long long j, const double (&re)[2], const double (&im)[2], bool full) { o.put(j, re, im, full); });
         o.zeros(j0);
@@ -680,11 +680,11 @@ __global__ __launch_bounds__(kBlock) void k_resample_modes(const double* __restr
     const double dT = dT_M[b], t0 = T[0];
     const long long nb = series_samples(T, len, dT, N);
     if (blockIdx.x == 0 && threadIdx.x == 0) nsamp[b] = (int)nb;
-    const SeriesOut o{hplus + (size_t)b * N, hcross + (size_t)b * N, amp[b], nb, N};
+    const SeriesOut<> o{hplus + (size_t)b * N, hcross + (size_t)b * N, amp[b], nb, N};
     typedef StagedRows<4 * (2 * kModes + 1), 8> Stage;   // rows at their own stride cs
     __shared__ Stage stages[kBlock / 64];
     Stage& st = stages[threadIdx.x >> 6];
-    for_runs(N, kBlock / 64, [&](long long j0) {
+    for_runs(N, kBlock / 64, gridDim.x, [&](long long j0) {
         if (j0 < nb)
             resample_rows<Stage::kRows>(
                 T, len, j0, nb, [&](long long j) { return t0 + (double)j * dT; }, [&](int i, int n) { st.copy(C + (size_t)cs * i, n, cs); },
