@@ -280,10 +280,8 @@ class EOBBatch:
         """Not-a-knot splines of phi, Re and Im of h22 e^{2 i phi} over each binary's knots."""
         if getattr(self, "coef", None) is None:
             self.coef = torch.empty((self.n, self.max_step, 12), dtype=torch.float64, device=self.device)
-            self.spline_scratch = torch.empty(int(lib().eobhip_spline_scratch_doubles(self.n, self.max_step)), dtype=torch.float64,
-                                              device=self.device)
         call("eobhip_spline_build_batched", self.dense.data_ptr(), self.knots.data_ptr(), self.num_steps.data_ptr(), self.n,
-             self.max_step, self.coef.data_ptr(), self.spline_scratch.data_ptr(), current_stream())
+             self.max_step, self.coef.data_ptr(), None, current_stream())
         return self.coef
 
     def resample_hplus(self, total_mass_msun, dt, N, amp=None, out=None):
@@ -791,7 +789,6 @@ class _Rows:
         self.modes = torch.empty((cap, self.md_bytes), dtype=torch.uint8, device=device)
         self.knots = torch.empty((cap, max_step, 3), dtype=torch.float64, device=device)
         self.coef = torch.empty((cap, max_step, 12), dtype=torch.float64, device=device)
-        self.spline_scratch = torch.empty(int(L.eobhip_spline_scratch_doubles(cap, max_step)), dtype=torch.float64, device=device)
         self.dT_M = torch.empty(cap, dtype=torch.float64, device=device)
         self.amp = torch.empty(cap, dtype=torch.float64, device=device)
         self.pos = torch.empty(cap, dtype=torch.int64, device=device)
@@ -808,7 +805,7 @@ class _Rows:
         v.n, v.max_step, v.device = k, self.max_step, self.device
         v.dense, v.num_steps = self.dense[:k], self.num_steps[:k]
         v.bindata, v.modes = self.bindata[:k], self.modes[:k]
-        v.knots, v.coef, v.spline_scratch = self.knots[:k], self.coef[:k], self.spline_scratch
+        v.knots, v.coef = self.knots[:k], self.coef[:k]
         return v
 
 
@@ -1087,7 +1084,6 @@ class GraphPass:
         b = self.batch
         b.knots = torch.zeros((n, b.max_step, 3), dtype=torch.float64, device=device)
         b.coef = torch.zeros((n, b.max_step, 12), dtype=torch.float64, device=device)
-        b.spline_scratch = torch.zeros(int(L.eobhip_spline_scratch_doubles(n, b.max_step)), dtype=torch.float64, device=device)
         self.cond = torch.zeros((4, n), dtype=torch.float64, device=device)
         self.nsamp = torch.zeros(n, dtype=torch.int32, device=device)
         self.hp = torch.zeros((n, self.N), dtype=torch.float64, device=device)
@@ -1124,7 +1120,7 @@ class GraphPass:
         call("eobhip_hlm22_knots", b.dense.data_ptr(), b.num_steps.data_ptr(), b.bindata.data_ptr(), b.modes.data_ptr(), n,
              b.max_step, b.knots.data_ptr(), s)
         call("eobhip_spline_build_batched", b.dense.data_ptr(), b.knots.data_ptr(), b.num_steps.data_ptr(), n, b.max_step,
-             b.coef.data_ptr(), b.spline_scratch.data_ptr(), s)
+             b.coef.data_ptr(), None, s)
         call("eobhip_resample_hplus", b.dense.data_ptr(), b.coef.data_ptr(), b.num_steps.data_ptr(), par[6].data_ptr(),
              par[5].data_ptr(), n, b.max_step, self.N, self.hp.data_ptr(), self.nsamp.data_ptr(), s)
         call("eobhip_rfft_batched", self.hp.data_ptr(), self.ht.data_ptr(), n, self.N, s)

@@ -102,8 +102,6 @@ class SlotPool:
         self.dense = torch.zeros((c, ms, 5), dtype=torch.float64, device=device)
         self.knots = torch.zeros((c, ms, 3), dtype=torch.float64, device=device)
         self.coef = torch.zeros((c, ms, 12), dtype=torch.float64, device=device)
-        self.spl_per_bin = int(L.eobhip_spline_scratch_doubles(1, ms))
-        self.spl = torch.zeros(c * self.spl_per_bin, dtype=torch.float64, device=device)
         self.hp = torch.zeros((c, self.N), dtype=torch.float64, device=device)
         self.ht = torch.zeros((c, self.F), dtype=torch.complex128, device=device)
         self.num_steps = torch.zeros(c, dtype=torch.int32, device=device)
@@ -119,7 +117,7 @@ class SlotPool:
         L = lib()
         F = N // 2 + 1
         return (int(L.eobhip_bindata_bytes()) + int(L.eobhip_modes_bytes())
-                + 8 * max_step * (5 + 3 + 12) + 8 * int(L.eobhip_spline_scratch_doubles(1, max_step)) + 8 * N + 16 * F
+                + 8 * max_step * (5 + 3 + 12) + 8 * N + 16 * F
                 + 4 * 4 + 8 * 2)
 
     def bytes_per_binary(self):
@@ -312,7 +310,7 @@ class Server:
             call("eobhip_hlm22_knots", dense.data_ptr(), pool.num_steps[sl].data_ptr(), bd.data_ptr(), md.data_ptr(), nb,
                  pool.max_step, pool.knots[sl].data_ptr(), s)
             call("eobhip_spline_build_batched", dense.data_ptr(), pool.knots[sl].data_ptr(), pool.num_steps[sl].data_ptr(), nb,
-                 pool.max_step, pool.coef[sl].data_ptr(), pool.spl[start * pool.spl_per_bin:].data_ptr(), s)
+                 pool.max_step, pool.coef[sl].data_ptr(), None, s)
             call("eobhip_resample_hplus", dense.data_ptr(), pool.coef[sl].data_ptr(), pool.num_steps[sl].data_ptr(),
                  par[6].data_ptr(), par[5].data_ptr(), nb, pool.max_step, self.N, pool.hp[sl].data_ptr(), pool.nsamp[sl].data_ptr(), s)
             row = start

@@ -237,9 +237,9 @@ int eobhip_hlm22_knots(const double* dense, const int* num_steps, const void* bi
 
 /* Not-a-knot splines of the three knot series (phi and Re, Im of h22 e^{2 i phi}) per
  * binary (CubicSplineInterpolantTD / interpolate_TD semantics, src/interpolate.cu:11-308),
- * by tiles of each binary's knots.  coef [n][max_step][12] = (y, c1, c2, c3) x 3;
- * scratch: eobhip_spline_scratch_doubles(n, max_step) doubles (binary b's part starts at
- * b * eobhip_spline_scratch_doubles(1, max_step)); the tiles leave it unused. */
+ * by tiles of each binary's knots.  coef [n][max_step][12] = (y, c1, c2, c3) x 3.
+ * scratch is not used and may be null; eobhip_spline_scratch_doubles is what callers that
+ * still allocate it ask. */
 size_t eobhip_spline_scratch_doubles(int n, int max_step);
 /* The same splines for any number of series: knots [n][max_step][nser],
  * coef [n][max_step][4 nser], 1 <= nser <= 32; scratch:
