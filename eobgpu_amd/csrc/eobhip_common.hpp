@@ -46,13 +46,14 @@ int fft_rows(int inverse, const void* in, void* out, int n, int N, void* stream)
 int rfft_own_log2(const void* in, const void* out, int n, int N);
 int rfft_own(const double* in, double* out, int n, int log2N, hipStream_t st);
 constexpr int kRfftMinLog2 = 10, kRfftMaxLog2 = 21;
+constexpr int kRfftOneMaxLog2 = 14;   // up to here a block of the most threads holds a row
 
 // sum_k w_k |X_k|^2 over the N/2 + 1 bins of n rows of N samples (same lengths),
 // without writing the bins: row r has count[map[r]] samples at in + r in_stride
 // (defined up to the next even count, zero after), its rfft_norm_partials(log2 N)
 // partial sums go to partial + map[r] pstride.  work: n N/2 complex (unused up
 // to N = 2^14).
-int rfft_norm_partials(int log2N);
+constexpr __host__ __device__ int rfft_norm_partials(int log2N) { return log2N <= kRfftOneMaxLog2 ? 1 : 1 << (log2N - kRfftOneMaxLog2); }
 int rfft_weighted_norm(const double* in, long long in_stride, double* work, int n, int log2N, const int* count, const long long* map,
                        const double* w, double* partial, int pstride, hipStream_t st);
 

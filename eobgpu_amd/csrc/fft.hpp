@@ -42,7 +42,7 @@ namespace eobhip_detail {
 constexpr int kFftThreads = 512;   // the most
 constexpr int kFftPoints = 16 * kFftThreads;
 constexpr int kFftMinLog2 = kRfftMinLog2, kFftMaxLog2 = kRfftMaxLog2;   // N
-constexpr int kFftOneMaxLog2 = 14;   // N whose H = N/2 points fit one block
+constexpr int kFftOneMaxLog2 = kRfftOneMaxLog2;   // N whose H = N/2 points fit one block
 static_assert((1 << (kFftOneMaxLog2 - 1)) == kFftPoints, "one-kernel limit");
 
 __device__ __forceinline__ double2 cmul2(double2 a, double2 b) { return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); }

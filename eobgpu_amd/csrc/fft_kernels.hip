@@ -181,6 +181,7 @@ __global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(T == kFftThre
         const unsigned k0 = (unsigned)ka + ((unsigned)p << LA), up = (unsigned)(per << LA);
         const double acc = real_norms<T>(v, buf, mate, self0, w0, [&](int u) { return w[k0 + up * u]; },
                                       [&](int u) { return w[(unsigned)H - (k0 + up * u)]; });
+        static_assert(T == kFftThreads, "rfft_norm_partials counts these blocks");
         const double s = group_sum<T>(acc, buf);
         if (t == 0) nm.partial[a.map[row] * nm.pstride + g] = s;
     } else {
@@ -269,8 +270,6 @@ int rfft_own_log2(const void* in, const void* out, int n, int N) {
     if (a < b + nb && b < a + na) return 0;
     return __builtin_ctz((unsigned)N);
 }
-
-int rfft_norm_partials(int log2N) { return log2N <= kFftOneMaxLog2 ? 1 : 1 << (log2N - kFftOneMaxLog2); }
 
 int rfft_weighted_norm(const double* in, long long in_stride, double* work, int n, int log2N, const int* count, const long long* map,
                        const double* w, double* partial, int pstride, hipStream_t st) {

@@ -236,7 +236,7 @@ __global__ __launch_bounds__(64) void k_lik_final(const double* __restrict__ cro
     if (b >= n) return;
     double c = 0.0, h = 0.0;
     const int nc = nsamp ? (nsamp[b] + kSpan - 1) / kSpan : gx;
-    const int nh = mlog2 ? (mlog2[b] <= 14 ? 1 : 1 << (mlog2[b] - 14)) : gx2;
+    const int nh = mlog2 ? rfft_norm_partials(mlog2[b]) : gx2;
     for (int i = threadIdx.x; i < nc; i += 64) c += cross_partial[(size_t)b * gx + i];
     for (int i = threadIdx.x; i < nh; i += 64) h += hh_partial[(size_t)b * gx2 + i];
 #pragma unroll
