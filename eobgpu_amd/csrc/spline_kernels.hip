@@ -27,14 +27,26 @@ constexpr int kBlock = 256;
 constexpr double kPi = 3.141592653589793;
 
 
-// The interior form of a row from its two intervals (spacing, slope).
+// The interior form of a row from its two intervals (spacing, slope); its right-hand
+// side without the factor 3.
 __device__ __forceinline__ Row interior_row(double d1, double m1, double d2, double m2) {
     Row r;
-    r.b = 3.0 * (d2 * m1 + d1 * m2);
+    r.b = d2 * m1 + d1 * m2;
     r.dg = 2 * (d1 + d2);
     r.ud = d1;
     r.ld = d2;
     return r;
+}
+
+// v / d from r = 1 / d: the product and one correction, which rounds as the division
+// does for normal numbers (Markstein's method).  With plain products, and 3 times a
+// right-hand side rounded before it is used, the coefficients' error against extended
+// precision was 4 to 25 % larger (rms; 1.5 to 2 times between the knots of uneven
+// chirps) than one elimination from the first row leaves; this way it is equal, for
+// 4 % of the builders' time.
+__device__ __forceinline__ double over(double v, double d, double r) {
+    const double w = v * r;
+    return fma(fma(-d, w, v), r, w);
 }
 
 // How far from its own rows a lane starts its eliminations (see the batched
@@ -75,12 +87,14 @@ __global__ __launch_bounds__(kBlock) void k_interpolate_TD(const double* __restr
     const int step = gridDim.y * (kBlock / 64);
     for (int ch = blockIdx.y * (kBlock / 64) + (threadIdx.x >> 6); ch < (len + kDropOwn - 1) / kDropOwn; ch += step) {
         const int s0 = ch * kDropOwn, e0 = s0 + kDropOwn < len ? s0 + kDropOwn : len;
-        // from above: s_{e0} = e - f s_{e0-1}
-        double f = 0.0, e = 0.0;
+        // rows are eliminated as D s + (the neighbour's coefficient) s' = B, a quotient each
+        // from above: Da s_{e0} + la s_{e0-1} = Ba, ia = 1 / Da
+        double Da = 1.0, ia = 1.0, Ba = 0.0, la = 0.0;
         for (int halo = kHalo; e0 < len; halo = kHaloMax) {
             const int hi = e0 + halo < len ? e0 + halo : len;
             double damp = hi == len ? 0.0 : 1.0;
-            f = e = 0.0;
+            Da = ia = 1.0;
+            Ba = la = 0.0;
             double tp = c.T(hi < len ? hi : len - 1), yp = c.Y(hi < len ? hi : len - 1);
             double t0 = c.T(hi - 1), y0 = c.Y(hi - 1);
             double d2 = tp - t0, m2 = (yp - y0) / d2;
@@ -89,22 +103,28 @@ __global__ __launch_bounds__(kBlock) void k_interpolate_TD(const double* __restr
                 const double tm = c.T(i - 1), ym = c.Y(i - 1);
                 const double d1 = t0 - tm, m1 = (y0 - ym) / d1;
                 Row r = interior_row(d1, m1, d2, m2);
-                if (i == len - 1) r = c.end(i);
-                const double up = i == hi - 1 ? 0.0 : r.ud;
-                const double inv = 1.0 / (r.dg - up * f);
-                damp *= r.ud * inv;
-                e = (r.b - up * e) * inv;
-                f = r.ld * inv;
+                double three = 3.0;
+                if (i == len - 1) {
+                    r = c.end(i);
+                    three = 1.0;
+                }
+                const double w = i == hi - 1 ? 0.0 : over(r.ud, Da, ia);
+                Da = r.dg - w * la;
+                Ba = fma(three, r.b, -(w * Ba));   // 3 r.b is not rounded by itself
+                la = r.ld;
+                ia = 1.0 / Da;
+                damp *= r.ud * ia;
                 t0 = tm; y0 = ym; d2 = d1; m2 = m1;
             }
             if (fabs(damp) < kDamped || halo == kHaloMax) break;
         }
-        // from below: s_{s0-1} = pd - pc s_{s0}
-        double pc = 0.0, pd = 0.0, t0 = 0.0, y0 = 0.0, d1 = 1.0, m1 = 0.0;
+        // from below: D s_{s0-1} + u s_{s0} = Bb, id = 1 / D
+        double D = 1.0, id = 1.0, Bb = 0.0, u = 0.0, t0 = 0.0, y0 = 0.0, d1 = 1.0, m1 = 0.0;
         for (int halo = kHalo;; halo = kHaloMax) {
             const int lo = s0 - halo > 0 ? s0 - halo : 0;
             double damp = lo == 0 ? 0.0 : 1.0;
-            pc = pd = 0.0;
+            D = id = 1.0;
+            Bb = u = 0.0;
             t0 = c.T(lo);
             y0 = c.Y(lo);
             if (lo > 0) {
@@ -116,18 +136,23 @@ __global__ __launch_bounds__(kBlock) void k_interpolate_TD(const double* __restr
                 const double tp = c.T(i + 1), yp = c.Y(i + 1);
                 const double d2 = tp - t0, m2 = (yp - y0) / d2;
                 Row r = interior_row(d1, m1, d2, m2);
-                if (i == 0) r = c.end(0);
-                const double dn = i == lo ? 0.0 : r.ld;
-                const double inv = 1.0 / (r.dg - dn * pc);
-                damp *= r.ld * inv;
-                pd = (r.b - dn * pd) * inv;
-                pc = r.ud * inv;
+                double three = 3.0;
+                if (i == 0) {
+                    r = c.end(0);
+                    three = 1.0;
+                }
+                const double w = i == lo ? 0.0 : over(r.ld, D, id);
+                D = r.dg - w * u;
+                Bb = fma(three, r.b, -(w * Bb));
+                u = r.ud;
+                id = 1.0 / D;
+                damp *= r.ld * id;
                 t0 = tp; y0 = yp; d1 = d2; m1 = m2;
             }
             if (fabs(damp) < kDamped || halo == kHaloMax) break;
         }
         // the lane's rows, then back through them
-        double pcs[kDropOwn], pds[kDropOwn], last_dg = 0.0, last_ld = 0.0;
+        double Ds[kDropOwn], Bs[kDropOwn], last_ld = 0.0;
 #pragma unroll
         for (int j = 0; j < kDropOwn; ++j) {
             const int i = s0 + j;
@@ -136,27 +161,35 @@ __global__ __launch_bounds__(kBlock) void k_interpolate_TD(const double* __restr
                 const double tp = c.T(k), yp = c.Y(k);
                 const double d2 = tp - t0, m2 = (yp - y0) / d2;
                 Row r = interior_row(d1, m1, d2, m2);
-                if (i == 0 || i == len - 1) r = c.end(i);
-                const double den = r.dg - r.ld * pc, inv = 1.0 / den;
-                pd = (r.b - r.ld * pd) * inv;
-                pc = r.ud * inv;
-                last_dg = den;
+                double three = 3.0;
+                if (i == 0 || i == len - 1) {
+                    r = c.end(i);
+                    three = 1.0;
+                }
+                const double w = over(r.ld, D, id);   // row 0: ld = 0
+                D = r.dg - w * u;
+                Bb = fma(three, r.b, -(w * Bb));
+                u = r.ud;
+                id = 1.0 / D;
                 last_ld = r.ld;
                 t0 = tp; y0 = yp; d1 = d2; m1 = m2;
             }
-            pcs[j] = pc;
-            pds[j] = pd;
+            Ds[j] = D;
+            Bs[j] = Bb;
         }
-        double xi = (pd - pc * e) / (1.0 - pc * f);
-        double xn = e - f * xi;
-        double tn = c.T(e0 < len ? e0 : len - 1), yn = c.Y(e0 < len ? e0 : len - 1);
+        const double w = over(u, Da, ia);
+        double xi = (Bb - w * Ba) / (D - w * la), xn = (Ba - la * xi) / Da;
+        double tn = c.T(e0 < len ? e0 : len - 1), yn = c.Y(e0 < len ? e0 : len - 1), ti = c.T(e0 - 1);
 #pragma unroll
         for (int j = kDropOwn - 1; j >= 0; --j) {
             const int i = s0 + j;
             if (i < e0) {
-                if (i < e0 - 1) xi = pds[j] - pcs[j] * xn;
+                const double tm = c.T(i > 0 ? i - 1 : 0), yi = c.Y(i);
+                if (i < e0 - 1) {
+                    const double ui = i > 0 ? ti - tm : c.end(0).ud;
+                    xi = over(Bs[j] - ui * xn, Ds[j], 1.0 / Ds[j]);
+                }
                 const size_t o = (size_t)i * ninterp + it;
-                const double ti = c.T(i), yi = c.Y(i);
                 B[o] = xi;
                 if (i < len - 1) {
                     const double dt = tn - ti, slope = (yn - yi) / dt;
@@ -167,10 +200,10 @@ __global__ __launch_bounds__(kBlock) void k_interpolate_TD(const double* __restr
                 } else {
                     // the last row keeps the eliminated system's values, as the reference leaves them
                     ud[o] = 0.0;
-                    dg[o] = last_dg;
+                    dg[o] = D;
                     ld[o] = last_ld;
                 }
-                xn = xi; tn = ti; yn = yi;
+                xn = xi; tn = ti; yn = yi; ti = tm;
             }
         }
     }
@@ -213,13 +246,13 @@ static_assert(kTile / kOwn == 64, "one wavefront per series");
 __device__ __forceinline__ int tile_at(int k) { return k + (k >> 4); }
 
 // One elimination row: from the neighbour's relation s_n = g - h s (g, h in, cut
-// rows g = h = 0) and the row a s_n + dg s + c s_next = b to s = b' - c' s_next.
+// rows g = h = 0) and the row a s_n + dg s + c s_next = k b to s = b' - c' s_next.
 struct Carry {
     double h, g;   // c', d'
-    __device__ __forceinline__ double step(double a, double dg, double c, double b) {
-        const double inv = eob::refined_rcp(dg - a * h);
-        g = (b - a * g) * inv;
-        h = c * inv;
+    __device__ __forceinline__ double step(double a, double dg, double c, double b, double k = 3.0) {
+        const double den = dg - a * h, inv = eob::refined_rcp(den);
+        g = over(fma(k, b, -(a * g)), den, inv);
+        h = over(c, den, inv);
         return inv;
     }
 };
@@ -292,22 +325,22 @@ __global__ __launch_bounds__(kTileThreads) void k_spline_build_tile(const double
                 if (i0 == 0) {
                     a1 = D(0);
                     am = M(0);
-                    dn.step(0.0, fdg, fud, fb);
+                    dn.step(0.0, fdg, fud, fb, 1.0);
                 } else {
                     const double b1 = D(i0 - 1), bm = M(i0 - 1);
                     a1 = D(i0);
                     am = M(i0);
-                    down = a1 * dn.step(0.0, 2 * (b1 + a1), b1, 3.0 * (a1 * bm + b1 * am));
+                    down = a1 * dn.step(0.0, 2 * (b1 + a1), b1, a1 * bm + b1 * am);
                 }
             }
             if (e0 < len) {
                 c2 = D(i9 - 2);
                 cm = M(i9 - 2);
                 if (i9 == len) {
-                    up.step(0.0, ldg, lld, lb);
+                    up.step(0.0, ldg, lld, lb, 1.0);
                 } else {
                     const double b2 = D(i9 - 1), bm = M(i9 - 1);
-                    above = c2 * up.step(0.0, 2 * (c2 + b2), b2, 3.0 * (b2 * cm + c2 * bm));
+                    above = c2 * up.step(0.0, 2 * (c2 + b2), b2, b2 * cm + c2 * bm);
                 }
             }
             // row i below: intervals i - 1 (a1, am) and i; row j above: j - 1 and j (c2, cm)
@@ -316,13 +349,13 @@ __global__ __launch_bounds__(kTileThreads) void k_spline_build_tile(const double
                 const int i = i0 + k, j = i9 - 1 - k;
                 if (i < s0) {
                     const double d2 = D(i), m2 = M(i);
-                    down *= d2 * dn.step(d2, 2 * (a1 + d2), a1, 3.0 * (d2 * am + a1 * m2));
+                    down *= d2 * dn.step(d2, 2 * (a1 + d2), a1, d2 * am + a1 * m2);
                     a1 = d2;
                     am = m2;
                 }
                 if (j >= e0) {
                     const double d0 = D(j - 1), m0 = M(j - 1);
-                    above *= d0 * up.step(d0, 2 * (d0 + c2), c2, 3.0 * (c2 * m0 + d0 * cm));
+                    above *= d0 * up.step(d0, 2 * (d0 + c2), c2, c2 * m0 + d0 * cm);
                     c2 = d0;
                     cm = m0;
                 }
@@ -341,8 +374,8 @@ __global__ __launch_bounds__(kTileThreads) void k_spline_build_tile(const double
                 const double d2 = D(k), m2 = M(k);
                 const bool first = i == 0, last = i == len - 1;
                 const double a = first ? 0.0 : (last ? lld : d2), dg = first ? fdg : (last ? ldg : 2 * (d1 + d2));
-                const double c = first ? fud : (last ? 0.0 : d1), r = first ? fb : (last ? lb : 3.0 * (d2 * m1 + d1 * m2));
-                dn.step(a, dg, c, r);
+                const double c = first ? fud : (last ? 0.0 : d1), r = first ? fb : (last ? lb : d2 * m1 + d1 * m2);
+                dn.step(a, dg, c, r, first || last ? 1.0 : 3.0);
                 d1 = d2;
                 m1 = m2;
             }
@@ -380,12 +413,11 @@ __global__ __launch_bounds__(kTileThreads) void k_spline_build_tile(const double
         if (i < len - 1) {
             const double xi = mq[p][tile_at(j)], xn = mq[p][tile_at(j + 1)];
             const double dt = dx[tile_at(i - lo)], rt = eob::refined_rcp(dt);
-            const auto over = [&](double v) { const double w = v * rt; return fma(fma(-dt, w, v), rt, w); };   // v / dt
-            const double slope = over(y[G] - yi);
-            const double tt = over(xi + xn - 2 * slope);
+            const double slope = over(y[G] - yi, dt, rt);
+            const double tt = over(xi + xn - 2 * slope, dt, rt);
             c1 = xi;
-            c2 = over(slope - xi) - tt;
-            c3 = over(tt);
+            c2 = over(slope - xi, dt, rt) - tt;
+            c3 = over(tt, dt, rt);
         }
         double* c = C + (size_t)(4 * G) * i + 4 * p;
         c[0] = yi;
