@@ -8,7 +8,8 @@
 // kFftThreads threads holds kFftPoints complex points, 16 per thread in
 // registers, and exchanges them through LDS between radix-16 stages (real
 // parts first, then imaginary parts, so that the exchange buffer is 8 bytes
-// per point and two blocks share a CU's LDS):
+// per point and two blocks share a CU's LDS; but for the column pass of 2^15,
+// whose 64 columns' step table makes it 87 kB and one block a CU):
 //   H <= kFftPoints   one kernel (k_rfft_one): whole rows in a block;
 //   larger H = A B    two kernels, the row as an A x B matrix (j = a B + b):
 //     k_rfft_cols: length-A transforms of C consecutive columns b, times

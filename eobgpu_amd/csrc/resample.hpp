@@ -195,9 +195,11 @@ __device__ __forceinline__ void resample_rows(const double* __restrict__ T, int 
     }
 }
 
-// Two consecutive samples of a series of N.  kStream: past the caches (a series
-// longer than they hold: 1682 us for the five-mode sum of 512 binaries x 2^20
-// against 2496 through them).
+// Two consecutive samples of a series of N.  kStream: past the caches.  The mode sum
+// of 512 binaries x 2^20 1682 us against 2496 through them, h+ of 64 x 2^18 46 against
+// 50, of one binary the same; what reads the series next loses at most what that
+// gains (h+ and its transform, streamed and not: 256 x 2^20 2183 and 2204 us, 64 x
+// 2^17 85 and 76, 16 x 2^14 20 and 20, 1 x 2^20 30 and 29), so that no size is worth a rule.
 template <bool kStream>
 __device__ __forceinline__ void store_pair(double* out, long long j, long long N, double a, double b) {
     if (j + 1 < N) {

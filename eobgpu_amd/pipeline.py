@@ -439,7 +439,10 @@ def _host_ints(xs):
 
 
 def rfft_batched(h, out=None):
-    """Row-wise real-to-complex FFT (hipFFT D2Z), no dt factor (as the reference's rfft)."""
+    """Row-wise real-to-complex FFT, no dt factor (as the reference's rfft): the library's
+    own kernels for rows of 2^10 .. 2^21 samples at 16-byte boundaries and an output
+    that does not overlap them, hipFFT's plans (per stream, length and row chunk)
+    otherwise."""
     n, N = h.shape
     if out is None:
         out = torch.empty((n, N // 2 + 1), dtype=torch.complex128, device=h.device)

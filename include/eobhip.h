@@ -302,8 +302,10 @@ int eobhip_detector_response(const double* ra, const double* dec, const double* 
 int eobhip_detector_signal(const double* hp_fd, const double* hc_fd, const double* Fplus, const double* Fcross, const double* time_shift,
                            int n, int nifo, int F, double df, int k_min, double* out, void* stream);
 
-/* Row-wise real-to-complex FFT, n rows of N doubles -> n rows of N/2+1 complex (hipFFT D2Z;
- * like the reference's rfft without a dt factor, eob/seobnrv4phm.py:742-744). */
+/* Row-wise real-to-complex FFT, n rows of N doubles -> n rows of N/2+1 complex (like the
+ * reference's rfft without a dt factor, eob/seobnrv4phm.py:742-744).  N = 2^10 .. 2^21 with in
+ * and out at 16-byte boundaries and not overlapping: the library's own kernels, with no plan
+ * or workspace; every other even N: hipFFT D2Z plans, kept per (N, rows per call, stream). */
 int eobhip_rfft_batched(const double* in, double* out, int n, int N, void* stream);
 /* log L_b = -1/2 * 4 df * sum_k |d_k - h_b,k|^2 / S(f_k) with the analytic
  * S(f) = (f/f0)^-4 + 1 + (f/f0)^2 (1/S(0) = 0): the reduction of all_in_one_likelihood
