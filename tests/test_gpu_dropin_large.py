@@ -51,4 +51,4 @@ def test_large_batches_are_no_slower_than_by_blocks(dev, base):  # noqa: F811
             torch.cuda.synchronize()
             t.append(a.elapsed_time(b))
         return min(t)
-    assert ms(131072) < 2.75 * ms(32768)
+    assert ms(131072) < 3.0 * ms(32768)

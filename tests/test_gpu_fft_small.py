@@ -56,4 +56,4 @@ def test_few_rows_take_no_longer_than_a_plan(dev, N, rows):
     us(8)
     plan, own = us(8), us(0)
     # 0.75 to 1.05 of the plan's time; with one block size for every batch 1.1 to 1.6
-    assert own <= (1.25 if N < 1 << 11 else 1.08) * plan, (own, plan)
+    assert own <= (1.25 if N <= 1 << 11 else 1.08) * plan, (own, plan)

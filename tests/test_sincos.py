@@ -56,24 +56,37 @@ def test_host_build():
 
 
 @pytest.mark.gpu
-def test_resampled_phases(dev):
+@pytest.mark.parametrize("every", [1, 64])   # samples a knot: every row past the staged ones, and staged rows of two
+@pytest.mark.parametrize("kind", ["hpc", "modes"])
+def test_resampled_phases(dev, every, kind):
     import torch
     from eobgpu_amd._lib import call
-    x = arguments(20000)
-    x = np.concatenate([[np.inf, -np.inf, np.nan], x])
-    K = 4096
-    n = -(-len(x) // K)
-    phase = np.zeros(n * K)
-    phase[:len(x)] = x / 2                      # h22 = S e^{-2 i phi}; the argument is twice this
+    x = arguments(4000)
+    x = np.concatenate([[np.inf, -np.inf, np.nan], np.random.default_rng(1).permutation(x)])
+    K = 2048
+    n, N = -(-len(x) // K), K * every
+    arg = np.zeros(n * K)
+    arg[:len(x)] = x
     dense, coef = np.zeros((n, K, 5)), np.zeros((n, K, 12))
-    dense[:, :, 0] = np.arange(K)               # sample j is knot j
-    coef[:, :, 0], coef[:, :, 4] = phase.reshape(n, K), 1.0
+    dense[:, :, 0] = every * np.arange(K)
+    if kind == "hpc":      # h22 = S e^{-2 i phi}; the argument is twice this
+        arg = 2 * (arg / 2)
+        coef[:, :, 0], coef[:, :, 4] = (arg / 2).reshape(n, K), 1.0
+    else:                  # S e^{-i phi}
+        coef[:, :, 8], coef[:, :, 0] = arg.reshape(n, K), 1.0
     dv = lambda a, t=torch.float64: torch.as_tensor(a, dtype=t, device=dev)  # noqa: E731
     d, cf, ns, one = dv(dense), dv(coef), dv(np.full(n, K), torch.int32), dv(np.ones(n))
-    hp, hc, cnt = dv(np.zeros((n, K))), dv(np.zeros((n, K))), dv(np.zeros(n), torch.int32)
-    call("eobhip_resample_hpc", d.data_ptr(), cf.data_ptr(), ns.data_ptr(), one.data_ptr(), one.data_ptr(), n, K, K, hp.data_ptr(),
-         hc.data_ptr(), cnt.data_ptr(), None)
-    c, s = hp.cpu().numpy().ravel(), -hc.cpu().numpy().ravel()
-    assert np.all(cnt.cpu().numpy() == K)
-    assert np.all(np.isnan(s[:3])) and np.all(np.isnan(c[:3]))
-    check(2 * phase[3:], s[3:], c[3:])
+    hp, hc, cnt = dv(np.zeros((n, N))), dv(np.zeros((n, N))), dv(np.zeros(n), torch.int32)
+    args = [d.data_ptr(), cf.data_ptr(), ns.data_ptr(), one.data_ptr(), one.data_ptr(), n, K, N]
+    if kind == "hpc":
+        call("eobhip_resample_hpc", *args, hp.data_ptr(), hc.data_ptr(), cnt.data_ptr(), None)
+    else:
+        call("eobhip_resample_modes", *args, 1, (ctypes.c_int * 1)(1), hp.data_ptr(), hc.data_ptr(), cnt.data_ptr(), None)
+    assert np.all(cnt.cpu().numpy() == every * (K - 1) + 1)
+    # all samples of a knot have its phase
+    for j in {0, every // 2, every - 1}:
+        c, s = (v.view(n, K, every)[:, :K - 1, j].cpu().numpy() for v in (hp, -hc))
+        a = arg.reshape(n, K)[:, :K - 1]
+        bad = ~np.isfinite(a)
+        assert bad.sum() == 3 and np.all(np.isnan(c[bad])) and np.all(np.isnan(s[bad]))
+        check(a[~bad], s[~bad], c[~bad])
