@@ -640,7 +640,7 @@ __global__ __launch_bounds__(64) void k_imr_params(BinInputs in, const double* _
 // the wavefront has |x| < 1/16 (first omitted terms below 2.3e-20 relative),
 // sincos_of otherwise.  The NQC phase of the inspiral samples is small except near the
 // attachment.
-template <SamplePath P>
+template <Phases P>
 __device__ __forceinline__ bool sincos_nqc(double x, double* s, double* c) {
     if (__all(fabs(x) < 0.0625)) {
         const double x2 = x * x;
@@ -662,7 +662,7 @@ constexpr int kRingBlocks = 4;   // blocks on a binary's ringdown
 // the binary's NQC coefficients (5 per mode).  sum_m h_m e^{-i m phi} by Horner's
 // rule in e^{-i phi} over the modes by falling m (mo): each mode then costs the
 // products between its m and the next one's, not m - 1 of its own.
-template <SamplePath kPath, class Ptr>
+template <Phases kPath, class Ptr>
 __device__ __forceinline__ bool imr_inspiral_sample(Ptr row, Ptr rpr, const Piece& p, int nm, const ModeOrder& mo, const double* nq,
                                                     double& re_out, double& im_out) {
     const double om = p.d(row + 4 * (2 * nm)), r = p.v(rpr), pr = p.v(rpr + 4);
@@ -797,10 +797,13 @@ __global__ __launch_bounds__(kImrBlock) void k_imr_resample(const double* __rest
                     }
                 },
                 [&](int k, double x, double& re, double& im) {
-                    return imr_inspiral_sample<kNear>(st.modes.c + k * cs, st.rp.c + 8 * k, Piece::at(x, false), nm, mo, st.nq, re, im);
+                    return imr_inspiral_sample<kBounded>(st.modes.c + k * cs, st.rp.c + 8 * k, Piece::at(x, false), nm, mo, st.nq, re, im);
                 },
                 [&](int i, double x, double& re, double& im) {
-                    return imr_inspiral_sample<kFar>(C + (size_t)cs * i, RP + (size_t)8 * i, Piece::at(x, i == len - 1), nm, mo, st.nq, re, im);
+                    return imr_inspiral_sample<kBounded>(C + (size_t)cs * i, RP + (size_t)8 * i, Piece::at(x, i == len - 1), nm, mo, st.nq, re, im);
+                },
+                [&](int i, double x, double& re, double& im) {
+                    return imr_inspiral_sample<kAny>(C + (size_t)cs * i, RP + (size_t)8 * i, Piece::at(x, i == len - 1), nm, mo, st.nq, re, im);
                 },
                 [&](long long j, const double (&re)[2], const double (&im)[2], bool full) { o.put(j, re, im, full); });
         o.zeros(j0);

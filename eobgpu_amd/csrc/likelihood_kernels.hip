@@ -149,7 +149,7 @@ struct LikRows {
 // the longest templates first, and a block index over what the sizes hold (ten
 // launches of 73 us, each with its own slow end; 616 in one; with the grid of
 // the longest for every row 729).  Otherwise row b at hbuf + rowoff[b], zero for nsamp <= j < M_b.
-// Five wavefronts a SIMD, by spills in the general way (resample_rows' far).
+// Five wavefronts a SIMD, by spills in rows of very large phases (resample_rows' exact).
 template <bool kSupport>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) void k_lik_resample(const double* __restrict__ dense, const double* __restrict__ coef,
                                                          const int* __restrict__ num_steps, const double* __restrict__ amp,

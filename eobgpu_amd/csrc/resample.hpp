@@ -69,14 +69,14 @@ __device__ __forceinline__ bool one_by_one(double xa, double xb, int ia, int ib,
     return good;
 }
 
-// How a sample's sine and cosine are taken: kNear only for |x| < 2^49 (false for the
-// others), kFar for any.  The hot loop takes kNear alone and a row with a larger
-// phase goes the general way: with the large reduction inside the loop the
-// likelihood of 1024 templates takes 5% longer.
-enum SamplePath { kNear, kFar };
-template <SamplePath P>
+// How a sample's sine and cosine are taken: kBounded only for |x| < 2^49 (false for the
+// others), kAny for any.  Rows are taken by the first and once more by the second if a
+// phase of theirs is larger: with the large reduction inside the loops the likelihood of
+// 1024 templates takes 5% longer, that of 512 with 5k to 60k knots 3%.
+enum Phases { kBounded, kAny };
+template <Phases P>
 __device__ __forceinline__ bool sincos_of(double x, double& s, double& c) {
-    if constexpr (P == kNear) return eob::sincos_bounded(x, s, c);
+    if constexpr (P == kBounded) return eob::sincos_bounded(x, s, c);
     eob::sincos_phase(x, s, c);
     return true;
 }
@@ -115,17 +115,18 @@ struct StagedRows {
 //   time(j)                the time of sample j
 //   stage(i, n)            table rows i .. i + n - 1 (n <= R) into the wavefront's LDS
 //   near(k, x, re, im)     one sample at x past the knot of staged row k (per lane); false
-//                          if the row needs far
-//   far(i, x, re, im)      one sample from table row i (per lane), read from memory
+//                          if its phase needs `exact`
+//   far(i, x, re, im)      the same from table row i (per lane), read from memory
+//   exact(i, x, re, im)    the same for any phase
 //   put(j, re, im, full)   a lane's samples j, j + 1 (full: all of the row's are below jend)
 // The run's knots (lane q holds the q-th after its first) and table rows are read
 // in two steps at its start; its rows then wait for no load.  Interval by interval
 // through the scalar cache, with gathers where a row passes a knot, the waits
 // (about 1 us each, four a row) were the time: 1024 templates' h+ for the likelihood
 // 880 us, 735 this way; the five modes with NQC factors of 512 binaries 3560, 3060.
-template <int R, class Time, class Stage, class Near, class Far, class Put>
+template <int R, class Time, class Stage, class Near, class Far, class Exact, class Put>
 __device__ __forceinline__ void resample_rows(const double* __restrict__ T, int len, long long j0, long long jend, const Time& time,
-                                              const Stage& stage, const Near& near, const Far& far, const Put& put) {
+                                              const Stage& stage, const Near& near, const Far& far, const Exact& exact, const Put& put) {
     static_assert(R <= 63, "a lane per knot");
     const int lane = threadIdx.x & 63;
     const double end = time((j0 + kRun < jend ? j0 + kRun : jend) - 1);
@@ -188,7 +189,9 @@ __device__ __forceinline__ void resample_rows(const double* __restrict__ T, int 
             ib = T[5 * (size_t)(ib + half)] <= tb ? ib + half : ib;
             m -= half;
         }
-        one_by_one(ta - T[5 * (size_t)ia], tb - T[5 * (size_t)ib], ia, ib, re, im, far);
+        const double xa = ta - T[5 * (size_t)ia], xb = tb - T[5 * (size_t)ib];
+        if (!large) large = __any(!one_by_one(xa, xb, ia, ib, re, im, far));
+        if (large) one_by_one(xa, xb, ia, ib, re, im, exact);
         put(j, re, im, false);
         ind = wave_interval(T, len, last);
         ++r;
@@ -213,7 +216,7 @@ __device__ __forceinline__ void store_pair(double* out, long long j, long long N
 
 // h22 = S e^{-2 i phi} at x past the knot of a row of the (2,2) splines (phi,
 // Re S, Im S; 4 coefficients each)
-template <SamplePath P, class Row>
+template <Phases P, class Row>
 __device__ __forceinline__ bool h22_sample(const Row& c, double x, double& re, double& im) {
     const double x2 = x * x, x3 = x2 * x;
     const double ph = c[0] + c[1] * x + c[2] * x2 + c[3] * x3;
@@ -233,8 +236,9 @@ __device__ __forceinline__ void h22_rows(H22Stage& st, const double* __restrict_
                                          long long j0, long long jend, const Put& put) {
     resample_rows<H22Stage::kRows>(
         T, len, j0, jend, [&](long long j) { return t0 + (double)j * dT; }, [&](int i, int n) { st.copy(C + (size_t)12 * i, n); },
-        [&](int k, double x, double& re, double& im) { return h22_sample<kNear>(st.row(k), x, re, im); },
-        [&](int i, double x, double& re, double& im) { return h22_sample<kFar>(C + (size_t)12 * i, x, re, im); }, put);
+        [&](int k, double x, double& re, double& im) { return h22_sample<kBounded>(st.row(k), x, re, im); },
+        [&](int i, double x, double& re, double& im) { return h22_sample<kBounded>(C + (size_t)12 * i, x, re, im); },
+        [&](int i, double x, double& re, double& im) { return h22_sample<kAny>(C + (size_t)12 * i, x, re, im); }, put);
 }
 
 // h+ and hx (hx may be null) of N samples, zero from nb on.  kHole: but samples nb <= j <

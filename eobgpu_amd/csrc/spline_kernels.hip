@@ -635,7 +635,7 @@ __device__ __forceinline__ long long series_samples(const double* T, int len, do
     return nb > N ? N : nb;
 }
 
-__global__ __launch_bounds__(kBlock) void k_resample_hplus(const double* __restrict__ dense, const double* __restrict__ coef,
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_resample_hplus(const double* __restrict__ dense, const double* __restrict__ coef,
                                                            const int* __restrict__ num_steps, const double* __restrict__ amp,
                                                            const double* __restrict__ dT_M, int max_step, int N,
                                                            double* __restrict__ hplus, int* __restrict__ nsamp,
@@ -668,7 +668,7 @@ constexpr int kMaxModeM = 8;
 // One sample's sum from a row (Re of each mode, Im of each mode, phi; 4
 // coefficients per series), by Horner's rule in e^{-i phi} over the modes by
 // falling m: a mode costs the products between its m and the next one's.
-template <SamplePath P, class Ptr>
+template <Phases P, class Ptr>
 __device__ __forceinline__ bool modes_sample(Ptr c, double x, int nm, const ModeOrder& mo, double& hr, double& hi) {
     const double x2 = x * x, x3 = x2 * x;
     const auto cubic = [&](Ptr p) { return p[0] + p[1] * x + p[2] * x2 + p[3] * x3; };
@@ -720,8 +720,9 @@ __global__ __launch_bounds__(kBlock) void k_resample_modes(const double* __restr
         if (j0 < nb)
             resample_rows<Stage::kRows>(
                 T, len, j0, nb, [&](long long j) { return t0 + (double)j * dT; }, [&](int i, int n) { st.copy(C + (size_t)cs * i, n, cs); },
-                [&](int k, double x, double& re, double& im) { return modes_sample<kNear>(st.c + k * cs, x, nm, mo, re, im); },
-                [&](int i, double x, double& re, double& im) { return modes_sample<kFar>(C + (size_t)cs * i, x, nm, mo, re, im); },
+                [&](int k, double x, double& re, double& im) { return modes_sample<kBounded>(st.c + k * cs, x, nm, mo, re, im); },
+                [&](int i, double x, double& re, double& im) { return modes_sample<kBounded>(C + (size_t)cs * i, x, nm, mo, re, im); },
+                [&](int i, double x, double& re, double& im) { return modes_sample<kAny>(C + (size_t)cs * i, x, nm, mo, re, im); },
                 [&](long long j, const double (&re)[2], const double (&im)[2], bool full) { o.put(j, re, im, full); });
         o.zeros(j0);
     });
