@@ -42,8 +42,8 @@ __device__ __forceinline__ Row interior_row(double d1, double m1, double d2, dou
 // does for normal numbers (Markstein's method).  With plain products, and 3 times a
 // right-hand side rounded before it is used, the coefficients' error against extended
 // precision was 4 to 25 % larger (rms; 1.5 to 2 times between the knots of uneven
-// chirps) than one elimination from the first row leaves; this way it is equal, for
-// 4 % of the builders' time.
+// chirps) than one elimination from the first row leaves; this way it is equal.  (Halo
+// rows keep the products: what they round is damped before it reaches a lane's own.)
 __device__ __forceinline__ double over(double v, double d, double r) {
     const double w = v * r;
     return fma(fma(-d, w, v), r, w);
@@ -108,7 +108,7 @@ __global__ __launch_bounds__(kBlock) void k_interpolate_TD(const double* __restr
                     r = c.end(i);
                     three = 1.0;
                 }
-                const double w = i == hi - 1 ? 0.0 : over(r.ud, Da, ia);
+                const double w = i == hi - 1 ? 0.0 : r.ud * ia;
                 Da = r.dg - w * la;
                 Ba = fma(three, r.b, -(w * Ba));   // 3 r.b is not rounded by itself
                 la = r.ld;
@@ -141,7 +141,7 @@ __global__ __launch_bounds__(kBlock) void k_interpolate_TD(const double* __restr
                     r = c.end(0);
                     three = 1.0;
                 }
-                const double w = i == lo ? 0.0 : over(r.ld, D, id);
+                const double w = i == lo ? 0.0 : r.ld * id;
                 D = r.dg - w * u;
                 Bb = fma(three, r.b, -(w * Bb));
                 u = r.ud;
@@ -249,10 +249,12 @@ __device__ __forceinline__ int tile_at(int k) { return k + (k >> 4); }
 // rows g = h = 0) and the row a s_n + dg s + c s_next = k b to s = b' - c' s_next.
 struct Carry {
     double h, g;   // c', d'
+    // kHalo: a row that is not the lane's own
+    template <bool kHalo = true>
     __device__ __forceinline__ double step(double a, double dg, double c, double b, double k = 3.0) {
-        const double den = dg - a * h, inv = eob::refined_rcp(den);
-        g = over(fma(k, b, -(a * g)), den, inv);
-        h = over(c, den, inv);
+        const double den = dg - a * h, inv = eob::refined_rcp(den), r = fma(k, b, -(a * g));
+        g = kHalo ? r * inv : over(r, den, inv);
+        h = kHalo ? c * inv : over(c, den, inv);
         return inv;
     }
 };
@@ -375,7 +377,7 @@ __global__ __launch_bounds__(kTileThreads) void k_spline_build_tile(const double
                 const bool first = i == 0, last = i == len - 1;
                 const double a = first ? 0.0 : (last ? lld : d2), dg = first ? fdg : (last ? ldg : 2 * (d1 + d2));
                 const double c = first ? fud : (last ? 0.0 : d1), r = first ? fb : (last ? lb : d2 * m1 + d1 * m2);
-                dn.step(a, dg, c, r, first || last ? 1.0 : 3.0);
+                dn.step<false>(a, dg, c, r, first || last ? 1.0 : 3.0);
                 d1 = d2;
                 m1 = m2;
             }
