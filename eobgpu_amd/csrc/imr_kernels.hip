@@ -739,9 +739,10 @@ struct Ringdown {
 // (Its few hundred samples in a launch of their own: 20 us for 17 where one binary
 // of 2^18 samples and one mode is the batch, 34 for 28 with five modes, 280 for 260
 // with 256 binaries of 2^16; by the lanes that would write zeros there: 23, 47 and 386.)
-//
-// kModes: the most modes the staged rows have room for.
-template <int kModes>
+// One build for any number of modes: 23 table rows of five are staged, 16 of eight (with
+// 8 rows 64 binaries x 2^14 of eight modes 44.9 us, 41.9 now; 21 rows are no faster).
+constexpr int kImrRoom = 1280;   // a wavefront's doubles of LDS
+template <int kRows>
 __global__ __launch_bounds__(kImrBlock) void k_imr_resample(const double* __restrict__ dense, const int* __restrict__ num_steps,
                                                             const double* __restrict__ coef, const double* __restrict__ rp,
                                                             const double* __restrict__ amp, const double* __restrict__ dT_M, int max_step,
@@ -767,7 +768,7 @@ __global__ __launch_bounds__(kImrBlock) void k_imr_resample(const double* __rest
     if (blockIdx.x >= blocks) {
         const double t_match = binf[(size_t)b * kBinCount + kBinTMatch], dt = binf[(size_t)b * kBinCount + kBinDt];
         const Ringdown ring{rd + (size_t)b * nm * kRdCount, t_match, dt, idx};
-        for (long long j = idx + 1 + (long long)(blockIdx.x - blocks) * kImrBlock + threadIdx.x; j < stop; j += kRingBlocks * kImrBlock) {
+        for (long long j = idx + 1 + (long long)(blockIdx.x - blocks) * blockDim.x + threadIdx.x; j < stop; j += kRingBlocks * blockDim.x) {
             double hr, hi;
             ring.sample(j, nm, hr, hi);
             o.out[j] = o.a * hr;
@@ -775,38 +776,35 @@ __global__ __launch_bounds__(kImrBlock) void k_imr_resample(const double* __rest
         }
         return;
     }
-    struct Stage {
-        StagedRows<4 * (2 * kModes + 1), 8> modes;   // rows at their own stride cs
-        StagedRows<8, 8> rp;
-        double nq[5 * kModes];
-    };
-    __shared__ Stage stages[kImrBlock / 64];
-    Stage& st = stages[threadIdx.x >> 6];
-    if ((int)(threadIdx.x & 63) < 5 * nm) st.nq[threadIdx.x & 63] = nqc[(size_t)b * nm * 5 + (threadIdx.x & 63)];
-    for_runs(N, kImrBlock / 64, blocks, [&](long long j0) {
+    // a wavefront's NQC factors and table rows: the modes', then those of rp
+    extern __shared__ __attribute__((aligned(16))) double staged[];
+    const int most = staged_rows(kImrRoom - 5 * kImrMaxModes, cs + 8);
+    double *nq = staged + wave_index() * kImrRoom, *ms = nq + 5 * kImrMaxModes, *rs = ms + most * cs;
+    if ((int)(threadIdx.x & 63) < 5 * nm) nq[threadIdx.x & 63] = nqc[(size_t)b * nm * 5 + (threadIdx.x & 63)];
+    for_runs(N, kRows, blocks, [&](long long j0) {
         if (j0 < jinsp)
-            resample_rows<8>(
-                T, len, j0, jinsp, [&](long long j) { return grid_t(j, dT, t0); },
+            resample_rows(
+                kRows, most, true, T, len, j0, jinsp, [&](long long j) { return grid_t(j, dT, t0); },
                 [&](int i, int n) {
-                    st.modes.copy(C + (size_t)cs * i, n, cs);
-                    st.rp.copy(RP + (size_t)8 * i, n);
+                    stage_rows<5>(ms, C + (size_t)cs * i, n, cs);
+                    stage_rows<1>(rs, RP + (size_t)8 * i, n, 8);
                     if (i + n == len) {   // the last knot's interval: its value, no slope
                         __builtin_amdgcn_wave_barrier();
-                        st.modes.flatten(n - 1, cs);
-                        st.rp.flatten(n - 1);
+                        flatten_row(ms + (n - 1) * cs, cs);
+                        flatten_row(rs + (n - 1) * 8, 8);
                     }
                 },
                 [&](int k, double x, double& re, double& im) {
-                    return imr_inspiral_sample<kBounded>(st.modes.c + k * cs, st.rp.c + 8 * k, Piece::at(x, false), nm, mo, st.nq, re, im);
+                    return imr_inspiral_sample<kBounded>(ms + k * cs, rs + 8 * k, Piece::at(x, false), nm, mo, nq, re, im);
                 },
                 [&](int i, double x, double& re, double& im) {
-                    return imr_inspiral_sample<kBounded>(C + (size_t)cs * i, RP + (size_t)8 * i, Piece::at(x, i == len - 1), nm, mo, st.nq, re, im);
+                    return imr_inspiral_sample<kBounded>(C + (size_t)cs * i, RP + (size_t)8 * i, Piece::at(x, i == len - 1), nm, mo, nq, re, im);
                 },
                 [&](int i, double x, double& re, double& im) {
-                    return imr_inspiral_sample<kAny>(C + (size_t)cs * i, RP + (size_t)8 * i, Piece::at(x, i == len - 1), nm, mo, st.nq, re, im);
+                    return imr_inspiral_sample<kAny>(C + (size_t)cs * i, RP + (size_t)8 * i, Piece::at(x, i == len - 1), nm, mo, nq, re, im);
                 },
                 [&](long long j, const double (&re)[2], const double (&im)[2], bool full) { o.put(j, re, im, full); });
-        o.zeros(j0);
+        o.zeros(j0, kRows);
     });
 }
 
@@ -910,14 +908,10 @@ int eobhip_imr_resample(const double* dense, const int* num_steps, const double*
     if (rc) return rc;
     EOBHIP_REQUIRE(n >= 0 && n <= 65535 && N >= 1, "bad sizes");
     if (n == 0) return EOBHIP_OK;
-    dim3 grid = resample_grid(N, n);
-    const dim3 block(kImrBlock);
-    hipStream_t st = as_stream(stream);
-    static_assert(kImrMaxModes == 8, "room for every mode");
-    grid.x += kRingBlocks;
-    const auto kernel = nm <= 5 ? k_imr_resample<5> : k_imr_resample<8>;
-    hipLaunchKernelGGL(kernel, grid, block, 0, st, dense, num_steps, coef, rp_coef, amp, dT_M, max_step, N, nm, mode_order(mm.m, nm), nqc, rd, binf,
-                       bini, hplus, hcross, nsamp);
+    ResampleShape s = resample_shape(N, n, kImrRoom);
+    s.grid.x += kRingBlocks;
+    hipLaunchKernelGGL(s.rows == 1 ? k_imr_resample<1> : k_imr_resample<kRunRows>, s.grid, s.block, s.lds, as_stream(stream), dense,
+                       num_steps, coef, rp_coef, amp, dT_M, max_step, N, nm, mode_order(mm.m, nm), nqc, rd, binf, bini, hplus, hcross, nsamp);
     return check_launch("imr_resample");
 }
 

@@ -177,11 +177,12 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) voi
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const long long j0 = (long long)bx * kSpan + wave * kRun;
     double acc = 0.0;
-    __shared__ H22Stage stages[kBlock / 64];
+    constexpr int kRows = 16;   // staged at once: with more the kernel spills in its ordinary rows (5% of the whole)
+    __shared__ __attribute__((aligned(16))) double stages[kBlock / 64][12 * kRows];
     if (j0 < nb) {
         const double* T = dense + (size_t)b * max_step * 5;
         const double a = amp[b];
-        h22_rows(stages[wave], T, coef + (size_t)b * max_step * 12, num_steps[b], T[0], dT_M[b], j0, nb,
+        h22_rows(stages[wave], kRunRows, kRows, false, T, coef + (size_t)b * max_step * 12, num_steps[b], T[0], dT_M[b], j0, nb,
                  [&](long long j, const double (&re)[2], const double (&)[2], bool full) {
                      const double ga = full || j < nb ? g[j] : 0.0, gb = full || j + 1 < nb ? g[j + 1] : 0.0;
                      const double va = full || j < nb ? a * re[0] : 0.0, vb = full || j + 1 < nb ? a * re[1] : 0.0;

@@ -637,6 +637,8 @@ __device__ __forceinline__ long long series_samples(const double* T, int len, do
     return nb > N ? N : nb;
 }
 
+constexpr int kH22Room = 12 * kMostStaged;   // doubles a wavefront stages
+template <int kRows>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_resample_hplus(const double* __restrict__ dense, const double* __restrict__ coef,
                                                            const int* __restrict__ num_steps, const double* __restrict__ amp,
                                                            const double* __restrict__ dT_M, int max_step, int N,
@@ -651,12 +653,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
     const SeriesOut<> o{hplus + (size_t)b * N, hcross ? hcross + (size_t)b * N : nullptr, amp[b], nb, N};
     const double* C = coef + (size_t)b * max_step * 12;
     const double t0 = T[0];
-    __shared__ H22Stage stages[kBlock / 64];
-    H22Stage& st = stages[threadIdx.x >> 6];
-    for_runs(N, kBlock / 64, gridDim.x, [&](long long j0) {
+    extern __shared__ __attribute__((aligned(16))) double staged[];
+    double* st = staged + wave_index() * kH22Room;
+    for_runs(N, kRows, gridDim.x, [&](long long j0) {
         if (j0 < nb)
-            h22_rows(st, T, C, len, t0, dT, j0, nb, [&](long long j, const double (&re)[2], const double (&im)[2], bool full) { o.put(j, re, im, full); });
-        o.zeros(j0);
+            h22_rows(st, kRows, kMostStaged, true, T, C, len, t0, dT, j0, nb,
+                     [&](long long j, const double (&re)[2], const double (&im)[2], bool full) { o.put(j, re, im, full); });
+        o.zeros(j0, kRows);
     });
 }
 
@@ -697,10 +700,12 @@ __device__ __forceinline__ bool modes_sample(Ptr c, double x, int nm, const Mode
     return good;
 }
 
-// kModes: the most modes the staged rows have room for.  Five modes of 512 binaries
-// x 2^20, 10% of the samples inside a template: 2470 us with knot windows per block,
-// 1520 interval by interval, 1470 to 1570 now (the writes alone 1360).
-template <int kModes>
+// Five modes of 512 binaries x 2^20, 10% of the samples inside a template: 2470 us with
+// knot windows per block, 1520 interval by interval, 1470 to 1570 now (the writes alone
+// 1360).  One build for any number of modes: what a wavefront stages is 63 rows of one
+// mode, 28 of five, 10 of fifteen.
+constexpr int kModesRoom = 1264;   // doubles a wavefront stages: four blocks fill a CU's LDS
+template <int kRows>
 __global__ __launch_bounds__(kBlock) void k_resample_modes(const double* __restrict__ dense, const double* __restrict__ coef,
                                                            const int* __restrict__ num_steps, const double* __restrict__ amp,
                                                            const double* __restrict__ dT_M, int max_step, int N, int nm, ModeOrder mo,
@@ -715,18 +720,18 @@ __global__ __launch_bounds__(kBlock) void k_resample_modes(const double* __restr
     const long long nb = series_samples(T, len, dT, N);
     if (blockIdx.x == 0 && threadIdx.x == 0) nsamp[b] = (int)nb;
     const SeriesOut<> o{hplus + (size_t)b * N, hcross + (size_t)b * N, amp[b], nb, N};
-    typedef StagedRows<4 * (2 * kModes + 1), 8> Stage;   // rows at their own stride cs
-    __shared__ Stage stages[kBlock / 64];
-    Stage& st = stages[threadIdx.x >> 6];
-    for_runs(N, kBlock / 64, gridDim.x, [&](long long j0) {
+    extern __shared__ __attribute__((aligned(16))) double staged[];
+    double* st = staged + wave_index() * kModesRoom;
+    for_runs(N, kRows, gridDim.x, [&](long long j0) {
         if (j0 < nb)
-            resample_rows<Stage::kRows>(
-                T, len, j0, nb, [&](long long j) { return t0 + (double)j * dT; }, [&](int i, int n) { st.copy(C + (size_t)cs * i, n, cs); },
-                [&](int k, double x, double& re, double& im) { return modes_sample<kBounded>(st.c + k * cs, x, nm, mo, re, im); },
+            resample_rows(
+                kRows, staged_rows(kModesRoom, cs), true, T, len, j0, nb, [&](long long j) { return t0 + (double)j * dT; },
+                [&](int i, int n) { stage_rows<6>(st, C + (size_t)cs * i, n, cs); },
+                [&](int k, double x, double& re, double& im) { return modes_sample<kBounded>(st + k * cs, x, nm, mo, re, im); },
                 [&](int i, double x, double& re, double& im) { return modes_sample<kBounded>(C + (size_t)cs * i, x, nm, mo, re, im); },
                 [&](int i, double x, double& re, double& im) { return modes_sample<kAny>(C + (size_t)cs * i, x, nm, mo, re, im); },
                 [&](long long j, const double (&re)[2], const double (&im)[2], bool full) { o.put(j, re, im, full); });
-        o.zeros(j0);
+        o.zeros(j0, kRows);
     });
 }
 
@@ -1006,8 +1011,9 @@ int eobhip_resample_hplus(const double* dense, const double* coef, const int* nu
                           int max_step, int N, double* hplus, int* nsamp, void* stream) {
     EOBHIP_REQUIRE(n >= 0 && N >= 1 && n <= 65535, "bad sizes");
     if (n == 0) return EOBHIP_OK;
-    hipLaunchKernelGGL(k_resample_hplus, resample_grid(N, n), dim3(kBlock), 0, as_stream(stream), dense, coef, num_steps, amp, dT_M, max_step, N, hplus,
-                       nsamp, nullptr);
+    const ResampleShape s = resample_shape(N, n, kH22Room);
+    hipLaunchKernelGGL(s.rows == 1 ? k_resample_hplus<1> : k_resample_hplus<kRunRows>, s.grid, s.block, s.lds, as_stream(stream), dense, coef,
+                       num_steps, amp, dT_M, max_step, N, hplus, nsamp, nullptr);
     return check_launch("resample_hplus");
 }
 
@@ -1018,9 +1024,9 @@ int eobhip_resample_modes(const double* dense, const double* coef, const int* nu
     EOBHIP_REQUIRE(hplus && hcross, "hplus and hcross are required");
     for (int q = 0; q < nm; ++q) EOBHIP_REQUIRE(ms[q] >= 1 && ms[q] <= kMaxModeM, "m must be 1 .. 8");
     if (n == 0) return EOBHIP_OK;
-    const auto kernel = nm <= 5 ? k_resample_modes<5> : k_resample_modes<kMaxModes>;
-    hipLaunchKernelGGL(kernel, resample_grid(N, n), dim3(kBlock), 0, as_stream(stream), dense, coef, num_steps, amp, dT_M, max_step,
-                       N, nm, mode_order(ms, nm), hplus, hcross, nsamp);
+    const ResampleShape s = resample_shape(N, n, kModesRoom);
+    hipLaunchKernelGGL(s.rows == 1 ? k_resample_modes<1> : k_resample_modes<kRunRows>, s.grid, s.block, s.lds, as_stream(stream), dense, coef,
+                       num_steps, amp, dT_M, max_step, N, nm, mode_order(ms, nm), hplus, hcross, nsamp);
     return check_launch("resample_modes");
 }
 
@@ -1045,8 +1051,9 @@ int eobhip_resample_hpc(const double* dense, const double* coef, const int* num_
     EOBHIP_REQUIRE(n >= 0 && N >= 1 && n <= 65535, "bad sizes");
     EOBHIP_REQUIRE(hcross != nullptr, "hcross is required");
     if (n == 0) return EOBHIP_OK;
-    hipLaunchKernelGGL(k_resample_hplus, resample_grid(N, n), dim3(kBlock), 0, as_stream(stream), dense, coef, num_steps, amp, dT_M, max_step, N, hplus,
-                       nsamp, hcross);
+    const ResampleShape s = resample_shape(N, n, kH22Room);
+    hipLaunchKernelGGL(s.rows == 1 ? k_resample_hplus<1> : k_resample_hplus<kRunRows>, s.grid, s.block, s.lds, as_stream(stream), dense, coef,
+                       num_steps, amp, dT_M, max_step, N, hplus, nsamp, hcross);
     return check_launch("resample_hpc");
 }
 

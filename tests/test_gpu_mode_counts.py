@@ -1,4 +1,4 @@
-"""The mode sum with more modes than its first build holds rows for (6 to 15), every m
+"""The mode sum of 6 to 15 modes, every m
 up to 8, repeated and in any order, against numpy: knots that several rows of 128
 samples share, that one row passes in tens and that it passes in hundreds."""
 import ctypes
