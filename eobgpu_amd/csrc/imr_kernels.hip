@@ -764,11 +764,15 @@ __global__ __launch_bounds__(kImrBlock) void k_imr_resample(const double* __rest
     const double t0 = T[0], dT = dT_M[b];
     const long long stop = nvalid < N ? nvalid : N;
     const SeriesOut<true> o{hplus + (size_t)b * N, hcross + (size_t)b * N, amp[b], jinsp, N, stop};   // nvalid >= idx + 1, or 0
-    const unsigned blocks = gridDim.x - kRingBlocks;
-    if (blockIdx.x >= blocks) {
+    // Blocks go to the eight XCDs in turn: in a grid of 8 k a row, each binary's ringdown
+    // would be on the same four, so that the rows take turns too (512 binaries x 2^13, one and
+    // five modes: 95 and 154 us, 57 and 93 in turn; where the grid is another, 64 x 2^14 33 and
+    // 37 in turn).
+    const unsigned blocks = gridDim.x - kRingBlocks, block = gridDim.x % 8 ? blockIdx.x : (blockIdx.x + blockIdx.y) % gridDim.x;
+    if (block >= blocks) {
         const double t_match = binf[(size_t)b * kBinCount + kBinTMatch], dt = binf[(size_t)b * kBinCount + kBinDt];
         const Ringdown ring{rd + (size_t)b * nm * kRdCount, t_match, dt, idx};
-        for (long long j = idx + 1 + (long long)(blockIdx.x - blocks) * blockDim.x + threadIdx.x; j < stop; j += kRingBlocks * blockDim.x) {
+        for (long long j = idx + 1 + (long long)(block - blocks) * blockDim.x + threadIdx.x; j < stop; j += kRingBlocks * blockDim.x) {
             double hr, hi;
             ring.sample(j, nm, hr, hi);
             o.out[j] = o.a * hr;
@@ -781,7 +785,7 @@ __global__ __launch_bounds__(kImrBlock) void k_imr_resample(const double* __rest
     const int most = staged_rows(kImrRoom - 5 * kImrMaxModes, cs + 8);
     double *nq = staged + wave_index() * kImrRoom, *ms = nq + 5 * kImrMaxModes, *rs = ms + most * cs;
     if ((int)(threadIdx.x & 63) < 5 * nm) nq[threadIdx.x & 63] = nqc[(size_t)b * nm * 5 + (threadIdx.x & 63)];
-    for_runs(N, kRows, blocks, [&](long long j0) {
+    for_runs(N, kRows, block, blocks, [&](long long j0) {
         if (j0 < jinsp)
             resample_rows(
                 kRows, most, true, T, len, j0, jinsp, [&](long long j) { return grid_t(j, dT, t0); },

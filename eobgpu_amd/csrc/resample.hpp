@@ -319,12 +319,12 @@ struct SeriesOut {
     }
 };
 
-// A wavefront's runs of `rows` rows of one binary's series by `blocks` blocks, f(j0);
-// shape resample_shape
+// A wavefront's runs of `rows` rows of one binary's series by `blocks` blocks, of which its
+// is number `block`, f(j0); shape resample_shape
 template <class F>
-__device__ __forceinline__ void for_runs(long long N, int rows, unsigned blocks, const F& f) {
+__device__ __forceinline__ void for_runs(long long N, int rows, unsigned block, unsigned blocks, const F& f) {
     const long long step = (long long)blocks * (blockDim.x >> 6) * (rows * kRow);
-    for (long long j0 = ((long long)blockIdx.x * (blockDim.x >> 6) + wave_index()) * (rows * kRow); j0 < N; j0 += step) f(j0);
+    for (long long j0 = ((long long)block * (blockDim.x >> 6) + wave_index()) * (rows * kRow); j0 < N; j0 += step) f(j0);
 }
 
 // (blocks of up to four wavefronts, binaries): about 131072 blocks in all, no more, so

@@ -655,7 +655,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
     const double t0 = T[0];
     extern __shared__ __attribute__((aligned(16))) double staged[];
     double* st = staged + wave_index() * kH22Room;
-    for_runs(N, kRows, gridDim.x, [&](long long j0) {
+    for_runs(N, kRows, blockIdx.x, gridDim.x, [&](long long j0) {
         if (j0 < nb)
             h22_rows(st, kRows, kMostStaged, true, T, C, len, t0, dT, j0, nb,
                      [&](long long j, const double (&re)[2], const double (&im)[2], bool full) { o.put(j, re, im, full); });
@@ -722,7 +722,7 @@ __global__ __launch_bounds__(kBlock) void k_resample_modes(const double* __restr
     const SeriesOut<> o{hplus + (size_t)b * N, hcross + (size_t)b * N, amp[b], nb, N};
     extern __shared__ __attribute__((aligned(16))) double staged[];
     double* st = staged + wave_index() * kModesRoom;
-    for_runs(N, kRows, gridDim.x, [&](long long j0) {
+    for_runs(N, kRows, blockIdx.x, gridDim.x, [&](long long j0) {
         if (j0 < nb)
             resample_rows(
                 kRows, staged_rows(kModesRoom, cs), true, T, len, j0, nb, [&](long long j) { return t0 + (double)j * dT; },

@@ -49,7 +49,45 @@ def test_series_meet_at_the_attachment(dev, modes):
         step = np.abs(np.diff(full[i]))
         assert step[idx[i]] < 2.0 * step[idx[i] - 40:idx[i] + 40].max()
     assert not full[3].any()
-    for N in sorted({int(v) + e for v in np.concatenate([idx, end]) for e in (-1, 0, 1, 2, 3)} | {1, 2, 129}):
+    turns = {N for k in range(4, full.shape[1] // 512, 8) for N in (512 * k, 512 * k - 5)}      # grids whose rows take turns
+    assert max(turns) > idx.min()
+    for N in sorted({int(v) + e for v in np.concatenate([idx, end]) for e in (-1, 0, 1, 2, 3)} | {1, 2, 129} | turns):
         h, ns = template(N)
         assert np.array_equal(h, full[:, :N]), N
         assert np.array_equal(ns[:3], np.minimum(end, N)) and ns[3] == 0
+
+
+def test_ringdowns_of_a_grid_of_eight(dev):
+    """512 binaries of 2^13 samples (eight blocks each, four of them the ringdown's) against 17 runs each (nine)."""
+    n = 512
+    p = configs.uneven_batch(n=n, seed=4)
+    b = P.EOBBatch.from_params(p["m1"], p["m2"], p["chi1"], p["chi2"])
+    b.initial_conditions(p["r0"])
+    b.integrate(rtol=1e-10, atol=1e-10)
+    b.hlm_modes_knots(P.REFERENCE_MODES)
+    b.build_mode_splines()
+    M, dt = p["m1"] + p["m2"], 1.0 / 16384
+    q = b.imr_params(M, dt)
+
+    def best(N):
+        times = []
+        for _ in range(10):
+            s, e = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            torch.cuda.synchronize()
+            big.sin_()   # the launches are made meanwhile
+            s.record()
+            for _ in range(4):
+                call("eobhip_imr_resample", *args[0], n, b.max_step, N, *args[1], P.current_stream())
+            e.record()
+            torch.cuda.synchronize()
+            times.append(s.elapsed_time(e))
+        return min(times)
+
+    big = torch.randn(1 << 28, device=dev)
+    hp, hc = (torch.empty(n * 9000, dtype=torch.float64, device=dev) for _ in range(2))
+    amp, ns = torch.ones(n, dtype=torch.float64, device=dev), torch.zeros(n, dtype=torch.int32, device=dev)
+    ls, ms = ((ctypes.c_int * 5)(*[lm[k] for lm in P.REFERENCE_MODES]) for k in (0, 1))
+    args = ([x.data_ptr() for x in (b.dense, b.num_steps, b.mode_coef, b.rp_coef, amp, q["dT_M"])],
+            [5, ls, ms] + [x.data_ptr() for x in (q["nqc"], q["rd"], q["binf"], q["bini"], hp, hc, ns)])
+    # 6 % fewer samples; with every ringdown on the same four of the eight XCDs 1.6 times as long
+    assert best(8192) < 1.25 * best(8704)
